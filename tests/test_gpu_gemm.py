@@ -577,3 +577,43 @@ def test_gemm_f32_products(M, N, K):
     gemm._run_f32(M, N, K, x, False, w, False, out, accumulate=True)
     assert _err(out, ref_acc.float()) < 1e-5
 
+
+
+@pytest.mark.parametrize("M,N,K", [
+    (1, 1, 1), (3, 5, 7), (31, 33, 17), (32, 32, 16), (65, 130, 257), (128, 1, 48),  # register tiles, every edge
+    (40, 24, 600), (33, 2, 4100),                                # split over waves; pieces of 16 bytes cut by N = 2
+    (1024, 800, 256), (260, 1028, 100), (2052, 516, 36),          # LDS tiles of 64 x 64, k tails of 4 in 32
+    (1000, 512, 1408), (1000, 1412, 520), (1400, 516, 1000)])     # two and four k groups, 64 x 32 tiles
+def test_gemm_f32_kernels_and_layouts(M, N, K):
+    """Both fp32 kernels and every operand layout (A and B k- or m/n-contiguous, aligned and at odd strides and
+    offsets) against float64.  The K roundings of partial sums of unit products, each up to 2^-24 of a partial of
+    size sqrt(k), add up to about 2^-24 K / 2, where the terms' absolute values sum to 0.64 K: an error of about
+    2^-24 of that sum, which (unlike the result) cannot cancel.  Four times that is allowed."""
+    from llattn_amd import gemm
+    dev = require_cuda()
+    g = torch.Generator(device=dev).manual_seed(M + 3 * N + 7 * K)
+    tol = 4 * 2.0 ** -24
+
+    def off(got, ref, terms):
+        return float((got.double() - ref).norm() / terms.norm())
+
+    def view(rows, cols, pad, start):  # a matrix of the values of its storage from (start, start) on
+        full = torch.randn(rows + start, cols + start + pad, device=dev, generator=g)
+        return full[start:, start:start + cols]
+
+    for pad, start in ((0, 0), (4, 4), (3, 1)):
+        for a_trans in (False, True):
+            for b_trans in (False, True):
+                print("case: gemm f32 layouts", M, N, K, pad, start, a_trans, b_trans, flush=True)
+                a = view(K, M, pad, start) if a_trans else view(M, K, pad, start)
+                b = view(K, N, pad, start) if b_trans else view(N, K, pad, start)
+                a64, b64 = (a.t() if a_trans else a).double(), (b if b_trans else b.t()).double()
+                bias = torch.randn(N, device=dev, generator=g)
+                out = torch.full((M, N), float("nan"), device=dev)
+                rs = torch.full((M,), float("nan"), device=dev)
+                gemm._run_f32(M, N, K, a, a_trans, b, b_trans, out, bias=bias, rowsum=rs)
+                assert off(out, a64 @ b64 + bias.double(), a64.abs() @ b64.abs() + bias.double().abs()) < tol
+                assert off(rs, a64.sum(1), a64.abs().sum(1)) < tol
+                again = torch.full((M, N), float("nan"), device=dev)
+                gemm._run_f32(M, N, K, a, a_trans, b, b_trans, again, bias=bias)
+                assert torch.equal(out, again)
