@@ -452,6 +452,8 @@ __global__ __launch_bounds__(256) void gemm_kernel(const GemmArgs a) {
           gelu_bf16x8(xo, g, gp);
           st16(pc, g);
           st16(a.aux + (int64_t)row * a.ld_aux + col, gp);
+        } else if (a.act == LLATTN_ACT_MUL_AUX) {
+          st16(pc, mul_bf16x8(xo, ld16(a.aux + (int64_t)row * a.ld_aux + col)));
         } else {
           st16(pc, xo);
         }
@@ -699,8 +701,8 @@ __global__ __launch_bounds__(256) void gemm_persistent_kernel(const GemmArgs a) 
 
   // C through a range-checked buffer (a masked lane's offset is past the extent; split-head C: the whole matrix)
   const __amdgpu_buffer_rsrc_t rc = make_rsrc(a.C, (CH ? (int64_t)a.M * a.ldc : (int64_t)(a.M - 1) * a.ldc + a.N) * 2);
-  const __amdgpu_buffer_rsrc_t raux = make_rsrc(ACT == LLATTN_ACT_GELU ? a.aux : a.C,
-                                                ((int64_t)(a.M - 1) * (ACT == LLATTN_ACT_GELU ? a.ld_aux : a.ldc) + a.N) * 2);
+  const __amdgpu_buffer_rsrc_t raux = make_rsrc(ACT != LLATTN_ACT_NONE ? a.aux : a.C,
+                                                ((int64_t)(a.M - 1) * (ACT != LLATTN_ACT_NONE ? a.ld_aux : a.ldc) + a.N) * 2);
   // this wave's 64-column slice of a tile's bias into sbias[slot] (lanes 0..15, 16 bytes each;
   // columns past N, or no bias: zero)
   auto bias_dma = [&](int n0t, int slot) {
@@ -806,8 +808,25 @@ __global__ __launch_bounds__(256) void gemm_persistent_kernel(const GemmArgs a) 
       bv[0] = b0.x; bv[1] = b0.y; bv[2] = b0.z; bv[3] = b0.w;
       bv[4] = b1.x; bv[5] = b1.y; bv[6] = b1.z; bv[7] = b1.w;
     }
+    // MUL_AUX: the aux rows of two fragment blocks (8 stores) are loaded together, ahead of the stores of the two
+    // blocks before them: a load waited for behind stores would drain every store first.  (32768 x 4096 x 1408, the
+    // FFN's w2 input gradient through the transposed weight: 376 us, against 566 us on gemm_kernel's transposing
+    // reads and LDS-staged epilogue.)
+    uint4 ax[2][8];
+    auto load_aux = [&](uint4 (&x)[8], int i0) {
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        const int row = rowb + 16 * (i0 + (u >> 2)) + (u & 3);
+        const uint32_t oa = (row < a.M && col < a.N) ? (uint32_t)((int64_t)row * a.ld_aux + col) * 2u : kOffOOB;
+        x[u] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(raux, oa, 0, 0));
+      }
+    };
+    if constexpr (ACT == LLATTN_ACT_MUL_AUX) load_aux(ax[0], 0);
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
+      if constexpr (ACT == LLATTN_ACT_MUL_AUX) {
+        if (i % 2 == 0 && i < 6) load_aux(ax[(i / 2 + 1) % 2], i + 2);
+      }
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const int row = rowb + 16 * i + e;
@@ -849,6 +868,8 @@ __global__ __launch_bounds__(256) void gemm_persistent_kernel(const GemmArgs a) 
           const uint32_t oa = (row < a.M && col < a.N) ? (uint32_t)((int64_t)row * a.ld_aux + col) * 2u : kOffOOB;
           __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(i32x4, gl), rc, oc, 0, 0);
           __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(i32x4, gp), raux, oa, 0, 0);
+        } else if constexpr (ACT == LLATTN_ACT_MUL_AUX) {
+          __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(i32x4, mul_bf16x8(x, ax[(i / 2) % 2][4 * (i % 2) + e])), rc, oc, 0, 0);
         } else {
           __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(i32x4, x), rc, oc, 0, 0);
         }
@@ -1340,6 +1361,8 @@ extern "C" int32_t llattn_gemm(const llattn_gemm_desc* d, void* workspace, size_
     const int tiles = a.tiles_m * a.tiles_n;
     if (a.act == LLATTN_ACT_GELU)
       hipLaunchKernelGGL(gemm_persistent_kernel<LLATTN_ACT_GELU>, dim3(std::min(tiles, cus)), dim3(256), 0, st, a);
+    else if (a.act == LLATTN_ACT_MUL_AUX)
+      hipLaunchKernelGGL(gemm_persistent_kernel<LLATTN_ACT_MUL_AUX>, dim3(std::min(tiles, cus)), dim3(256), 0, st, a);
     else if (ch.T)
       hipLaunchKernelGGL((gemm_persistent_kernel<LLATTN_ACT_NONE, true>), dim3(std::min(tiles, cus)), dim3(256), 0, st, a);
     else if (rowadd)

@@ -102,9 +102,11 @@ def linear_gelu(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None = No
     return g, gp
 
 
-def matmul_nn_scaled(a: torch.Tensor, b: torch.Tensor, s: torch.Tensor) -> torch.Tensor:
+def matmul_nn_scaled(a: torch.Tensor, b: torch.Tensor, s: torch.Tensor, b_t: torch.Tensor | None = None) -> torch.Tensor:
     """``bf16(a [M, K] @ b [K, N]) * s`` elementwise in bf16 (``s`` bf16 ``[M, N]``): with ``s = gelu'(h)`` from
-    :func:`linear_gelu`, the input gradient of a projection whose input was ``gelu(h)``, through the GELU."""
+    :func:`linear_gelu`, the input gradient of a projection whose input was ``gelu(h)``, through the GELU.
+    ``b_t``: ``b``'s transposed copy, if the caller has it; for large M (:func:`input_grad_persistent`) the product
+    then runs on the persistent kernel, as :func:`input_grad` does (the same bits)."""
     _check2d("a", a)
     _check2d("b", b)
     M, K = a.shape
@@ -112,6 +114,12 @@ def matmul_nn_scaled(a: torch.Tensor, b: torch.Tensor, s: torch.Tensor) -> torch
     if b.shape[0] != K:
         raise ValueError(f"a is [{M}, {K}] but b is {tuple(b.shape)}")
     out = torch.empty((M, N), dtype=torch.bfloat16, device=a.device)
+    if b_t is not None and input_grad_persistent(M, K, N):
+        _check2d("b_t", b_t)
+        if tuple(b_t.shape) != (N, K):
+            raise ValueError(f"b_t is {tuple(b_t.shape)}, expected the transpose of b {tuple(b.shape)}")
+        _run(M, N, K, a, False, b_t, False, out, None, False, act=L.ACT_MUL_AUX, aux=s)
+        return out
     _run(M, N, K, a, False, b, True, out, None, False, act=L.ACT_MUL_AUX, aux=s)
     return out
 

@@ -617,3 +617,22 @@ def test_gemm_f32_kernels_and_layouts(M, N, K):
                 again = torch.full((M, N), float("nan"), device=dev)
                 gemm._run_f32(M, N, K, a, a_trans, b, b_trans, again, bias=bias)
                 assert torch.equal(out, again)
+
+
+@pytest.mark.parametrize("M,K,N", [(4096, 72, 8), (4099, 128, 264), (8200, 256, 1040), (16384, 64, 2048), (4096, 4096, 4096)])
+def test_scaled_input_grad_through_the_transpose(M, K, N):
+    """``matmul_nn_scaled`` with the transposed copy (the persistent kernel's MUL_AUX epilogue, or its split-K
+    counterpart where the tiles are few): within the two bf16 roundings (2 x 2^-9) and the fp32 sum of the float32
+    product, and where neither route splits K the same bits as the route through the untransposed operand."""
+    from llattn_amd import gemm
+    dev = require_cuda()
+    print("case: scaled input grad", M, K, N, flush=True)
+    g = torch.Generator(device=dev).manual_seed(M + K + N)
+    dy = torch.randn(M, K, device=dev, generator=g).bfloat16()
+    w = torch.randn(K, N, device=dev, generator=g).bfloat16()
+    s = torch.randn(M, N, device=dev, generator=g).bfloat16()
+    got = gemm.matmul_nn_scaled(dy, w, s, gemm.transpose(w))
+    ref = (dy.float() @ w.float()) * s.float()
+    assert float((got.float() - ref).norm() / ref.norm()) < 2 * 2.0 ** -9
+    if ((M + 255) // 256) * ((N + 255) // 256) >= 224:
+        assert torch.equal(got, gemm.matmul_nn_scaled(dy, w, s))
