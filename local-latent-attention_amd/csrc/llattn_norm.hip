@@ -13,6 +13,7 @@
 // kernel adds the per-workgroup rows in a fixed order (deterministic, no atomics).
 #include "llattn_abi.h"
 #include "llattn_device.h"
+#include "llattn_steps.h"
 
 namespace llattn {
 namespace {
@@ -92,14 +93,25 @@ __global__ __launch_bounds__(256) void rmsnorm_fwd_kernel(const XT* x, int64_t l
   }
 }
 
-template <typename XT, typename DYT, int NCH>
+// RES: dres (the residual path's gradient) is added to dx, and with dx16 the sum is also written in bf16, for a
+// residual addend that is bf16: without it a conversion pass over dx read and wrote 6 bytes an element more.
+// HBM-bound: 14 bytes an element moved, 16 with dx16 (fp32 stream, bf16 dy).  A row's x, dy, dres and rstd are held
+// as stored, two rows per wave in flight and two waves per SIMD (dres loaded with the row: loaded where it is
+// added, each row waited for it).  32768 x 1408: 143 + 41 us with the conversion pass before, 151 us (4.9 TB/s) now.
+//
+// The arithmetic is spelled out in fused multiply-adds with contraction off, so that every instance (with and
+// without the residual) forms the same bits.
+template <typename XT, typename DYT, int NCH, bool RES>
 __global__ __launch_bounds__(256, NCH <= 6 ? 2 : 1) void rmsnorm_bwd_kernel(const DYT* __restrict__ dy, int64_t lddy,
                                                           const XT* __restrict__ x, int64_t ldx,
                                                           const float* __restrict__ rstd,
                                                           const float* __restrict__ w, int M, int D,
-                                                          XT* __restrict__ dx, int64_t lddx,
-                                                          float* __restrict__ part, const XT* dres, int64_t lddres) {
-  extern __shared__ float red[];  // [4][D]
+                                                          XT* dx, int64_t lddx, float* __restrict__ part,
+                                                          const XT* dres, int64_t lddres, uint16_t* dx16,
+                                                          int64_t lddx16) {
+#pragma clang fp contract(off)
+  constexpr bool WL = RES && NCH <= 8;  // weights in LDS
+  extern __shared__ float red[];        // [4][D] dw of the four waves; with WL then the [D] weights
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int nq = D >> 2;
   const int nw = gridDim.x * 4, gw = blockIdx.x * 4 + wave;
@@ -108,86 +120,124 @@ __global__ __launch_bounds__(256, NCH <= 6 ? 2 : 1) void rmsnorm_bwd_kernel(cons
   // Chunks past the row read a valid chunk (0) and are then zeroed by a select: every array element is
   // written unconditionally, so the arrays stay in registers (element writes under a branch made the
   // compiler keep them in scratch memory).
-  float wv[NCH][4], dw[NCH][4];
+  // The weights: in registers, or with WL in LDS, read again for each row: beside two rows with their residual
+  // gradients they would spill at D = 1408.
+  float wv[WL ? 1 : NCH][4], dw[NCH][4];
+  float* wl = red + 4 * D;
+  if constexpr (WL) {
+    for (int c = threadIdx.x; c < nq; c += 256)
+      *reinterpret_cast<float4*>(wl + 4 * c) = *reinterpret_cast<const float4*>(w + 4 * c);
+    __syncthreads();
+  }
 #pragma unroll
   for (int i = 0; i < NCH; ++i) {
-    const int c = lane + 64 * i;
-    const bool ok = c < nq;
-    const float4 w4 = *reinterpret_cast<const float4*>(w + 4 * (ok ? c : 0));
-    wv[i][0] = ok ? w4.x : 0.f;
-    wv[i][1] = ok ? w4.y : 0.f;
-    wv[i][2] = ok ? w4.z : 0.f;
-    wv[i][3] = ok ? w4.w : 0.f;
+    if constexpr (!WL) {
+      const int c = lane + 64 * i;
+      const bool ok = c < nq;
+      const float4 w4 = *reinterpret_cast<const float4*>(w + 4 * (ok ? c : 0));
+      wv[i][0] = ok ? w4.x : 0.f;
+      wv[i][1] = ok ? w4.y : 0.f;
+      wv[i][2] = ok ? w4.z : 0.f;
+      wv[i][3] = ok ? w4.w : 0.f;
+    }
 #pragma unroll
     for (int e = 0; e < 4; ++e) dw[i][e] = 0.f;
   }
+  auto weights = [&](int i, float (&o)[4]) {
+    if constexpr (WL) {  // values past the row meet dy = 0
+      const float4 w4 = *reinterpret_cast<const float4*>(wl + 4 * min(lane + 64 * i, nq - 1));
+      o[0] = w4.x; o[1] = w4.y; o[2] = w4.z; o[3] = w4.w;
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) o[e] = wv[i][e];
+    }
+  };
   const float inv_d = 1.0f / (float)D;
-  // row data of the next row -- x, dy and rstd -- is loaded before the current row is computed (two
-  // register sets), so no load issued while a row is computed is waited for by that row
-  auto load_row = [&](int row, float (&xv)[NCH][4], float (&dv)[NCH][4], float& rs) {
+  struct Row {
+    Raw4<XT> x[NCH];
+    Raw4<DYT> dy[NCH];
+    Raw4<XT> g[RES ? NCH : 1];
+    float rs;
+  };
+  // the next row is loaded before the current row is computed (two register sets), so no load issued while a row
+  // is computed is waited for by that row
+  auto load_row = [&](int row, Row& o) {
     const XT* xr = x + (int64_t)row * ldx;
     const DYT* dr = dy + (int64_t)row * lddy;
-    rs = rstd[row];
+    o.rs = rstd[row];
 #pragma unroll
     for (int i = 0; i < NCH; ++i) {
-      const int c = lane + 64 * i;
-      const bool ok = c < nq;
-      float xt[4], dt[4];
-      ld4(xr + 4 * (ok ? c : 0), xt);
-      ld4(dr + 4 * (ok ? c : 0), dt);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        xv[i][e] = ok ? xt[e] : 0.f;
-        dv[i][e] = ok ? dt[e] : 0.f;
-      }
+      const int c = lane + 64 * i < nq ? lane + 64 * i : 0;
+      o.x[i].load(xr + 4 * c, true);
+      o.dy[i].load(dr + 4 * c, true);
+      if constexpr (RES) o.g[i].load(dres + (int64_t)row * lddres + 4 * c, true);
     }
   };
-  const int64_t ldo = lddx, ldr = lddres;
   // xh = x * rstd and g = dy * w are formed twice (for the row dot product, then for dx) rather than kept
-  auto do_row = [&](int row, const float (&xv)[NCH][4], const float (&dv)[NCH][4], const float r) {
+  auto do_row = [&](int row, const Row& in) {
+#pragma clang fp contract(off)
+    const float r = in.rs;
     float dot = 0.f;
+    auto chunk = [&](int i, float (&xv)[4], float (&dv)[4]) {
+      const bool ok = lane + 64 * i < nq;
+      in.x[i].get(xv);
+      in.dy[i].get(dv);
 #pragma unroll
-    for (int i = 0; i < NCH; ++i)
+      for (int e = 0; e < 4; ++e) {
+        xv[e] = ok ? xv[e] : 0.f;
+        dv[e] = ok ? dv[e] : 0.f;
+      }
+    };
 #pragma unroll
-      for (int e = 0; e < 4; ++e) dot += (dv[i][e] * wv[i][e]) * (xv[i][e] * r);
+    for (int i = 0; i < NCH; ++i) {
+      float xv[4], dv[4], wi[4];
+      chunk(i, xv, dv);
+      weights(i, wi);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) dot = fmaf(dv[e] * wi[e], xv[e] * r, dot);
+    }
     const float mdot = wave_sum(dot) * inv_d;
-    XT* o = dx + (int64_t)row * ldo;
+    if constexpr (WL) asm volatile("" ::: "memory");  // the weights are read again, not kept
+    XT* o = dx + (int64_t)row * lddx;
 #pragma unroll
     for (int i = 0; i < NCH; ++i) {
       const int c = lane + 64 * i;
-      float v[4];
+      float xv[4], dv[4], wi[4], v[4];
+      chunk(i, xv, dv);
+      weights(i, wi);
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const float xh = xv[i][e] * r;
-        v[e] = r * (dv[i][e] * wv[i][e] - xh * mdot);
-        dw[i][e] += dv[i][e] * xh;
+        const float xh = xv[e] * r;
+        v[e] = r * fmaf(-xh, mdot, dv[e] * wi[e]);
+        dw[i][e] = fmaf(dv[e], xh, dw[i][e]);
+      }
+      if constexpr (RES) {  // the gradient that reaches the normalised rows' input through the residual path
+        float g[4];
+        in.g[i].get(g);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = v[e] + g[e];
       }
       if (c < nq) {
-        if (dres) {  // the gradient that reaches the normalised rows' input through the residual path
-          float g[4];
-          ld4(dres + (int64_t)row * ldr + 4 * c, g);
-#pragma unroll
-          for (int e = 0; e < 4; ++e) v[e] += g[e];
-        }
         st4(o + 4 * c, v);
+        if (RES && dx16) st4(dx16 + (int64_t)row * lddx16 + 4 * c, v);
       }
     }
   };
-  float xa[NCH][4], da[NCH][4], ra = 0.f;
-  if constexpr (NCH <= 8) {  // two register sets: the next row loads while this one is computed
-    float xb[NCH][4], db[NCH][4], rb = 0.f;
-    if (r0 < r1) load_row(r0, xa, da, ra);
+  Row ra;
+  if constexpr (NCH <= (RES ? 6 : 8)) {  // two register sets: the next row loads while this one is computed
+    Row rb;
+    if (r0 < r1) load_row(r0, ra);
     for (int row = r0; row < r1; row += 2) {
-      if (row + 1 < r1) load_row(row + 1, xb, db, rb);
-      do_row(row, xa, da, ra);
+      load_row(min(row + 1, r1 - 1), rb);
+      do_row(row, ra);
       if (row + 1 >= r1) break;
-      if (row + 2 < r1) load_row(row + 2, xa, da, ra);
-      do_row(row + 1, xb, db, rb);
+      load_row(min(row + 2, r1 - 1), ra);
+      do_row(row + 1, rb);
     }
   } else {
     for (int row = r0; row < r1; ++row) {
-      load_row(row, xa, da, ra);
-      do_row(row, xa, da, ra);
+      load_row(row, ra);
+      do_row(row, ra);
     }
   }
   // the workgroup's four waves, added in wave order
@@ -249,22 +299,41 @@ void launch_fwd(int nch, const void* x, int64_t ldx, const float* w, int M, int 
   }
 }
 
+struct BwdArgs {
+  const void* dy; int64_t lddy;
+  const void* x; int64_t ldx;
+  const float* rstd;
+  const float* w;
+  int M, D;
+  void* dx; int64_t lddx;
+  float* part;
+  const void* dres; int64_t lddres;
+  uint16_t* dx16; int64_t lddx16;
+};
+
+template <typename XT, typename DYT, int NCH>
+void launch_bwd_n(const BwdArgs& a, hipStream_t st) {
+  const dim3 grid(kBwdBlocks), block(256);
+  const size_t lds = (size_t)(a.dres && NCH <= 8 ? 5 : 4) * a.D * sizeof(float);
+  const DYT* dy = static_cast<const DYT*>(a.dy);
+  const XT* x = static_cast<const XT*>(a.x);
+  const XT* dres = static_cast<const XT*>(a.dres);
+  XT* dx = static_cast<XT*>(a.dx);
+  if (dres)
+    hipLaunchKernelGGL((rmsnorm_bwd_kernel<XT, DYT, NCH, true>), grid, block, lds, st, dy, a.lddy, x, a.ldx, a.rstd, a.w, a.M, a.D, dx, a.lddx, a.part, dres, a.lddres, a.dx16, a.lddx16);
+  else
+    hipLaunchKernelGGL((rmsnorm_bwd_kernel<XT, DYT, NCH, false>), grid, block, lds, st, dy, a.lddy, x, a.ldx, a.rstd, a.w, a.M, a.D, dx, a.lddx, a.part, dres, a.lddres, a.dx16, a.lddx16);
+}
+
 template <typename XT, typename DYT>
-void launch_bwd(int nch, int nblk, const void* dy, int64_t lddy, const void* x, int64_t ldx, const float* rstd,
-                const float* w, int M, int D, void* dx, int64_t lddx, float* part, const void* dres, int64_t lddres,
-                hipStream_t st) {
-  const dim3 grid(nblk), block(256);
-  const size_t lds = (size_t)4 * D * sizeof(float);
-  const DYT* dyp = static_cast<const DYT*>(dy);
-  const XT* xp = static_cast<const XT*>(x);
-  XT* dxp = static_cast<XT*>(dx);
+void launch_bwd(int nch, const BwdArgs& a, hipStream_t st) {
   switch (nch) {
-    case 2: hipLaunchKernelGGL((rmsnorm_bwd_kernel<XT, DYT, 2>), grid, block, lds, st, dyp, lddy, xp, ldx, rstd, w, M, D, dxp, lddx, part, static_cast<const XT*>(dres), lddres); break;
-    case 4: hipLaunchKernelGGL((rmsnorm_bwd_kernel<XT, DYT, 4>), grid, block, lds, st, dyp, lddy, xp, ldx, rstd, w, M, D, dxp, lddx, part, static_cast<const XT*>(dres), lddres); break;
-    case 6: hipLaunchKernelGGL((rmsnorm_bwd_kernel<XT, DYT, 6>), grid, block, lds, st, dyp, lddy, xp, ldx, rstd, w, M, D, dxp, lddx, part, static_cast<const XT*>(dres), lddres); break;
-    case 8: hipLaunchKernelGGL((rmsnorm_bwd_kernel<XT, DYT, 8>), grid, block, lds, st, dyp, lddy, xp, ldx, rstd, w, M, D, dxp, lddx, part, static_cast<const XT*>(dres), lddres); break;
-    case 12: hipLaunchKernelGGL((rmsnorm_bwd_kernel<XT, DYT, 12>), grid, block, lds, st, dyp, lddy, xp, ldx, rstd, w, M, D, dxp, lddx, part, static_cast<const XT*>(dres), lddres); break;
-    default: hipLaunchKernelGGL((rmsnorm_bwd_kernel<XT, DYT, 16>), grid, block, lds, st, dyp, lddy, xp, ldx, rstd, w, M, D, dxp, lddx, part, static_cast<const XT*>(dres), lddres); break;
+    case 2: launch_bwd_n<XT, DYT, 2>(a, st); break;
+    case 4: launch_bwd_n<XT, DYT, 4>(a, st); break;
+    case 6: launch_bwd_n<XT, DYT, 6>(a, st); break;
+    case 8: launch_bwd_n<XT, DYT, 8>(a, st); break;
+    case 12: launch_bwd_n<XT, DYT, 12>(a, st); break;
+    default: launch_bwd_n<XT, DYT, 16>(a, st); break;
   }
 }
 
@@ -323,16 +392,19 @@ extern "C" size_t llattn_rmsnorm_workspace_size(int32_t M, int32_t D) {
   return (size_t)kBwdBlocks * D * sizeof(float);
 }
 
-extern "C" int32_t llattn_rmsnorm_bwd(const void* dy, int32_t dy_dtype, int64_t lddy, const void* x, int32_t x_dtype,
-                                      int64_t ldx, const float* rstd, const float* weight, int32_t M, int32_t D,
-                                      void* dx, int64_t lddx, float* dweight, const void* dres, int64_t lddres,
-                                      void* workspace, size_t workspace_bytes, void* stream) {
+extern "C" int32_t llattn_rmsnorm_bwd_residual(const void* dy, int32_t dy_dtype, int64_t lddy, const void* x,
+                                               int32_t x_dtype, int64_t ldx, const float* rstd, const float* weight,
+                                               int32_t M, int32_t D, void* dx, int64_t lddx, float* dweight,
+                                               const void* dres, int64_t lddres, void* dx16, int64_t lddx16,
+                                               void* workspace, size_t workspace_bytes, void* stream) {
   const char* what = "llattn_rmsnorm_bwd";
   int32_t rc;
   if ((rc = check_dims(what, M, D)) || (rc = check_rows(what, "dy", dy, lddy, dy_dtype, D)) ||
       (rc = check_rows(what, "x", x, ldx, x_dtype, D)) || (rc = check_rows(what, "dx", dx, lddx, x_dtype, D)))
     return rc;
   if (dres && (rc = check_rows(what, "dres", dres, lddres, x_dtype, D))) return rc;
+  if (dx16 && !dres) return fail(LLATTN_ERR_UNSUPPORTED, "%s: a bf16 copy of dx comes with a residual gradient", what);
+  if (dx16 && (rc = check_rows(what, "dx16", dx16, lddx16, LLATTN_BF16, D))) return rc;
   if (!weight || !aligned16(weight) || !rstd || !dweight)
     return fail(LLATTN_ERR_LAYOUT, "%s: weight (16-byte aligned fp32 [D]), rstd and dweight are required", what);
   const size_t need = llattn_rmsnorm_workspace_size(M, D);
@@ -341,10 +413,19 @@ extern "C" int32_t llattn_rmsnorm_bwd(const void* dy, int32_t dy_dtype, int64_t 
   hipStream_t st = static_cast<hipStream_t>(stream);
   const int nch = chunks_for(D);
   float* part = static_cast<float*>(workspace);
-  if (x_dtype == LLATTN_F32 && dy_dtype == LLATTN_F32) launch_bwd<float, float>(nch, kBwdBlocks, dy, lddy, x, ldx, rstd, weight, M, D, dx, lddx, part, dres, lddres, st);
-  else if (x_dtype == LLATTN_F32) launch_bwd<float, uint16_t>(nch, kBwdBlocks, dy, lddy, x, ldx, rstd, weight, M, D, dx, lddx, part, dres, lddres, st);
-  else if (dy_dtype == LLATTN_F32) launch_bwd<uint16_t, float>(nch, kBwdBlocks, dy, lddy, x, ldx, rstd, weight, M, D, dx, lddx, part, dres, lddres, st);
-  else launch_bwd<uint16_t, uint16_t>(nch, kBwdBlocks, dy, lddy, x, ldx, rstd, weight, M, D, dx, lddx, part, dres, lddres, st);
+  const BwdArgs a{dy, lddy, x, ldx, rstd, weight, M, D, dx, lddx, part, dres, lddres, static_cast<uint16_t*>(dx16), lddx16};
+  if (x_dtype == LLATTN_F32 && dy_dtype == LLATTN_F32) launch_bwd<float, float>(nch, a, st);
+  else if (x_dtype == LLATTN_F32) launch_bwd<float, uint16_t>(nch, a, st);
+  else if (dy_dtype == LLATTN_F32) launch_bwd<uint16_t, float>(nch, a, st);
+  else launch_bwd<uint16_t, uint16_t>(nch, a, st);
   hipLaunchKernelGGL(rmsnorm_dw_kernel, dim3((D + 63) / 64), dim3(256), 0, st, part, kBwdBlocks, D, dweight);
   return check_launch(what);
+}
+
+extern "C" int32_t llattn_rmsnorm_bwd(const void* dy, int32_t dy_dtype, int64_t lddy, const void* x, int32_t x_dtype,
+                                      int64_t ldx, const float* rstd, const float* weight, int32_t M, int32_t D,
+                                      void* dx, int64_t lddx, float* dweight, const void* dres, int64_t lddres,
+                                      void* workspace, size_t workspace_bytes, void* stream) {
+  return llattn_rmsnorm_bwd_residual(dy, dy_dtype, lddy, x, x_dtype, ldx, rstd, weight, M, D, dx, lddx, dweight, dres,
+                                     lddres, nullptr, 0, workspace, workspace_bytes, stream);
 }

@@ -93,6 +93,12 @@ SIGNATURES = {
     "llattn_xent": (_I32, [_P, _I64, _I32, _I32, _P, _I64, _P, _P, _P, _I64, _P, _P]),
 }
 
+# the same for include/llattn_steps.h
+STEP_SIGNATURES = {
+    "llattn_rmsnorm_bwd_residual": (_I32, [_P, _I32, _I64, _P, _I32, _I64, _P, _P, _I32, _I32, _P, _I64, _P, _P, _I64,
+                                           _P, _I64, _P, _SZ, _P]),
+}
+
 _lib = None
 
 
@@ -105,7 +111,7 @@ def load() -> ctypes.CDLL:
         raise RuntimeError(f"llattn HIP library not built ({LIB_PATH} missing); run __graft_entry__.build() "
                            "or `python -m llattn_amd._build` on a machine with ROCm hipcc")
     lib = ctypes.CDLL(str(LIB_PATH))
-    for name, (res, args) in SIGNATURES.items():
+    for name, (res, args) in (SIGNATURES | STEP_SIGNATURES).items():
         fn = getattr(lib, name)
         fn.restype = res
         fn.argtypes = args

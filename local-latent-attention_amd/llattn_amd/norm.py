@@ -121,16 +121,21 @@ class _AddRMSNorm(torch.autograd.Function):
             dres = dres.clone()
         dx = torch.empty((M, D), dtype=torch.float32, device=dev)
         dw = torch.empty((D,), dtype=torch.float32, device=dev)
+        # a bf16 addend's gradient is dx in bf16: written by the same pass where there is a residual gradient
+        dx16 = torch.empty((M, D), dtype=torch.bfloat16, device=dev) \
+            if dres is not None and rdt == torch.bfloat16 and ctx.needs_input_grad[1] else None
         lib = L.load()
         nws = lib.llattn_rmsnorm_workspace_size(M, D)
         ws = torch.empty((nws,), dtype=torch.uint8, device=dev)
         from .ops import _call
-        _call("llattn_rmsnorm_bwd", dy2.data_ptr(), L.dtype_code(dy2.dtype), dy2.stride(0), s2.data_ptr(), L.F32,
+        _call("llattn_rmsnorm_bwd_residual", dy2.data_ptr(), L.dtype_code(dy2.dtype), dy2.stride(0), s2.data_ptr(), L.F32,
               s2.stride(0), rstd.data_ptr(), w.data_ptr(), M, D, dx.data_ptr(), dx.stride(0), dw.data_ptr(),
               dres.data_ptr() if dres is not None else None, dres.stride(0) if dres is not None else 0,
+              dx16.data_ptr() if dx16 is not None else None, dx16.stride(0) if dx16 is not None else 0,
               ws.data_ptr(), nws, L.stream_ptr(dev),
-              work=M * D * (dy2.element_size() + 8 + (4 if dres is not None else 0)) + 4 * M)
-        return dx.view(shape), _copy_as(dx, rdt).view(shape), dw.to(wdt), None, None
+              work=M * D * (dy2.element_size() + 8 + (4 if dres is not None else 0) + (2 if dx16 is not None else 0)) + 4 * M)
+        gres = dx16 if dx16 is not None else _copy_as(dx, rdt)
+        return dx.view(shape), gres.view(shape), dw.to(wdt), None, None
 
 
 def add_rms_norm(x: torch.Tensor, res: torch.Tensor, weight: torch.Tensor, eps: float):

@@ -134,3 +134,26 @@ def test_lm_fused_residual_norms_match_unfused():
     assert torch.equal(runs[0][0], runs[1][0])
     for n, g in runs[0][1].items():
         assert torch.equal(g, runs[1][1][n]), n
+
+
+@pytest.mark.parametrize("M,D", [(1, 4), (5, 260), (2049, 1028), (4097, 1408), (70, 1540), (33, 2048), (700, 2052), (9, 4096)])
+def test_residual_gradient_copy(M, D):
+    """The bf16 copy of dx that the residual backward writes is dx rounded (bit for bit), for every row-chunk count
+    and fewer, as many and more rows than the backward has waves; dx itself is the norm's input gradient plus the
+    residual path's gradient, bit for bit as one fp32 addition."""
+    from llattn_amd.norm import add_rms_norm, rms_norm
+    dev = require_cuda()
+    print("case: residual gradient copy", M, D, flush=True)
+    g = torch.Generator(device=dev).manual_seed(M + D)
+    r = lambda dt=torch.float32: torch.randn(M, D, device=dev, generator=g).to(dt)  # noqa: E731
+    x, res, w = r().requires_grad_(), r(torch.bfloat16).requires_grad_(), torch.randn(D, device=dev, generator=g).requires_grad_()
+    ds, dy = r(), r(torch.bfloat16)
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        s, y = add_rms_norm(x, res, w, 1e-6)
+    torch.autograd.backward([s, y], [ds, dy])
+    assert res.grad.dtype == torch.bfloat16 and torch.equal(res.grad, x.grad.bfloat16())
+    s2, w2 = s.detach().requires_grad_(), w.detach().requires_grad_()
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        y2 = rms_norm(s2, w2, 1e-6)
+    y2.backward(dy)
+    assert torch.equal(x.grad, s2.grad + ds) and torch.equal(w.grad, w2.grad)
