@@ -337,6 +337,7 @@ int32_t llattn_rmsnorm_bwd(const void* dy, int32_t dy_dtype, int64_t lddy, const
                            int64_t ldx, const float* rstd, const float* weight, int32_t M, int32_t D, void* dx,
                            int64_t lddx, float* dweight, const void* dres, int64_t lddres, void* workspace,
                            size_t workspace_bytes, void* stream);
+
 /* Cross entropy of bf16 logit rows and its gradient in one pass (the tied LM
  * head's loss, reference train.py:354-370: F.cross_entropy over [B*T, V]
  * logits in fp32 under autocast, ignore_index, and logits.argmax(-1) for the

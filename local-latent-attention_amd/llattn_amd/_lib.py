@@ -57,6 +57,27 @@ class LlattnGemmDesc(ctypes.Structure):
                 ("aux", ctypes.c_void_p), ("ld_aux", ctypes.c_int64), ("c_heads", LlattnHeadsLayout)]
 
 
+class LlattnBlockCfg(ctypes.Structure):  # include/llattn_steps.h
+    _fields_ = [("shape", LlattnShape)] + [(n, ctypes.c_int32) for n in (
+        "d_model", "macro", "has_bias", "saved", "heads", "remote_heads", "dy_heads", "lat_heads")]
+
+
+# parameters and their gradients, in the order in which the module holds them
+BLOCK_PARAMS = ("w_qkv", "b_qkv", "w_rq", "b_rq", "w_rkv", "b_rkv", "w_r", "b_r", "w_out", "b_out", "gate_l", "gate_r")
+
+
+class LlattnBlockParams(ctypes.Structure):
+    _fields_ = [(n, ctypes.c_void_p) for n in BLOCK_PARAMS]
+
+
+class LlattnCoreViews(ctypes.Structure):
+    _fields_ = [(n, LlattnTensor) for n in ("q", "k", "v", "gq", "gk", "gv")]
+
+
+class LlattnFfnCfg(ctypes.Structure):
+    _fields_ = [(n, ctypes.c_int32) for n in ("rows", "d", "d_ff", "d_out", "saved")]
+
+
 _P = ctypes.c_void_p
 _T = ctypes.POINTER(LlattnTensor)
 _G = ctypes.POINTER(LlattnGemmDesc)
@@ -94,9 +115,19 @@ SIGNATURES = {
 }
 
 # the same for include/llattn_steps.h
+_BC, _BP, _CV, _FC = (ctypes.POINTER(t) for t in (LlattnBlockCfg, LlattnBlockParams, LlattnCoreViews, LlattnFfnCfg))
 STEP_SIGNATURES = {
     "llattn_rmsnorm_bwd_residual": (_I32, [_P, _I32, _I64, _P, _I32, _I64, _P, _P, _I32, _I32, _P, _I64, _P, _P, _I64,
                                            _P, _I64, _P, _SZ, _P]),
+    "llattn_block_bytes": (_SZ, [_BC, _I32]),
+    "llattn_block_fwd": (_I32, [_BC, _BP, _P, _P, _P, _SZ, _P, _P]),
+    "llattn_block_bwd": (_I32, [_BC, _BP, _P, _P, _P, _P, _BP, _P, _SZ, _P]),
+    "llattn_core_bytes": (_SZ, [_BC, _I32]),
+    "llattn_core_fwd": (_I32, [_BC, _CV, _P, _P, _P, _P, _P, _P, _SZ, _T, _P]),
+    "llattn_core_bwd": (_I32, [_BC, _CV, _P, _P, _P, _P, _T, _CV, _P, _P, _P, _P, _P, _SZ, _P]),
+    "llattn_ffn_bytes": (_SZ, [_FC, _I32]),
+    "llattn_ffn_fwd": (_I32, [_FC, _P, _P, _P, _P, _P, _P, _P, _SZ, _P, _P]),
+    "llattn_ffn_bwd": (_I32, [_FC, _P, _P, _P, _P, _P, _P, _P, _P, _P, _SZ, _P]),
 }
 
 _lib = None

@@ -17,8 +17,10 @@ from __future__ import annotations
 
 import torch
 
-from . import gemm
+from . import _lib as L
+from . import gemm, ops
 from .linear import pack_params, weight_grad
+from .steps import Ffn, ffn_forward, plain
 
 BF16 = torch.bfloat16
 
@@ -69,4 +71,14 @@ class _FeedForward(torch.autograd.Function):
 
 def feed_forward(x: torch.Tensor, w1: torch.nn.Linear, w2: torch.nn.Linear) -> torch.Tensor:
     """bf16 ``w2(gelu(w1(x)))`` on the GEMM kernels (GPU only; widths multiples of 8)."""
-    return _FeedForward.apply(x, w1.weight, w1.bias, w2.weight, w2.bias)
+    ps = (w1.weight, w1.bias, w2.weight, w2.bias)
+    dev = x.device
+    rows = x.numel() // max(1, x.shape[-1])
+    d, d_ff, d_out = x.shape[-1], ps[0].shape[0], ps[2].shape[0]
+    if x.is_cuda and not ops.observed() and 0 < rows < 1 << 31 and d % 8 == 0 and d_ff % 8 == 0 and d_out % 8 == 0 \
+            and ps[0].shape[1] == d and ps[2].shape[1] == d_ff and plain(x, dev, BF16) \
+            and all(p is None or plain(p, dev) for p in ps):
+        saved = torch.is_grad_enabled() and (x.requires_grad or any(p is not None and p.requires_grad for p in ps))
+        cfg = L.LlattnFfnCfg(rows, d, d_ff, d_out, int(saved))
+        return Ffn.apply(x, cfg, *ps) if saved else ffn_forward(x, cfg, *ps)[0]
+    return _FeedForward.apply(x, *ps)

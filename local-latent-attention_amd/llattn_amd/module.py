@@ -27,6 +27,7 @@ import torch
 import torch.nn as nn
 
 from . import _lib as L
+from . import ops, steps
 from .linear import pack_params, project, project_f32
 from .ops import LLAttnCore, _Prof, grad_heads_ok, heads_layout_ok, pool
 
@@ -107,6 +108,10 @@ class LocalLatentAttentionTriton(nn.Module):
             raise ValueError(f"expected d_model={self.d_model}, got input of width {D}")
         L.require_gpu(x)
         lay = self.layout(B, T)
+        if not self.profile_enabled and not ops.observed():
+            out = self._forward_native(x, lay)
+            if out is not None:
+                return out
         prof = _Prof(self.profile_enabled, x.device) if self.profile_enabled else None
         if prof is not None:
             prof.start()
@@ -158,6 +163,32 @@ class LocalLatentAttentionTriton(nn.Module):
         if not bf16:
             return project_f32(y, self.out)
         return project(y, self.out, packed=packed["out"], grad_heads=(T, lay.Dh, self.n_heads) if dy_heads else None)
+
+    def _forward_native(self, x: torch.Tensor, lay: L.Layout) -> Optional[torch.Tensor]:
+        """The whole block as one native call per direction (:mod:`llattn_amd.steps`), or None where the parameters
+        or the input are not what that takes (then the products are issued one by one, as under profiling)."""
+        B, T, D = x.shape
+        dev = x.device
+        bf16 = torch.is_autocast_enabled("cuda") and torch.get_autocast_dtype("cuda") == torch.bfloat16
+        dt = torch.bfloat16 if bf16 else torch.float32
+        lins = (self.qkv_proj, self.rq_proj, self.rkv_proj, self.r_out, self.out)
+        params = []
+        for m in lins:
+            params += (m.weight, m.bias)
+        params += (self.gate_local.weight, self.gate_remote.weight)
+        biases = [p is not None for p in params[1:10:2]]
+        if not steps.plain(x, dev, dt) or any(p is not None and not steps.plain(p, dev) for p in params) \
+                or any(b != biases[0] for b in biases):
+            return None
+        if bf16 and (D % 8 or lay.Dh % 8 or lay.Ldh % 8):
+            return None
+        macro = self.latent_query_block_size > 1
+        saved = torch.is_grad_enabled() and (x.requires_grad or any(p is not None and p.requires_grad for p in params))
+        cfg = L.LlattnBlockCfg(lay.shape(dt), D, int(macro), int(biases[0]), int(saved),
+                               int(bf16 and heads_layout_ok(lay, D, not macro)), int(ops._remote_heads(lay, dt)),
+                               int(bf16 and grad_heads_ok(B * T, D, D, lay.Dh)),
+                               int(bf16 and ops._latent_grad_heads(lay)))
+        return steps.Block.apply(x, cfg, *params) if saved else steps.block_forward(x, cfg, params)[0]
 
     def _packed_weights(self, macro: bool) -> dict:
         """The bf16 copies of every projection weight that this forward multiplies with (what bf16 autocast casts

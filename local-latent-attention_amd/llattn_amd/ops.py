@@ -24,6 +24,7 @@ import time
 import torch
 
 from . import _lib as L
+from . import steps
 from .gemm import input_grad_persistent, linear_f32, matmul_nn_f32, matmul_tn_f32
 from .linear import input_grad, linear_fwd, weight_grad
 
@@ -46,6 +47,15 @@ def _call(name: str, *args, work=None) -> None:
         end.record()
         EVENT_LOG.append((name, start, end, work))
     L.check(rc, name)
+
+
+_CALL = _call
+
+
+def observed() -> bool:
+    """Whether something looks at the C-ABI calls one by one: a log (``EVENT_LOG``) or a wrapper put in the place of
+    ``_call``.  The native steps (:mod:`llattn_amd.steps`), which make those calls themselves, are not used then."""
+    return EVENT_LOG is not None or _call is not _CALL
 
 
 def _empty(shape, dtype, device):
@@ -440,35 +450,57 @@ class LLAttnFunction(torch.autograd.Function):
         dt, device = Q.dtype, Q.device
         Q, K, V, GQ, GK, GV = (_contig_last(t.to(dt)) for t in (Q, K, V, GQ, GK, GV))
         gl, gr = _aligned_f32(gate_local_w), _aligned_f32(gate_remote_w)
-        y, ol, lse, w, lat, lse_lat, R = _core_forward(
-            lay, L.view_bhnd(Q), L.view_bhnd(K), L.view_bhnd(V), L.view_bhnd(GQ), L.view_bhnd(GK), L.view_bhnd(GV),
-            gl, gr, r_out_w, r_out_b, dt, device)
-        ctx.save_for_backward(Q, K, V, GQ, GK, GV, gl, gr, r_out_w, lat, lse_lat, R, ol, lse, w)
         ctx.lay, ctx.has_rb = lay, r_out_b is not None
         ctx.like = (gate_local_w, gate_remote_w)
         ctx.r_b_dtype = None if r_out_b is None else r_out_b.dtype
+        views = (L.view_bhnd(t) for t in (Q, K, V, GQ, GK, GV))
+        # one native call (steps.py); the products one by one while calls are observed, or for an r_out that is not
+        # plain fp32
+        ctx.native = not observed() and steps.plain(r_out_w, device) and \
+            (r_out_b is None or steps.plain(r_out_b, device)) and tuple(r_out_w.shape) == (H * Dh, Lh * Ldh) and \
+            (r_out_b is None or r_out_b.numel() == H * Dh) and (dt == torch.float32 or (Dh % 8 == 0 and Ldh % 8 == 0))
+        if ctx.native:
+            per_head = gl.dim() == 2 and gl.shape[0] > 1
+            ctx.cfg = L.LlattnBlockCfg(lay.shape(dt, per_head), H * Dh, 0, 0, 1, 0, int(_remote_heads(lay, dt)), 0,
+                                       int(dt == torch.bfloat16 and _latent_grad_heads(lay)))
+            y = _empty((B, S, H, Dh), dt, device)
+            kept = steps.core_forward(ctx.cfg, L.LlattnCoreViews(*views), gl, gr, r_out_w, r_out_b, L.view_bnhd(y),
+                                      device)
+            ctx.save_for_backward(Q, K, V, GQ, GK, GV, gl, gr, r_out_w, kept)
+            return y.permute(0, 2, 1, 3)
+        y, ol, lse, w, lat, lse_lat, R = _core_forward(lay, *views, gl, gr, r_out_w, r_out_b, dt, device)
+        ctx.save_for_backward(Q, K, V, GQ, GK, GV, gl, gr, r_out_w, lat, lse_lat, R, ol, lse, w)
         return y.permute(0, 2, 1, 3)
 
     @staticmethod
     def backward(ctx, dOut):
-        Q, K, V, GQ, GK, GV, gl, gr, r_w, lat, lse_lat, R, ol, lse, w = ctx.saved_tensors
+        Q, K, V, GQ, GK, GV, gl, gr, r_w, *kept = ctx.saved_tensors
         lay = ctx.lay
         dt, device = Q.dtype, Q.device
-        B, H, S, Dh = Q.shape
         dy = _contig_last(dOut.to(dt).permute(0, 2, 1, 3))  # [B, S, H, Dh], read by its strides
-        dQ, dK, dV = (_empty((B, S, H, Dh), dt, device) for _ in range(3))
-        dGQ = _empty((B, lay.n_q, lay.Lh, lay.Ldh), dt, device)
-        dGK = _empty((B, lay.n_chunks, lay.Lh, lay.Ldh), dt, device)
-        dGV = _empty((B, lay.n_chunks, lay.Lh, lay.Ldh), dt, device)
-        dgl, dgr, dr_w, dr_b = _core_backward(
-            lay, dy, L.view_bhnd(Q), L.view_bhnd(K), L.view_bhnd(V), L.view_bhnd(GQ),
-            L.view_bhnd(GK), L.view_bhnd(GV), gl, gr, r_w, ctx.has_rb, lat, lse_lat, R, ol, lse, w,
-            L.view_bnhd(dQ), L.view_bnhd(dK), L.view_bnhd(dV), L.view_bnhd(dGQ), L.view_bnhd(dGK), L.view_bnhd(dGV),
-            dt, device)
+        ins = (Q, K, V, GQ, GK, GV)
+        grads = [_grad_like(t) for t in ins]
+        views, dviews = [L.view_bhnd(t) for t in ins], [L.view_bhnd(t) for t in grads]
+        if ctx.native:
+            dgl, dgr, dr_w, dr_b = steps.core_backward(
+                ctx.cfg, L.LlattnCoreViews(*views), gl, gr, r_w, ctx.has_rb, kept[0],
+                L.view(dy, dy.stride(0), dy.stride(1), dy.stride(2)), L.LlattnCoreViews(*dviews), device)
+        else:
+            lat, lse_lat, R, ol, lse, w = kept
+            dgl, dgr, dr_w, dr_b = _core_backward(lay, dy, *views, gl, gr, r_w, ctx.has_rb, lat, lse_lat, R, ol, lse,
+                                                  w, *dviews, dt, device)
         like_l, like_r = ctx.like
-        t = lambda x: x.permute(0, 2, 1, 3)  # noqa: E731
-        return (t(dQ), t(dK), t(dV), t(dGQ), t(dGK), t(dGV), _gate_grad(dgl, like_l), _gate_grad(dgr, like_r),
+        return (*grads, _gate_grad(dgl, like_l), _gate_grad(dgr, like_r),
                 dr_w.to(r_w.dtype), None, None, None if dr_b is None else dr_b.to(ctx.r_b_dtype), None, None)
+
+
+def _grad_like(t: torch.Tensor) -> torch.Tensor:
+    """A gradient buffer for head tensor ``t [B, H, N, d]``: laid out like a contiguous ``t`` (autograd then keeps it
+    as it is; a permuted one it copies into ``t``'s layout), else as rows ``[B, N, H, d]``."""
+    if t.is_contiguous():
+        return torch.empty(t.shape, dtype=t.dtype, device=t.device)
+    B, H, N, d = t.shape
+    return torch.empty((B, N, H, d), dtype=t.dtype, device=t.device).permute(0, 2, 1, 3)
 
 
 def _contig_last(t: torch.Tensor) -> torch.Tensor:

@@ -1,0 +1,223 @@
+"""The native steps (one call per direction) against the Python path that issues the same products one by one: the
+same bits for every output and gradient.  The Python path runs while calls are logged."""
+from __future__ import annotations
+
+import contextlib
+
+import pytest
+import torch
+
+from gpu_helpers import require_cuda
+
+pytestmark = pytest.mark.gpu
+
+
+@contextlib.contextmanager
+def _logged():
+    from llattn_amd import ops
+    ops.EVENT_LOG = []
+    try:
+        yield ops.EVENT_LOG
+    finally:
+        ops.EVENT_LOG = None
+
+
+def _both(fn, entry):
+    """fn() by native steps (asserted: ``entry`` is called) and, logged, by the Python path."""
+    from llattn_amd import steps
+    seen, real = [], steps._call
+    steps._call = lambda name, *a: (seen.append(name), real(name, *a))[1]
+    try:
+        native = fn()
+    finally:
+        steps._call = real
+    assert entry in seen, seen
+    with _logged() as log:
+        python = fn()
+    assert log
+    return native, python
+
+
+def _same(native, python):
+    assert len(native) == len(python)
+    for i, (a, b) in enumerate(zip(native, python)):
+        assert (a is None) == (b is None), i
+        if a is not None:
+            assert a.dtype == b.dtype and a.shape == b.shape and torch.equal(a, b), i
+
+
+BLOCKS = [  # B, T, d_model, heads, latent width, latent heads, window, latents, query block
+    (2, 97, 64, 2, 16, 2, 16, 6, 0),      # one small tile, ragged
+    (1, 1, 128, 4, 64, 2, 64, 16, 0),     # one token
+    (1, 1, 128, 4, 64, 2, 64, 16, 64),    # one token, one query block
+    (3, 333, 128, 4, 64, 2, 64, 16, 0),
+    (2, 640, 256, 4, 32, 2, 128, 10, 64),  # query blocks that are the latent chunks: one pooling
+    (2, 650, 256, 4, 32, 2, 300, 10, 48),  # others
+    (2, 2100, 256, 4, 128, 2, 64, 16, 0),  # transposed weights (4200 rows), split-head storage
+    (16, 1024, 1408, 16, 512, 8, 64, 16, 0),  # gradients stored split-head as well
+]
+
+
+@pytest.mark.parametrize("cfg", BLOCKS)
+@pytest.mark.parametrize("bf16", [True, False])
+@pytest.mark.parametrize("bias", [True, False])
+def test_block_step_matches_python_path(cfg, bf16, bias):
+    from llattn_amd import LocalLatentAttentionTriton
+    B, T, D, H, Ld, Lh, W, N, qb = cfg
+    if not bf16 and B * T > 5000:
+        pytest.skip("the fp32 path has one layout")
+    dev = require_cuda()
+    print("case: block step", cfg, bf16, bias, flush=True)
+    torch.manual_seed(1)
+    m = LocalLatentAttentionTriton(D, H, Lh, Ld, N, W, bias=bias, latent_query_block_size=qb).to(dev)
+    g = torch.Generator(device=dev).manual_seed(2)
+    x = torch.randn(B, T, D, device=dev, generator=g).to(torch.bfloat16 if bf16 else torch.float32)
+    dy = torch.randn(B, T, D, device=dev, generator=g).to(x.dtype)
+
+    def cast():
+        return torch.autocast("cuda", dtype=torch.bfloat16, enabled=bf16)
+
+    def train(need_dx=True):
+        xx = x.clone().requires_grad_(need_dx)
+        m.zero_grad(set_to_none=True)
+        with cast():
+            y = m(xx)
+        y.backward(dy)
+        return [y.detach(), xx.grad, *(p.grad for p in m.parameters())]
+
+    native, python = _both(train, "llattn_block_bwd")
+    if bf16:
+        _same(native, python)
+    else:  # the Python path forms the poolings' input gradients apart and adds them; here they are added in place
+        _same(native[:1] + native[2:], python[:1] + python[2:])
+        assert float((native[1] - python[1]).norm()) <= 2.0 ** -22 * float(python[1].norm())
+    _same(*_both(lambda: train(False), "llattn_block_bwd"))
+
+    def infer():
+        with torch.no_grad(), cast():
+            return [m(x)]
+
+    a, b = _both(infer, "llattn_block_fwd")
+    _same(a, b)
+    assert torch.equal(a[0], native[0])
+
+
+def test_block_step_retained_graph_checkpoint_and_streams():
+    """Two backward passes of one graph, the block under non-reentrant checkpointing, and a pass on another stream
+    give the gradients of a plain pass."""
+    from torch.utils.checkpoint import checkpoint
+    from llattn_amd import LocalLatentAttentionTriton
+    dev = require_cuda()
+    torch.manual_seed(3)
+    m = LocalLatentAttentionTriton(128, 4, 2, 64, 16, 64).to(dev)
+    x = torch.randn(2, 200, 128, device=dev).bfloat16()
+    dy = torch.randn_like(x)
+
+    def grads(run):
+        xx = x.clone().requires_grad_()
+        m.zero_grad(set_to_none=True)
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            y = run(xx)
+        return xx, y
+
+    xx, y = grads(m)
+    y.backward(dy, retain_graph=True)
+    first = [xx.grad.clone()] + [p.grad.clone() for p in m.parameters()]
+    xx.grad = None
+    m.zero_grad(set_to_none=True)
+    y.backward(dy)
+    _same(first, [xx.grad] + [p.grad for p in m.parameters()])
+    xx, y = grads(lambda t: checkpoint(m, t, use_reentrant=False))
+    y.backward(dy)
+    _same(first, [xx.grad] + [p.grad for p in m.parameters()])
+    s = torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(s):
+        xx, y = grads(m)
+        y.backward(dy)
+    torch.cuda.current_stream().wait_stream(s)
+    _same(first, [xx.grad] + [p.grad for p in m.parameters()])
+
+
+def test_block_step_leaves_other_inputs_to_the_python_path():
+    """Inputs and parameters that the native step does not take give the results they gave: a strided and a float32
+    input under bf16 autocast, a misaligned parameter."""
+    from llattn_amd import LocalLatentAttentionTriton, steps
+    dev = require_cuda()
+    torch.manual_seed(4)
+    m = LocalLatentAttentionTriton(128, 4, 2, 64, 16, 64).to(dev)
+    x = torch.randn(2, 96, 256, device=dev).bfloat16()
+    called, real = [], steps._call
+    steps._call = lambda name, *a: (called.append(name), real(name, *a))[1]
+    try:
+        with torch.no_grad(), torch.autocast("cuda", dtype=torch.bfloat16):
+            ref = m(x[..., :128].contiguous())
+            assert called
+            del called[:]
+            assert torch.equal(m(x[..., :128]), ref)
+            wide = m(x[..., :128].float().contiguous())  # pooled in float32 before the rounding
+            assert float((wide - ref).float().norm() / ref.float().norm()) < 0.02
+            odd = torch.empty(m.out.weight.numel() + 1, device=dev)[1:].view_as(m.out.weight).copy_(m.out.weight)
+            m.out.weight = torch.nn.Parameter(odd)
+            assert torch.equal(m(x[..., :128].contiguous()), ref)
+        assert not called
+    finally:
+        steps._call = real
+
+
+@pytest.mark.parametrize("contiguous", [True, False])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("qb,T,per_head", [(0, 300, False), (48, 500, True), (0, 2100, False)])
+def test_op_step_matches_python_path(contiguous, dtype, qb, T, per_head):
+    from llattn_amd import LLAttnFunction
+    dev = require_cuda()
+    print("case: op step", contiguous, dtype, qb, T, per_head, flush=True)
+    B, H, Dh, Lh, Ldh, chunk = 2, 3, 40, 2, 64, 50
+    g = torch.Generator(device=dev).manual_seed(T)
+    nq = -(-T // qb) if qb > 1 else T
+    nc = -(-T // chunk)
+
+    def heads(h, n, d):
+        t = torch.randn(B, n, h, d, device=dev, generator=g).to(dtype).transpose(1, 2)
+        return t.contiguous() if contiguous else t
+
+    ins = [heads(H, T, Dh) for _ in range(3)] + [heads(Lh, nq, Ldh), heads(Lh, nc, Ldh), heads(Lh, nc, Ldh)]
+    ins += [torch.randn(H if per_head else 1, Dh, device=dev, generator=g) for _ in range(2)]
+    ins += [torch.randn(H * Dh, Lh * Ldh, device=dev, generator=g) * 0.1]
+    rb, dO = torch.randn(H * Dh, device=dev, generator=g), heads(H, T, Dh)
+
+    def run():
+        leaves = [t.detach().requires_grad_() for t in ins]
+        b = rb.detach().requires_grad_()
+        y = LLAttnFunction.apply(*leaves, 64, chunk, b, 128, qb)
+        y.backward(dO)
+        for t in leaves:
+            assert t.grad.stride() == t.stride()
+        return [y.detach(), *(t.grad for t in leaves), b.grad]
+
+    _same(*_both(run, "llattn_core_bwd"))
+
+
+@pytest.mark.parametrize("shape,d_ff,bias", [((3, 7, 64), 128, True), ((2, 600, 128), 256, False),
+                                             ((1, 1000, 1408), 4096, True), ((2, 2100, 256), 1024, True)])
+def test_ffn_step_matches_python_path(shape, d_ff, bias):
+    from llattn_amd.ffn import feed_forward
+    dev = require_cuda()
+    print("case: ffn step", shape, d_ff, bias, flush=True)
+    torch.manual_seed(5)
+    w1, w2 = torch.nn.Linear(shape[-1], d_ff, bias=bias).to(dev), torch.nn.Linear(d_ff, shape[-1], bias=bias).to(dev)
+    x, dy = (torch.randn(shape, device=dev).bfloat16() for _ in range(2))
+
+    def run(grad=True):
+        xx = x.clone().requires_grad_(grad)
+        for p in (*w1.parameters(), *w2.parameters()):
+            p.grad = None
+        with torch.set_grad_enabled(grad), torch.autocast("cuda", dtype=torch.bfloat16):
+            y = feed_forward(xx, w1, w2)
+        if not grad:
+            return [y]
+        y.backward(dy)
+        return [y.detach(), xx.grad, *(p.grad for p in (*w1.parameters(), *w2.parameters()))]
+
+    _same(*_both(run, "llattn_ffn_bwd"))
+    _same(*_both(lambda: run(False), "llattn_ffn_fwd"))

@@ -1,0 +1,60 @@
+"""CPU tests of the native steps' interface (include/llattn_steps.h): nothing is launched."""
+from __future__ import annotations
+
+import ctypes
+import re
+import shutil
+import subprocess
+
+import pytest
+
+from conftest import REPO
+
+
+def test_steps_header_matches_the_binding(tmp_path):
+    from llattn_amd import _lib as L
+    text = (REPO / "include" / "llattn_steps.h").read_text()
+    names = set(re.findall(r"^(?:int32_t|size_t)\s+(llattn_\w+)\s*\(", text, re.M))
+    assert names == set(L.STEP_SIGNATURES) and all(hasattr(L.load(), n) for n in names)
+    if shutil.which("gcc") is None:
+        pytest.skip("gcc not available")
+    structs = {"llattn_block_cfg": L.LlattnBlockCfg, "llattn_block_params": L.LlattnBlockParams,
+               "llattn_block_grads": L.LlattnBlockParams, "llattn_core_views": L.LlattnCoreViews,
+               "llattn_ffn_cfg": L.LlattnFfnCfg}
+    lines = ["#include <stddef.h>", "#include <stdio.h>", '#include "llattn_steps.h"', "int main(void) {"]
+    for name, cls in structs.items():
+        lines.append(f'  printf("%zu ", sizeof({name}));')
+        lines += [f'  printf("%zu ", offsetof({name}, {f}));' for f, _ in cls._fields_]
+    src = tmp_path / "layout.c"
+    src.write_text("\n".join(lines) + "\n  return 0;\n}\n")
+    subprocess.run(["gcc", "-std=c11", f"-I{REPO / 'include'}", str(src), "-o", str(tmp_path / "layout")], check=True)
+    got = [int(n) for n in subprocess.run([str(tmp_path / "layout")], check=True, capture_output=True, text=True).stdout.split()]
+    want = []
+    for cls in structs.values():
+        want += [ctypes.sizeof(cls)] + [getattr(cls, f).offset for f, _ in cls._fields_]
+    assert got == want
+
+
+def test_step_sizes_and_refusals():
+    from llattn_amd import _lib as L
+    from llattn_amd._lib import resolve_layout
+    import torch
+    lib, ref = L.load(), ctypes.byref
+    lay = resolve_layout(2, 100, 128, 4, 64, 2, 64, 256, 16, 0)
+    cfg = L.LlattnBlockCfg(lay.shape(torch.bfloat16), 128, 0, 1, 1, 1, 0, 0, 0)
+    kept = lib.llattn_block_bytes(ref(cfg), 0)
+    # the projection output, the attention outputs and the weight copies at least
+    assert kept > 200 * (3 * 128 + 64) * 2 + 4 * 200 * 128 * 2 + (5 * 128 * 128) * 2
+    cfg.saved = 0
+    assert 0 < lib.llattn_block_bytes(ref(cfg), 0) < kept
+    cfg.saved = 1
+    buf = ctypes.create_string_buffer(64)
+    p = L.LlattnBlockParams()
+    small = lib.llattn_block_bwd(ref(cfg), ref(p), buf, buf, buf, None, ref(p), buf, 16, None)
+    assert small in (L.ERR_WORKSPACE, L.ERR_LAYOUT)
+    cfg.d_model = 136
+    assert lib.llattn_block_bytes(ref(cfg), 0) == 0
+    assert lib.llattn_block_fwd(ref(cfg), ref(p), buf, buf, None, 0, buf, None) == L.ERR_SHAPE
+    assert lib.llattn_block_fwd(None, ref(p), buf, buf, None, 0, buf, None) == L.ERR_SHAPE
+    f = L.LlattnFfnCfg(0, 64, 128, 64, 1)
+    assert lib.llattn_ffn_bytes(ref(f), 0) == 0 and b"positive" in lib.llattn_last_error()
