@@ -37,226 +37,10 @@
 // operand past K lie beyond its buffer extent and read zero by themselves; a k-contiguous operand
 // (K a multiple of 8) masks the lanes whose 8 k values start at or past K with an out-of-range
 // offset (kmask), so no lane reads the next row's elements.
-#include <type_traits>
-
-#include "llattn_abi.h"
-#include "llattn_device.h"
-#include "llattn_heads.h"
+#include "llattn_gemm.h"
 
 namespace llattn {
 namespace gemm {
-
-constexpr int BM = 256, BN = 256;  // output tile
-
-enum Epi { EPI_BF16 = 0, EPI_F32 = 1, EPI_PART = 2 };
-
-struct GemmArgs {
-  int M, N, K, k_pairs, n_split, tiles_m, tiles_n, accumulate;  // k_pairs: 64-wide k steps, ceil(K / 64)
-  const uint16_t* A; int64_t lda, a_bytes;
-  const uint16_t* B; int64_t ldb, b_bytes;
-  void* C; int64_t ldc;
-  const float* bias;
-  float* part;     // split-K partials [S][M][N], then (rowsum) [S][M]
-  float* rowsum;   // fp32 [M] or null: sum_k A(m, k), from a column of ones in place of B's column N
-  // bf16 C only: C[m][n] += ra[(m / T) * n_seg + (m % T) / seg][n] / divisor for each of up to two addends
-  const uint16_t* ra_ptr[2];
-  int64_t ra_ld[2];
-  int ra_T[2], ra_seg[2], ra_nseg[2], ra_div[2];
-  // bf16 C only: LLATTN_ACT_GELU writes C = gelu(pre), aux = gelu'(pre); LLATTN_ACT_MUL_AUX scales C by aux
-  int act;
-  uint16_t* aux;
-  int64_t ld_aux;
-  HeadsMap ch;  // bf16 C stored split-head (ch.T > 0; persistent kernel)
-};
-
-// Exact GELU u * Phi(u) of the reference FeedForward (reference models.py:57, F.gelu) and its derivative
-// Phi(u) + u phi(u), in fp32.  erf comes from Abramowitz & Stegun 7.1.26 (Handbook of Mathematical
-// Functions): erf(z) = 1 - t (a1 + t (a2 + t (a3 + t (a4 + t a5)))) exp(-z^2), t = 1 / (1 + p z), z >= 0,
-// absolute error below 1.5e-7 (far under the bf16 rounding of the outputs).  With z = |u| / sqrt(2),
-// exp(-z^2) = exp(-u^2 / 2) is also the Gaussian density's exponential, so Phi and phi share one exp:
-//   q = t P(t) exp(-u^2/2) / 2,  Phi(u) = 1 - q (u >= 0) or q (u < 0),  phi(u) = exp(-u^2/2) / sqrt(2 pi).
-struct NormalCdf {
-  float cdf, pdf;
-};
-__device__ __forceinline__ NormalCdf normal_cdf_pdf(float u) {
-  constexpr float p = 0.3275911f, a1 = 0.254829592f, a2 = -0.284496736f, a3 = 1.421413741f,
-                  a4 = -1.453152027f, a5 = 1.061405429f;
-  const float z = fabsf(u) * 0.70710678118654752f;
-  const float t = __builtin_amdgcn_rcpf(fmaf(p, z, 1.f));
-  const float poly = t * fmaf(t, fmaf(t, fmaf(t, fmaf(t, a5, a4), a3), a2), a1);
-  const float e = __builtin_amdgcn_exp2f(-0.5f * 1.4426950408889634f * u * u);  // exp(-u^2 / 2)
-  const float q = 0.5f * poly * e;
-  return NormalCdf{u >= 0.f ? 1.f - q : q, e * 0.39894228040143268f};
-}
-// gelu(u) and gelu'(u) of one value
-__device__ __forceinline__ void gelu_pair(float u, float& g, float& gp) {
-  const NormalCdf n = normal_cdf_pdf(u);
-  g = u * n.cdf;
-  gp = fmaf(u, n.pdf, n.cdf);
-}
-// Eight bf16 pre-activations (packed pairs; the activation acts on the bf16-rounded value, as bf16
-// autocast does) -> gelu and gelu' as bf16.
-__device__ __forceinline__ void gelu_bf16x8(uint4 x, uint4& g, uint4& gp) {
-  const uint32_t xs[4] = {x.x, x.y, x.z, x.w};
-  uint32_t o[4], d[4];
-#pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    float g0, g1, p0, p1;
-    gelu_pair(__uint_as_float(xs[e] << 16), g0, p0);
-    gelu_pair(__uint_as_float(xs[e] & 0xffff0000u), g1, p1);
-    o[e] = pack_bf16x2(g0, g1);
-    d[e] = pack_bf16x2(p0, p1);
-  }
-  g = make_uint4(o[0], o[1], o[2], o[3]);
-  gp = make_uint4(d[0], d[1], d[2], d[3]);
-}
-// bf16 x * s elementwise (eight packed values each)
-__device__ __forceinline__ uint4 mul_bf16x8(uint4 x, uint4 s) {
-  const uint32_t xs[4] = {x.x, x.y, x.z, x.w}, ss[4] = {s.x, s.y, s.z, s.w};
-  uint32_t o[4];
-#pragma unroll
-  for (int e = 0; e < 4; ++e)
-    o[e] = pack_bf16x2(__uint_as_float(xs[e] << 16) * __uint_as_float(ss[e] << 16),
-                       __uint_as_float(xs[e] & 0xffff0000u) * __uint_as_float(ss[e] & 0xffff0000u));
-  return make_uint4(o[0], o[1], o[2], o[3]);
-}
-
-// Row of addend q (0, 1) that C row m reads, and its scale (the pooled gradient broadcast to its tokens).
-__device__ __forceinline__ const uint16_t* rowadd_row(const GemmArgs& a, int q, int m, float& sc) {
-  const int T = a.ra_T[q], t = m % T, s = t / a.ra_seg[q];
-  sc = a.ra_div[q] == LLATTN_DIV_COUNT ? 1.f / (float)(min((s + 1) * a.ra_seg[q], T) - s * a.ra_seg[q])
-     : a.ra_div[q] == LLATTN_DIV_SEG ? 1.f / (float)a.ra_seg[q] : 1.f;
-  return a.ra_ptr[q] + ((int64_t)(m / T) * a.ra_nseg[q] + s) * a.ra_ld[q];
-}
-__device__ __forceinline__ void add_bf16x4(uint2 u, float sc, float (&v)[4]) {
-  v[0] += sc * __uint_as_float(u.x << 16);
-  v[1] += sc * __uint_as_float(u.x & 0xffff0000u);
-  v[2] += sc * __uint_as_float(u.y << 16);
-  v[3] += sc * __uint_as_float(u.y & 0xffff0000u);
-}
-__device__ __forceinline__ void rowadd4(const GemmArgs& a, int q, int m, int c, float (&v)[4]) {
-  float sc;
-  const uint16_t* p = rowadd_row(a, q, m, sc);
-  add_bf16x4(*reinterpret_cast<const uint2*>(p + c), sc, v);
-}
-
-typedef __attribute__((address_space(3))) void lds_void;
-typedef __attribute__((address_space(1))) const void gbl_void;
-typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
-
-typedef int i32x4 __attribute__((ext_vector_type(4)));
-
-// LDS byte address of a pointer into shared memory
-__device__ __forceinline__ uint32_t lds_addr(const void* p) {
-  return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)p;
-}
-
-constexpr int kRsrcWord3 = 0x00020000;  // raw buffer, gfx9 family
-
-// One wave copies 64 x 16 bytes from global memory into the 1 KB LDS block at
-// `dst` (lane i lands at dst + 16 i) with buffer_load_dwordx4 ... lds: the
-// step's base address lives in the scalar buffer descriptor and each lane
-// adds its fixed 32-bit offset.  Offsets past the descriptor's extent read 0.
-// Written as inline asm so that the compiler does not see an LDS write in
-// flight: it would otherwise make every later LDS read wait for all of it
-// (vmcnt(0)), although the reads target another stage.  The main loop waits
-// for these loads itself (vmcnt) before the barrier that publishes them.
-// The descriptor and the LDS address are wave-uniform at every call; readfirstlane states it for the
-// cases where the compiler cannot prove it (it then keeps them in SGPRs, as the instruction requires).
-__device__ __forceinline__ void dma_block(const i32x4& rs, uint32_t off, const unsigned char* dst) {
-  const i32x4 srs = {__builtin_amdgcn_readfirstlane(rs[0]), __builtin_amdgcn_readfirstlane(rs[1]),
-                     __builtin_amdgcn_readfirstlane(rs[2]), __builtin_amdgcn_readfirstlane(rs[3])};
-  const uint32_t sdst = __builtin_amdgcn_readfirstlane(lds_addr(dst));
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds"
-               :
-               : "v"(off), "s"(srs), "s"(sdst)
-               : "memory", "m0");
-}
-
-// s_waitcnt immediates (gfx9 encoding: vmcnt [3:0]+[15:14], expcnt [6:4], lgkmcnt [11:8]);
-// issued through the builtin so that the compiler's own wait insertion sees them.
-constexpr int wait_vm(int n) { return (n & 15) | ((n >> 4) << 14) | 0x0070 | 0x0F00; }       // vmcnt(n)
-constexpr int wait_vm_lgkm0(int n) { return (n & 15) | ((n >> 4) << 14) | 0x0070; }        // vmcnt(n) lgkmcnt(0)
-
-// An offset past every operand extent (operands are below 4 GiB - 16 bytes): the lane reads zero.
-constexpr uint32_t kOffPastK = 0xFFFFFFF0u;
-// A k-contiguous lane's offset for a step whose K tail starts `klim` elements in, its chunk starting at kc.
-__device__ __forceinline__ uint32_t kmask(uint32_t off, int kc, int klim) { return kc < klim ? off : kOffPastK; }
-
-// Buffer descriptor of an operand from step k0 on (`bytes`: storage extent of the operand).
-template <bool KMAJ>
-__device__ __forceinline__ i32x4 step_rsrc(const uint16_t* base, int64_t ld, int64_t bytes, int k0) {
-  const int64_t skip = (KMAJ ? (int64_t)k0 : (int64_t)k0 * ld) * 2;
-  const uint64_t addr = reinterpret_cast<uint64_t>(base) + (uint64_t)skip;
-  // a step wholly past K can start beyond a small operand's end: extent 0, every lane reads zero
-  const int64_t ext = bytes > skip ? bytes - skip : 0;
-  return i32x4{(int)(uint32_t)addr, (int)((addr >> 32) & 0xffff), (int)(uint32_t)ext, kRsrcWord3};
-}
-
-// 64-k LDS stages (two of 64 KB), shared by gemm_kernel and the persistent kernel.  k-contiguous tiles:
-// 256 rows of 128 bytes, 16-byte chunk c of row r at slot c ^ pswz(r) (A fragments read rows o16 + r, eight
-// consecutive rows per LDS cycle -> r & 7; permuted B fragments read rows o16 + 8 (r / 4) + r % 4 ->
-// (r & 3) | (bit 3 of the row at bit 2); both conflict-free).  mn-contiguous tiles: 64 k-rows of 512 bytes,
-// chunk c of k-row k at c ^ 2 (k & 3) (transposing reads, conflict-free).
-constexpr int PBK = 64;                  // k per LDS stage
-constexpr int PTILE = BM * PBK * 2;      // 32 KB per operand per stage
-constexpr int PSTAGE = 2 * PTILE;        // A then B
-constexpr int PDMA = PTILE / 1024 / 4;   // 1 KB DMA blocks per wave per operand and step (8)
-
-template <bool PERM>
-__device__ __forceinline__ int pswz(int row) {
-  return PERM ? ((row & 3) | (((row >> 3) & 1) << 2)) : (row & 7);
-}
-
-// Byte offsets (relative to the operand base at the step's first k) of this lane's 16-byte chunk in each
-// of the wave's 8 DMA blocks of a 64-k operand tile (rows / columns [o0, o0 + 256)).  k-contiguous: block i
-// = rows 8 (8 wave + i) .. + 7, lane -> row + lane / 8, LDS slot lane % 8 receives the row's chunk
-// (lane % 8) ^ pswz(row); rows past omax are clamped to a valid row (their outputs are never stored).
-// mn-contiguous: block i = k-rows 2 (8 wave + i) + lane / 32, 32 chunks each; columns clamped likewise.
-// kc: first k of the lane's chunk (k-contiguous K tail; mn-contiguous rows past K lie beyond the extent).
-template <bool KMAJ, bool PERM = false>
-__device__ __forceinline__ void tile_offsets64(uint32_t (&off)[PDMA], int (&kc)[PDMA], int64_t ld, int o0, int omax,
-                                               int wave, int lane) {
-#pragma unroll
-  for (int i = 0; i < PDMA; ++i) {
-    const int bi = wave * PDMA + i;
-    if constexpr (KMAJ) {
-      const int row = 8 * bi + (lane >> 3);
-      const int c = (lane & 7) ^ pswz<PERM>(row);
-      off[i] = (uint32_t)(((int64_t)min(o0 + row, omax - 1) * ld + 8 * c) * 2);
-      kc[i] = 8 * c;
-    } else {
-      const int k = 2 * bi + (lane >> 5);
-      const int c = (lane & 31) ^ (2 * (k & 3));
-      off[i] = (uint32_t)(((int64_t)k * ld + min(o0 + 8 * c, omax - 8)) * 2);
-      kc[i] = 0;
-    }
-  }
-}
-
-// 8 k values (32h + 8g .. + 7 of a 64-k stage) of tile row / column o16 + r for lane (r, g).  PERM
-// (k-contiguous B only): lane r reads row o16 + 8 (r / 4) + r % 4 instead, so that with o16 = 32p + 4u the
-// output columns a lane accumulates for the block pair (u = 0, 1) are 8 consecutive ones.
-template <bool KMAJ, bool PERM = false>
-__device__ __forceinline__ bf16x8 frag64(const unsigned char* tile, int o16, int r, int g, int h) {
-  if constexpr (KMAJ) {
-    const int row = PERM ? o16 + 8 * (r >> 2) + (r & 3) : o16 + r;
-    return *reinterpret_cast<const bf16x8*>(tile + row * 128 + (((4 * h + g) ^ pswz<PERM>(row)) << 4));
-  } else {
-    // transposing reads: the 16 lanes of group g supply k-rows kb + j/4, 8 bytes at column o16 + 4(j%4);
-    // lane r receives column o16 + r of those four rows
-    const int kb = 32 * h + 8 * g;
-    const int col = o16 + 4 * (r & 3), chunk = col >> 3, inner = (col & 7) << 1;
-    bf16x4 hv[2];
-#pragma unroll
-    for (int half = 0; half < 2; ++half) {
-      const int k = kb + 4 * half + (r >> 2);
-      const unsigned char* p = tile + k * 512 + ((chunk ^ (2 * (k & 3))) << 4) + inner;
-      hv[half] = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((__attribute__((address_space(3))) bf16x4*)(p));
-    }
-    return bf16x8{hv[0][0], hv[0][1], hv[0][2], hv[0][3], hv[1][0], hv[1][1], hv[1][2], hv[1][3]};
-  }
-}
 
 // RS: row sums of A for an N with no spare column (a multiple of 256): every lane adds the 8 k values of each of
 // its A fragments into one fp32 sum per fragment block (v_dot2 against a pair of ones, 32 per 32-k sub-step,
@@ -984,218 +768,6 @@ void launch(const GemmArgs& a, int S, int c_dtype, hipStream_t st) {
 }
 
 
-// ---------------------------------------------------------------------------------------------------------
-// Small products: the pooled-latent projection rkv_proj (reference models.py:333-342) and its backward have
-// a few hundred rows or a contraction of a few hundred (config 2: 256 x 1024 x 1408 and its transposes).
-// On the 256 x 256 tiles they run as ~20 workgroups whose pipelines never fill.  Here: 64 x 64 output tiles,
-// one 256-thread workgroup each (4 waves of 32 x 32), the whole contraction per workgroup in 64-wide k
-// chunks staged through two LDS panel buffers (the next chunk's loads in flight during the current chunk's
-// MFMAs).  Either operand may be k- or m/n-contiguous: k-contiguous rows are copied as 16-byte pieces,
-// m/n-contiguous ones are transposed on their way into LDS, so fragments are always k-contiguous.  LDS rows
-// of 64 k (128 bytes) with 16-byte chunk c of row r at c ^ ((r >> 1) & 7): conflict-free ds_read_b128.
-// ---------------------------------------------------------------------------------------------------------
-constexpr int SBT = 64, SBK = 64;
-
-__device__ __forceinline__ int sswz(int row) { return (row >> 1) & 7; }
-
-// This thread's two 16-byte pieces of a 64 x 64 operand panel (rows o0 .., k from k0) -> registers.
-template <bool KMAJ>
-__device__ __forceinline__ void small_load(uint4 (&v)[2], const uint16_t* base, int64_t ld, int o0, int omax, int k0,
-                                           int K, int tid) {
-#pragma unroll
-  for (int u = 0; u < 2; ++u) {
-    const int q = tid + 256 * u;
-    if constexpr (KMAJ) {  // piece: row q / 8, k 8 (q % 8) .. +7
-      const int row = o0 + (q >> 3), k = k0 + 8 * (q & 7);
-      v[u] = (row < omax && k < K) ? *reinterpret_cast<const uint4*>(base + (int64_t)row * ld + k)
-                                   : make_uint4(0u, 0u, 0u, 0u);
-    } else {  // piece: k-row q / 8, rows 8 (q % 8) .. +7 of the panel
-      const int k = k0 + (q >> 3), row = o0 + 8 * (q & 7);
-      v[u] = (k < K && row < omax) ? *reinterpret_cast<const uint4*>(base + (int64_t)k * ld + row)
-                                   : make_uint4(0u, 0u, 0u, 0u);
-    }
-  }
-}
-template <bool KMAJ>
-__device__ __forceinline__ void small_store(const uint4 (&v)[2], unsigned char* panel, int tid) {
-#pragma unroll
-  for (int u = 0; u < 2; ++u) {
-    const int q = tid + 256 * u;
-    if constexpr (KMAJ) {
-      const int row = q >> 3, c = q & 7;
-      *reinterpret_cast<uint4*>(panel + row * 128 + ((c ^ sswz(row)) << 4)) = v[u];
-    } else {  // eight rows of one k: one element each
-      const int k = q >> 3, r0 = 8 * (q & 7);
-      const uint32_t w[4] = {v[u].x, v[u].y, v[u].z, v[u].w};
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const int row = r0 + e;
-        *reinterpret_cast<uint16_t*>(panel + row * 128 + (((k >> 3) ^ sswz(row)) << 4) + 2 * (k & 7)) =
-            (uint16_t)((e & 1) ? (w[e >> 1] >> 16) : (w[e >> 1] & 0xffffu));
-      }
-    }
-  }
-}
-
-template <bool AK, bool BKM, int EPI>
-__global__ __launch_bounds__(256) void gemm_small_kernel(const GemmArgs a) {
-  __shared__ __align__(16) unsigned char As[2][SBT * 128], Bs[2][SBT * 128];
-  const int tid = threadIdx.x, lane = tid & 63, r = lane & 15, g = lane >> 4;
-  const int wave = tid >> 6, wm = wave >> 1, wn = wave & 1;
-  const int tn_count = (a.N + SBT - 1) / SBT, tiles = ((a.M + SBT - 1) / SBT) * tn_count;
-  // EPI_PART: split blockIdx / tiles takes chunks [s C / S, (s+1) C / S) of the C 64-wide chunks
-  const int split = EPI == EPI_PART ? blockIdx.x / tiles : 0, t = EPI == EPI_PART ? blockIdx.x % tiles : blockIdx.x;
-  const int tm = t / tn_count, tn = t % tn_count;
-  const int m0 = tm * SBT, n0 = tn * SBT;
-  const bool want_rowsum = a.rowsum && tn == 0;
-  const int call = (a.K + SBK - 1) / SBK;
-  const int cbeg = EPI == EPI_PART ? split * call / a.n_split : 0;
-  const int nchunks = (EPI == EPI_PART ? (split + 1) * call / a.n_split : call) - cbeg;
-  const int kbase = cbeg * SBK;
-  f32x4 acc[2][2];
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  float rs = 0.f;  // threads 0..63: the row sum of A row m0 + tid
-  // chunk c's loads land in register set c % 4: four chunks in flight ahead of the MFMAs
-  uint4 va[4][2], vb[4][2];
-#pragma unroll
-  for (int d = 0; d < 4; ++d) {
-    if (d < nchunks) {
-      small_load<AK>(va[d], a.A, a.lda, m0, a.M, kbase + d * SBK, a.K, tid);
-      small_load<BKM>(vb[d], a.B, a.ldb, n0, a.N, kbase + d * SBK, a.K, tid);
-    }
-  }
-  auto chunk = [&](int c, uint4 (&ra)[2], uint4 (&rb)[2]) {
-    unsigned char* pa = As[c & 1];
-    unsigned char* pb = Bs[c & 1];
-    small_store<AK>(ra, pa, tid);
-    small_store<BKM>(rb, pb, tid);
-    __syncthreads();  // the panels of chunk c are complete; the other buffer (chunk c-1) is no longer read
-    if (c + 4 < nchunks) {  // this register set is free again: chunk c + 4
-      small_load<AK>(ra, a.A, a.lda, m0, a.M, kbase + (c + 4) * SBK, a.K, tid);
-      small_load<BKM>(rb, a.B, a.ldb, n0, a.N, kbase + (c + 4) * SBK, a.K, tid);
-    }
-    if (want_rowsum && tid < SBT) {
-#pragma unroll
-      for (int cc = 0; cc < 8; ++cc) {
-        const uint4 x = *reinterpret_cast<const uint4*>(pa + tid * 128 + ((cc ^ sswz(tid)) << 4));
-        const uint32_t w[4] = {x.x, x.y, x.z, x.w};
-#pragma unroll
-        for (int e = 0; e < 4; ++e) rs += __uint_as_float(w[e] << 16) + __uint_as_float(w[e] & 0xffff0000u);
-      }
-    }
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {  // two 32-wide k steps per chunk
-      bf16x8 fa[2], fb[2];
-#pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        const int row = wm * 32 + 16 * i + r, cc = 4 * h + g;
-        fa[i] = *reinterpret_cast<const bf16x8*>(pa + row * 128 + ((cc ^ sswz(row)) << 4));
-      }
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        const int row = wn * 32 + 16 * j + r, cc = 4 * h + g;
-        fb[j] = *reinterpret_cast<const bf16x8*>(pb + row * 128 + ((cc ^ sswz(row)) << 4));
-      }
-#pragma unroll
-      for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[j], fa[i], acc[i][j], 0, 0, 0);
-    }
-    __syncthreads();  // every wave is done with buffer c & 1 before chunk c + 2 overwrites it
-  };
-  for (int c = 0; c < nchunks; c += 4) {
-    chunk(c, va[0], vb[0]);
-    if (c + 1 < nchunks) chunk(c + 1, va[1], vb[1]);
-    if (c + 2 < nchunks) chunk(c + 2, va[2], vb[2]);
-    if (c + 3 < nchunks) chunk(c + 3, va[3], vb[3]);
-  }
-  if (want_rowsum && tid < SBT && m0 + tid < a.M) {
-    if constexpr (EPI == EPI_PART) a.part[(int64_t)a.n_split * a.M * a.N + (int64_t)split * a.M + m0 + tid] = rs;
-    else a.rowsum[m0 + tid] = rs;
-  }
-  // lane (r, g) holds C[m0 + wm*32 + 16i + r][n0 + wn*32 + 16j + 4g + e]
-#pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    const int col = n0 + wn * 32 + 16 * j + 4 * g;
-    if (col >= a.N) continue;
-    const float4 b4 = (EPI != EPI_PART && a.bias) ? *reinterpret_cast<const float4*>(a.bias + col)
-                                                   : make_float4(0.f, 0.f, 0.f, 0.f);
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const int row = m0 + wm * 32 + 16 * i + r;
-      if (row >= a.M) continue;
-      float v[4] = {acc[i][j][0] + b4.x, acc[i][j][1] + b4.y, acc[i][j][2] + b4.z, acc[i][j][3] + b4.w};
-      if constexpr (EPI == EPI_PART) {  // this split's fp32 partial [split][M][N]
-        *reinterpret_cast<float4*>(a.part + ((int64_t)split * a.M + row) * a.N + col) = make_float4(v[0], v[1], v[2], v[3]);
-      } else if constexpr (EPI == EPI_BF16) {
-        uint16_t* p = static_cast<uint16_t*>(a.C) + (int64_t)row * a.ldc + col;
-        if (a.accumulate) {
-          float o[4];
-          load4<uint16_t>(p, o);
-#pragma unroll
-          for (int e = 0; e < 4; ++e) v[e] += o[e];
-        }
-        store4<uint16_t>(p, v);
-      } else {
-        float* p = static_cast<float*>(a.C) + (int64_t)row * a.ldc + col;
-        if (a.accumulate) {
-          const float4 o = *reinterpret_cast<const float4*>(p);
-          v[0] += o.x; v[1] += o.y; v[2] += o.z; v[3] += o.w;
-        }
-        *reinterpret_cast<float4*>(p) = make_float4(v[0], v[1], v[2], v[3]);
-      }
-    }
-  }
-}
-
-template <bool AK, bool BKM>
-void launch_small(const GemmArgs& a, int c_dtype, hipStream_t st) {
-  const int tiles = ((a.M + SBT - 1) / SBT) * ((a.N + SBT - 1) / SBT);
-  const dim3 block(256);
-  if (a.n_split > 1) {  // K splits: fp32 partials, then the ordered reduction of the large products
-    hipLaunchKernelGGL((gemm_small_kernel<AK, BKM, EPI_PART>), dim3(tiles * a.n_split), block, 0, st, a);
-    const int64_t quads = (int64_t)a.M * (a.N / 4) + (a.rowsum ? a.M : 0);
-    const dim3 rg((unsigned)((quads + 255) / 256));
-    if (c_dtype == LLATTN_F32) hipLaunchKernelGGL((splitk_reduce_kernel<EPI_F32>), rg, block, 0, st, a, a.n_split);
-    else hipLaunchKernelGGL((splitk_reduce_kernel<EPI_BF16>), rg, block, 0, st, a, a.n_split);
-    return;
-  }
-  if (c_dtype == LLATTN_F32) hipLaunchKernelGGL((gemm_small_kernel<AK, BKM, EPI_F32>), dim3(tiles), block, 0, st, a);
-  else hipLaunchKernelGGL((gemm_small_kernel<AK, BKM, EPI_BF16>), dim3(tiles), block, 0, st, a);
-}
-
-// The small-tile path: no K split requested, no activation or row addends, an output of at most 32 tiles of
-// 256 x 256 with one side at most 1024, and a contraction of at most 4096.
-bool use_small(const llattn_gemm_desc* d) {
-  const int64_t tiles = (int64_t)((d->M + BM - 1) / BM) * ((d->N + BN - 1) / BN);
-  return d->split_k == 0 && d->act == LLATTN_ACT_NONE && !d->rowadd[0].ptr && !d->rowadd[1].ptr &&
-         d->c_heads.T == 0 && tiles <= 32 &&
-         std::min(d->M, d->N) <= 1024 && d->K <= 4096;
-}
-
-// K splits of a small product: its 64 x 64 tiles run their chunks one after another, ~0.7 us per 64-wide
-// chunk when a few workgroups cover the output, so a long contraction over few tiles is split while the
-// splits fit one round on the chip; the ordered reduction then costs ~3.5 us plus its fp32 traffic (E.g.
-// the 512 x 64 x 1024 query-block projection of config 4: 8 tiles of 16 chunks, 8 splits of 2.)
-int small_split(const llattn_gemm_desc* d) {
-  const int64_t tiles = (int64_t)((d->M + SBT - 1) / SBT) * ((d->N + SBT - 1) / SBT);
-  const int64_t chunks = (d->K + SBK - 1) / SBK;
-  int best = 1;
-  double best_t = (double)chunks * 0.7e-6;
-  for (int64_t S = 2; S <= std::min<int64_t>(chunks / 2, 16) && tiles * S <= 256; ++S) {
-    const double t = (double)((chunks + S - 1) / S) * 0.7e-6 + 3.5e-6 +
-                     2.0 * S * d->M * (double)(d->N + (d->a_rowsum ? 1 : 0)) * 4.0 / 5e12;
-    if (t < best_t * 0.9) {
-      best_t = t;
-      best = (int)S;
-    }
-  }
-  return best;
-}
-
 // Number of K splits: 1 when the output tiles alone fill most of the chip; otherwise the split count S
 // that minimises a time model of the product: the busiest CU runs ceil(tiles S / 256) workgroups of
 // 1/S of a tile's k range each (one 128 KB workgroup per CU), plus the fp32 partials that the ordered
@@ -1242,7 +814,8 @@ using namespace llattn::gemm;
 
 extern "C" size_t llattn_gemm_workspace_size(const llattn_gemm_desc* d) {
   if (!d) return 0;
-  const int S = use_small(d) ? small_split(d) : resolve_split(d);
+  if (tile_plan(d).mb) return 0;
+  const int S = resolve_split(d);
   return S > 1 ? (size_t)S * d->M * (d->N + (d->a_rowsum ? 1 : 0)) * sizeof(float) : 0;
 }
 
@@ -1314,7 +887,7 @@ extern "C" int32_t llattn_gemm(const llattn_gemm_desc* d, void* workspace, size_
   const size_t need = llattn_gemm_workspace_size(d);
   if (need && (!workspace || workspace_bytes < need || !aligned16(workspace)))
     return fail(LLATTN_ERR_WORKSPACE, "llattn_gemm: %d K splits need %zu workspace bytes (got %zu)",
-                use_small(d) ? small_split(d) : S, need, workspace_bytes);
+                S, need, workspace_bytes);
   GemmArgs a{};
   a.M = d->M; a.N = d->N; a.K = d->K; a.k_pairs = k_pairs; a.n_split = S;
   a.tiles_m = (d->M + BM - 1) / BM; a.tiles_n = (d->N + BN - 1) / BN;
@@ -1338,12 +911,8 @@ extern "C" int32_t llattn_gemm(const llattn_gemm_desc* d, void* workspace, size_
   a.aux = static_cast<uint16_t*>(d->aux);
   a.ld_aux = d->ld_aux;
   hipStream_t st = static_cast<hipStream_t>(stream);
-  if (use_small(d)) {
-    a.n_split = small_split(d);
-    if (!d->a_trans && !d->b_trans) launch_small<true, true>(a, d->c_dtype, st);
-    else if (!d->a_trans && d->b_trans) launch_small<true, false>(a, d->c_dtype, st);
-    else if (d->a_trans && d->b_trans) launch_small<false, false>(a, d->c_dtype, st);
-    else launch_small<false, true>(a, d->c_dtype, st);
+  if (const TilePlan tp = tile_plan(d); tp.mb) {
+    launch_tile(a, tp, !d->a_trans, !d->b_trans, d->c_dtype, st);
     return check_launch("llattn_gemm");
   }
   // bf16 x Wᵀ (+ bias) (+ row addends) without K split or accumulation: the persistent kernel, one workgroup

@@ -636,3 +636,80 @@ def test_scaled_input_grad_through_the_transpose(M, K, N):
     assert float((got.float() - ref).norm() / ref.norm()) < 2 * 2.0 ** -9
     if ((M + 255) // 256) * ((N + 255) // 256) >= 224:
         assert torch.equal(got, gemm.matmul_nn_scaled(dy, w, s))
+
+
+@pytest.mark.parametrize("M,N,K", [(8, 8, 8), (64, 64, 64), (264, 136, 72), (72, 136, 200), (1000, 520, 328),
+                                   (1000, 4104, 264), (1000, 4104, 1032), (1024, 4096, 1408), (1288, 72, 4008)])
+def test_gemm_tiles_layouts_and_epilogues(M, N, K):
+    """The smaller tiles (64 x 64 and 128 x 128, one and two k groups): every operand layout at strides of its own,
+    into bf16 and fp32, with bias, accumulation, row addends, the activations, split-head storage and row sums,
+    against float64, element by element.  fp32: 2^-20 of the sum of the terms' absolute values (an fp32 sum's typical
+    error is 2^-24 of it; the largest of millions of elements is several times that); bf16: 2^-8 of the result more,
+    twice a rounding's 2^-9."""
+    from llattn_amd import _lib as L
+    from llattn_amd import gemm
+    dev = require_cuda()
+    g = torch.Generator(device=dev).manual_seed(M + 3 * N + 7 * K)
+
+    def rnd(rows, cols, pad=8):
+        return torch.randn(rows, cols + pad, device=dev, generator=g).bfloat16()[:, :cols]
+
+    def near(got, ref, terms, roundings):
+        off = (got.double() - ref).abs()
+        return bool((off <= roundings * 2.0 ** -8 * ref.abs() + 2.0 ** -20 * terms).all())
+
+    bias = torch.randn(N, device=dev, generator=g)
+    for a_trans in (False, True):
+        for b_trans in (False, True):
+            print("case: gemm tiles", M, N, K, a_trans, b_trans, flush=True)
+            a = rnd(K, M) if a_trans else rnd(M, K)
+            b = rnd(K, N) if b_trans else rnd(N, K)
+            a64, b64 = (a.t() if a_trans else a).double(), (b if b_trans else b.t()).double()
+            ref, terms = a64 @ b64, a64.abs() @ b64.abs() + 8
+            out = torch.full((M, N), float("nan"), device=dev, dtype=torch.bfloat16)
+            gemm._run(M, N, K, a, a_trans, b, b_trans, out, bias, False)
+            assert near(out, ref + bias.double(), terms, 1)
+            plain = torch.empty_like(out)
+            gemm._run(M, N, K, a, a_trans, b, b_trans, plain, None, False)
+            start = rnd(M, N, 0)
+            acc = start.clone()
+            gemm._run(M, N, K, a, a_trans, b, b_trans, acc, None, True)
+            assert near(acc, ref + start.double(), terms, 1)
+            f = torch.full((M, N), float("nan"), device=dev)
+            rs = torch.full((M,), float("nan"), device=dev) if b_trans and (N % 256 or a_trans) else None
+            gemm._run(M, N, K, a, a_trans, b, b_trans, f, bias, False, rowsum=rs)
+            assert near(f, ref + bias.double(), terms, 0)
+            if rs is not None:
+                assert near(rs, a64.sum(1), a64.abs().sum(1) + 8, 0)
+            f2 = f.clone()
+            gemm._run(M, N, K, a, a_trans, b, b_trans, f2, None, True)
+            assert near(f2, 2 * ref + bias.double(), 2 * terms, 0)
+            if a_trans:
+                continue
+            aux = torch.empty(M, N, device=dev, dtype=torch.bfloat16)
+            gl = torch.empty_like(out)
+            gemm._run(M, N, K, a, a_trans, b, b_trans, gl, bias, False, act=L.ACT_GELU, aux=aux)
+            h = out.double()
+            phi = 0.5 * (1 + torch.erf(h / 2 ** 0.5))
+            assert near(gl, h * phi, h.abs() + 8, 1)
+            assert near(aux, phi + h * torch.exp(-h * h / 2) / (2 * torch.pi) ** 0.5, torch.full_like(h, 8), 1)
+            sc = rnd(M, N, 0)
+            gemm._run(M, N, K, a, a_trans, b, b_trans, gl, None, False, act=L.ACT_MUL_AUX, aux=sc)
+            assert torch.equal(gl, (plain.float() * sc.float()).bfloat16())
+            if b_trans:
+                seg, T = 24, M // 2
+                n = -(-T // seg)
+                rows = rnd(2 * n, N, 0)
+                add = rows.view(2, n, N).double().repeat_interleave(seg, 1)[:, :T].reshape(M, N) / seg
+                gemm._run(M, N, K, a, a_trans, b, b_trans, gl, None, False, rowadd=[(rows, T, seg, n, L.DIV_SEG)])
+                assert near(gl, ref + add, terms, 1)
+            elif M % 2 == 0:  # two sequences, heads of 8 columns over half the width, the rest in slabs of 8
+                heads = N // 16
+                st = torch.empty(M * N, device=dev, dtype=torch.bfloat16).view(M, N)
+                gemm._run(M, N, K, a, a_trans, b, b_trans, st, None, False, c_heads=(M // 2, 8, heads, 8) if heads else (M // 2, 8, 1, 0))
+                flat, cols = st.view(-1), 8 * max(heads, 1)
+                got = flat[:M * cols].view(2, -1, M // 2, 8).transpose(1, 2).reshape(M, cols)
+                assert torch.equal(got, plain[:, :cols])
+                if heads:
+                    tail = flat[M * cols:].view(2, -1, M // 2, 8).transpose(1, 2).reshape(M, N - cols)
+                    assert torch.equal(tail, plain[:, cols:])
