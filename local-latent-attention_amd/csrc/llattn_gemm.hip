@@ -38,6 +38,7 @@
 // (K a multiple of 8) masks the lanes whose 8 k values start at or past K with an out-of-range
 // offset (kmask), so no lane reads the next row's elements.
 #include "llattn_gemm.h"
+#include "llattn_pair.h"
 
 namespace llattn {
 namespace gemm {
@@ -819,7 +820,10 @@ extern "C" size_t llattn_gemm_workspace_size(const llattn_gemm_desc* d) {
   return S > 1 ? (size_t)S * d->M * (d->N + (d->a_rowsum ? 1 : 0)) * sizeof(float) : 0;
 }
 
-extern "C" int32_t llattn_gemm(const llattn_gemm_desc* d, void* workspace, size_t workspace_bytes, void* stream) {
+namespace {
+
+// Checks a product and fills its launch arguments; `paired`: no workspace is used.
+int32_t prepare(const llattn_gemm_desc* d, void* workspace, size_t workspace_bytes, bool paired, GemmArgs& a) {
   if (!d) return fail(LLATTN_ERR_SHAPE, "llattn_gemm: null descriptor");
   if (d->M <= 0 || d->N <= 0 || d->K <= 0)
     return fail(LLATTN_ERR_SHAPE, "llattn_gemm: sizes must be positive (M=%d N=%d K=%d)", d->M, d->N, d->K);
@@ -878,17 +882,17 @@ extern "C" int32_t llattn_gemm(const llattn_gemm_desc* d, void* workspace, size_
     if (((int64_t)(d->M - 1) * d->ld_aux + d->N) * 2 >= (int64_t(1) << 31))
       return fail(LLATTN_ERR_UNSUPPORTED, "llattn_gemm: the activation's aux matrix must be below 2 GiB");
   }
-  HeadsMap ch;
+  HeadsMap ch{};
   if (const int32_t rc = heads_map("llattn_gemm (C)", &d->c_heads, d->M, d->ldc, d->N, &ch)) return rc;
   if (ch.T && (d->a_trans || d->b_trans || d->c_dtype != LLATTN_BF16 || d->accumulate || d->act != LLATTN_ACT_NONE ||
                d->rowadd[0].ptr || d->rowadd[1].ptr || S != 1))
     return fail(LLATTN_ERR_UNSUPPORTED, "llattn_gemm: a split-head C needs a_trans = b_trans = 0, bf16 C, no "
                 "accumulation, activation, row addends or K split");
-  const size_t need = llattn_gemm_workspace_size(d);
+  const size_t need = paired ? 0 : llattn_gemm_workspace_size(d);
   if (need && (!workspace || workspace_bytes < need || !aligned16(workspace)))
     return fail(LLATTN_ERR_WORKSPACE, "llattn_gemm: %d K splits need %zu workspace bytes (got %zu)",
                 S, need, workspace_bytes);
-  GemmArgs a{};
+  a = GemmArgs{};
   a.M = d->M; a.N = d->N; a.K = d->K; a.k_pairs = k_pairs; a.n_split = S;
   a.tiles_m = (d->M + BM - 1) / BM; a.tiles_n = (d->N + BN - 1) / BN;
   a.accumulate = d->accumulate;
@@ -910,6 +914,41 @@ extern "C" int32_t llattn_gemm(const llattn_gemm_desc* d, void* workspace, size_
   a.act = d->act;
   a.aux = static_cast<uint16_t*>(d->aux);
   a.ld_aux = d->ld_aux;
+  return LLATTN_OK;
+}
+
+}  // namespace
+
+namespace llattn {
+namespace gemm {
+
+size_t pair_workspace(const llattn_gemm_desc* d0, const llattn_gemm_desc* d1) {
+  if (pair_plan(d0, d1)) return 0;
+  return std::max(llattn_gemm_workspace_size(d0), llattn_gemm_workspace_size(d1));
+}
+
+int32_t run_pair(const llattn_gemm_desc* d0, const llattn_gemm_desc* d1, void* workspace, size_t workspace_bytes,
+                 void* stream) {
+  const int mb = pair_plan(d0, d1);
+  if (!mb) {
+    if (const int32_t rc = llattn_gemm(d0, workspace, workspace_bytes, stream)) return rc;
+    return llattn_gemm(d1, workspace, workspace_bytes, stream);
+  }
+  GemmArgs a0, a1;
+  if (const int32_t rc = prepare(d0, nullptr, 0, true, a0)) return rc;
+  if (const int32_t rc = prepare(d1, nullptr, 0, true, a1)) return rc;
+  launch_pair(a0, a1, mb, !d0->b_trans, d1->a_trans, static_cast<hipStream_t>(stream));
+  return check_launch("llattn_gemm");
+}
+
+}  // namespace gemm
+}  // namespace llattn
+
+extern "C" int32_t llattn_gemm(const llattn_gemm_desc* d, void* workspace, size_t workspace_bytes, void* stream) {
+  GemmArgs a;
+  if (const int32_t rc = prepare(d, workspace, workspace_bytes, false, a)) return rc;
+  const int S = a.n_split, k_pairs = a.k_pairs;
+  const HeadsMap ch = a.ch;
   hipStream_t st = static_cast<hipStream_t>(stream);
   if (const TilePlan tp = tile_plan(d); tp.mb) {
     launch_tile(a, tp, !d->a_trans, !d->b_trans, d->c_dtype, st);

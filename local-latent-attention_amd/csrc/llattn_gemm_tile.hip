@@ -112,19 +112,21 @@ __device__ __forceinline__ void finish4(const GemmArgs& a, int row, int col, f32
   }
 }
 
+constexpr int stage_bytes(int mb, int nb) { return 32 * (mb + nb) * 128; }
+
+// Workgroup `block` of `blocks` of a product; smem: KG NST stages, rsl: [KG][32 MB].
 template <bool AK, bool BKM, int EPI, int MB, int NB, int KG, int NST>
-__global__ __launch_bounds__(256 * KG) void gemm_tile_kernel(const GemmArgs a) {
+__device__ __forceinline__ void tile_product(const GemmArgs& a, int block, int blocks, unsigned char* smem, float* rsl) {
   constexpr int TM = 32 * MB, TN = 32 * NB;
   typedef TileOp<AK, false, TM> OpA;
   typedef TileOp<BKM, false, TN> OpB;
-  constexpr int STAGE = OpA::BYTES + OpB::BYTES, LOADS = OpA::NB + OpB::NB;  // loads of a wave per step
-  __shared__ __align__(1024) unsigned char smem[KG * NST * STAGE];
-  __shared__ float rsl[KG][TM];
+  constexpr int STAGE = stage_bytes(MB, NB), LOADS = OpA::NB + OpB::NB;  // loads of a wave per step
+  static_assert(STAGE == OpA::BYTES + OpB::BYTES, "a stage holds both tiles");
   const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), w4 = wave & 3, kg = wave >> 2;
   const int wm = w4 >> 1, wn = w4 & 1;
   // contiguous tile ranges per XCD, then groups of 8 tile rows
-  const int t = xcd_remap(blockIdx.x, gridDim.x);
+  const int t = xcd_remap(block, blocks);
   constexpr int GM = 8;
   const int group = t / (GM * a.tiles_n), first_m = group * GM, gm = min(a.tiles_m - first_m, GM);
   const int m0 = (first_m + (t % (GM * a.tiles_n)) % gm) * TM, n0 = (t % (GM * a.tiles_n)) / gm * TN;
@@ -199,7 +201,7 @@ __global__ __launch_bounds__(256 * KG) void gemm_tile_kernel(const GemmArgs a) {
       float v = rsum[i];
       v += __shfl_xor(v, 16);
       v += __shfl_xor(v, 32);
-      if (g == 0) rsl[kg][wm * 16 * MB + 16 * i + r] = v;
+      if (g == 0) rsl[kg * TM + wm * 16 * MB + 16 * i + r] = v;
     }
   }
   __syncthreads();
@@ -226,10 +228,32 @@ __global__ __launch_bounds__(256 * KG) void gemm_tile_kernel(const GemmArgs a) {
     }
   }
   if (a.rowsum && n0 == 0 && threadIdx.x < TM && m0 + (int)threadIdx.x < a.M) {
-    float v = rsl[0][threadIdx.x];
+    float v = rsl[threadIdx.x];
 #pragma unroll
-    for (int w = 1; w < KG; ++w) v += rsl[w][threadIdx.x];
+    for (int w = 1; w < KG; ++w) v += rsl[w * TM + threadIdx.x];
     a.rowsum[m0 + threadIdx.x] = v;
+  }
+}
+
+template <bool AK, bool BKM, int EPI, int MB, int NB, int KG, int NST>
+__global__ __launch_bounds__(256 * KG) void gemm_tile_kernel(const GemmArgs a) {
+  __shared__ __align__(1024) unsigned char smem[KG * NST * stage_bytes(MB, NB)];
+  __shared__ float rsl[KG * 32 * MB];
+  tile_product<AK, BKM, EPI, MB, NB, KG, NST>(a, blockIdx.x, gridDim.x, smem, rsl);
+}
+
+// Two independent products in one launch: the first n0 workgroups (a multiple of 8, so that both see their XCD) take
+// the first one.  An input and a weight gradient of the same dy, or two projections, each fill the chip badly at a
+// few thousand rows; together they share its last round and one launch.
+template <bool AK0, bool BK0, int EPI0, bool AK1, bool BK1, int EPI1, int MB>
+__global__ __launch_bounds__(256) void gemm_tile_pair_kernel(const GemmArgs a0, const GemmArgs a1, int n0) {
+  __shared__ __align__(1024) unsigned char smem[2 * stage_bytes(MB, MB)];
+  __shared__ float rsl[32 * MB];
+  const int b = blockIdx.x, c0 = a0.tiles_m * a0.tiles_n, c1 = a1.tiles_m * a1.tiles_n;
+  if (b < n0) {
+    if (b < c0) tile_product<AK0, BK0, EPI0, MB, MB, 1, 2>(a0, b, c0, smem, rsl);
+  } else if (b - n0 < c1) {
+    tile_product<AK1, BK1, EPI1, MB, MB, 1, 2>(a1, b - n0, c1, smem, rsl);
   }
 }
 
@@ -273,7 +297,7 @@ static double big_us(int64_t M, int64_t N, int steps, int S) {
 // Measured against the 256 x 256 kernels and the register-staged 64 x 64 tiles that this replaced:
 //   333 x 4736 x 1408: 30 -> 12.5 us;  1024 x 4096 x 1408: 30 -> 17;  1536 x 384 x 4011 (dyT x): 52 -> 18;
 //   4011 x 384 x 1536 (dy W): 25 -> 13;  32768 x 64 x 1024: 24 -> 13;  1024 x 1408 x 1408: 15 -> 12.
-TilePlan tile_plan(const llattn_gemm_desc* d) {
+TilePlan tile_plan(const llattn_gemm_desc* d, double* us) {
   const TilePlan none{0, 0, 0};
   if (d->split_k > 0 || d->M <= 0 || d->N <= 0 || d->K <= 0) return none;
   const int64_t M = d->M, N = d->N;
@@ -296,6 +320,7 @@ TilePlan tile_plan(const llattn_gemm_desc* d) {
   const double lengthy = 1.0 + 0.2 * std::min(1.0, steps / 48.0), last[] = {0.0, 0.35 * lengthy, 0.44 * lengthy, 0.6, 0.82};
   take(3.0 + steps * ((double)(t64 / 1024) * 0.85 + last[r64]), 2, 1);
   if (steps >= 4) take(0.6 + rounds(t64) * (2.4 + split(2) * 0.45), 2, 2);
+  if (us) *us = best_t;
   return best;
 }
 
@@ -307,6 +332,69 @@ void launch_tile(const GemmArgs& a0, const TilePlan& p, bool a_kmaj, bool b_kmaj
   else if (a_kmaj) launch_dt<true, false>(a, p, c_dtype, st);
   else if (!b_kmaj) launch_dt<false, false>(a, p, c_dtype, st);
   else launch_dt<false, true>(a, p, c_dtype, st);
+}
+
+namespace {
+
+// Time in us of a product by itself, as tile_plan and resolve_split leave it.
+double alone_us(const llattn_gemm_desc* d) {
+  double t = 0.0;
+  const TilePlan p = tile_plan(d, &t);
+  const int64_t tiles = ((d->M + BM - 1) / BM) * (int64_t)((d->N + BN - 1) / BN);
+  if (!p.mb) t = tiles >= 224 ? big_us(d->M, d->N, (d->K + SK - 1) / SK, 1) : big_us(d->M, d->N, (d->K + SK - 1) / SK, resolve_split(d));
+  return t;
+}
+
+template <int MB>
+void launch_pair_mb(const GemmArgs& a0, const GemmArgs& a1, bool nt0, bool nt1, int n0, dim3 grid, hipStream_t st) {
+  const dim3 block(256);
+  if (nt1) hipLaunchKernelGGL((gemm_tile_pair_kernel<true, true, EPI_BF16, true, true, EPI_BF16, MB>), grid, block, 0, st, a0, a1, n0);
+  else if (nt0) hipLaunchKernelGGL((gemm_tile_pair_kernel<true, true, EPI_BF16, false, false, EPI_F32, MB>), grid, block, 0, st, a0, a1, n0);
+  else hipLaunchKernelGGL((gemm_tile_pair_kernel<true, false, EPI_BF16, false, false, EPI_F32, MB>), grid, block, 0, st, a0, a1, n0);
+}
+
+}  // namespace
+
+// Tile of two products in one launch (32 mb squared, one k group), or 0 where they are better run one by one: the
+// work of all tiles at a full chip's rate per (tile, step), or the longest tile at the rate of the tiles that share
+// its CU, and a third of a shorter one for the ragged end; taken where that saves 5%.  (q|k|v and the latents' keys and
+// values of a 0.55b layer over 333 tokens: 18 us in one launch, 17 + 8 in two; the latent projections' two gradients of
+// 4 x 8192 tokens with 64-token query blocks 11.5 us, 5 + 10.  The gradients of a few thousand tokens' large projections stay apart: the weight
+// gradient's long contraction wants its own k split.)
+int pair_plan(const llattn_gemm_desc* d0, const llattn_gemm_desc* d1) {
+  for (const llattn_gemm_desc* d : {d0, d1})
+    if (d->split_k > 0 || d->M <= 0 || d->N <= 0 || d->K <= 0) return 0;
+  const bool bf0 = d0->c_dtype == LLATTN_BF16 && !d0->a_trans, nt1 = d1->c_dtype == LLATTN_BF16 && !d1->a_trans && !d1->b_trans;
+  const bool tn1 = d1->c_dtype == LLATTN_F32 && d1->a_trans && d1->b_trans;
+  if (!bf0 || !(tn1 || (nt1 && !d0->b_trans))) return 0;
+  const double s0 = (d0->K + SK - 1) / SK, s1 = (d1->K + SK - 1) / SK;
+  double best_t = 0.95 * (alone_us(d0) + alone_us(d1));
+  int best = 0;
+  for (int mb : {4, 2}) {
+    const int64_t T = 32 * mb;
+    const double t0 = (double)(((d0->M + T - 1) / T) * ((d0->N + T - 1) / T)), t1 = (double)(((d1->M + T - 1) / T) * ((d1->N + T - 1) / T));
+    const double n = t0 + t1, most = std::max(s0, s1), least = std::min(s0, s1);
+    double t;
+    if (mb == 4) t = 4.0 + std::max((t0 * s0 + t1 * s1) * 1.27 / 512.0, (n <= 256 ? 0.75 : 1.1) * most) + 0.3 * least;
+    else t = 3.0 + std::max((t0 * s0 + t1 * s1) * 0.85 / 1024.0, (n <= 256 ? 0.38 : n <= 512 ? 0.5 : n <= 768 ? 0.6 : 0.82) * most) + 0.15 * least;
+    if (t < best_t) {
+      best_t = t;
+      best = mb;
+    }
+  }
+  return best;
+}
+
+void launch_pair(GemmArgs a0, GemmArgs a1, int mb, bool b_kmaj0, bool weight1, hipStream_t st) {
+  const int T = 32 * mb;
+  for (GemmArgs* a : {&a0, &a1}) {
+    a->tiles_m = (a->M + T - 1) / T;
+    a->tiles_n = (a->N + T - 1) / T;
+  }
+  const int n0 = (a0.tiles_m * a0.tiles_n + 7) / 8 * 8;
+  const dim3 grid(n0 + a1.tiles_m * a1.tiles_n);
+  if (mb == 4) launch_pair_mb<4>(a0, a1, b_kmaj0, !weight1, n0, grid, st);
+  else launch_pair_mb<2>(a0, a1, b_kmaj0, !weight1, n0, grid, st);
 }
 
 }  // namespace gemm

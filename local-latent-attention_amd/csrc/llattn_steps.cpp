@@ -7,13 +7,16 @@
 // inputs, which autograd then need not copy), the 0.55b model over 1024 tokens 9.4 -> 4.9 ms.
 //
 // The sequences are those of the Python path (module.py, ops.py, linear.py, ffn.py: kept for profiling and for
-// parameters this path does not take), product by product with the same routes, so both give the same bits.
+// parameters this path does not take), product by product with the same operands and roundings.  Two products that do
+// not depend on each other share a launch where that pays (llattn_pair.h); the k order of their sums can then differ
+// from the single products', otherwise both paths give the same bits.
 //
 // Every step is one function run twice: by the size query with a null base, where buffers only count and launches
 // only ask for their workspace, and by the call itself.
 #include <algorithm>
 
 #include "llattn_abi.h"
+#include "llattn_pair.h"
 #include "llattn_steps.h"
 
 namespace llattn {
@@ -55,8 +58,19 @@ struct Exec {
     need = std::max(need, n);
     run([&] { return llattn_gemm(&d, n ? gemm_ws : nullptr, n ? gemm_bytes : 0, stream); });
   }
+  // two products that do not depend on each other
+  void gemm(const llattn_gemm_desc& d0, const llattn_gemm_desc& d1, bool f32) {
+    if (f32) {
+      gemm(d0, true);
+      gemm(d1, true);
+      return;
+    }
+    const size_t n = llattn::gemm::pair_workspace(&d0, &d1);
+    need = std::max(need, n);
+    run([&] { return llattn::gemm::run_pair(&d0, &d1, n ? gemm_ws : nullptr, n ? gemm_bytes : 0, stream); });
+  }
   // y [M][N] = x [M][K] w [N][K]ᵀ (+ b)
-  void linear(int dt, int M, int N, int K, const void* x, const void* w, const float* b, void* y,
+  static llattn_gemm_desc linear(int dt, int M, int N, int K, const void* x, const void* w, const float* b, void* y,
               const llattn_heads_layout* heads = nullptr, int act = LLATTN_ACT_NONE, void* aux = nullptr) {
     llattn_gemm_desc d{};
     d.M = M; d.N = N; d.K = K;
@@ -66,10 +80,10 @@ struct Exec {
     d.bias = b;
     if (heads) d.c_heads = *heads;
     d.act = act; d.aux = aux; d.ld_aux = aux ? N : 0;
-    gemm(d, dt == LLATTN_F32);
+    return d;
   }
   // dx [M][K] = dy [M][N] w [N][K] (+ row addends; * aux): through w_t where the persistent kernel takes it
-  void input_grad(int dt, int M, int N, int K, const void* dy, const void* w, const void* w_t, void* dx,
+  static llattn_gemm_desc input_grad(int dt, int M, int N, int K, const void* dy, const void* w, const void* w_t, void* dx,
                   const llattn_heads_layout* heads = nullptr, const llattn_gemm_rowadd* ra = nullptr, int n_ra = 0,
                   void* aux = nullptr) {
     llattn_gemm_desc d{};
@@ -89,10 +103,10 @@ struct Exec {
       d.aux = aux;
       d.ld_aux = K;
     }
-    gemm(d, dt == LLATTN_F32);
+    return d;
   }
   // dw [N][D] = dy [M][N]ᵀ x [M][D] in fp32, db [N] = the column sums of dy
-  void weight_grad(int dt, int M, int N, int D, const void* dy, const void* x, float* dw, float* db) {
+  static llattn_gemm_desc weight_grad(int dt, int M, int N, int D, const void* dy, const void* x, float* dw, float* db) {
     llattn_gemm_desc d{};
     d.M = N; d.N = D; d.K = M;
     d.a_trans = d.b_trans = 1;
@@ -100,7 +114,7 @@ struct Exec {
     d.B = x; d.ldb = D;
     d.C = dw; d.ldc = D; d.c_dtype = LLATTN_F32;
     d.a_rowsum = db;
-    gemm(d, dt == LLATTN_F32);
+    return d;
   }
   void pool(int dt, const void* x, void* out, int B, int T, int D, int seg, int n, int div) {
     run([&] {
@@ -186,7 +200,8 @@ void core_fwd(Exec& e, const llattn_block_cfg& c, const llattn_core_views& in, c
   const llattn_tensor lat = view(k.lat, 0, d.es, d.nq * d.Ld, d.Ld, d.Ldh);
   e.run([&] { return llattn_latent_fwd(&c.shape, &in.gq, &in.gk, &in.gv, &lat, k.lse_lat, e.stream); });
   const llattn_heads_layout rh{d.nq, d.Dh, d.H, 0};
-  e.linear(d.dt, (int)d.Mq, (int)d.D, (int)d.Ld, k.lat, r_w, r_b, k.R, c.remote_heads ? &rh : nullptr);
+  e.gemm(e.linear(d.dt, (int)d.Mq, (int)d.D, (int)d.Ld, k.lat, r_w, r_b, k.R, c.remote_heads ? &rh : nullptr),
+         d.dt == LLATTN_F32);
   const llattn_tensor R = remote_view(c, d, k.R);
   // o_local is the op's own: head-major, a head's rows one contiguous run
   const llattn_tensor ol = view(k.ol, 0, d.es, (int64_t)d.H * d.T * d.Dh, d.Dh, (int64_t)d.T * d.Dh);
@@ -216,8 +231,8 @@ void core_bwd(Exec& e, Arena& a, const llattn_block_cfg& c, const llattn_core_vi
   }
   void* dlat = a.take(d.Mq * d.Ld * d.es);
   const llattn_heads_layout lh{d.nq, d.Ldh, d.Lh, 0};
-  e.input_grad(d.dt, (int)d.Mq, (int)d.D, (int)d.Ld, dR, r_w, k.r_wt, dlat, c.lat_heads ? &lh : nullptr);
-  e.weight_grad(d.dt, (int)d.Mq, (int)d.D, (int)d.Ld, dR, k.lat, dr_w, nullptr);
+  e.gemm(e.input_grad(d.dt, (int)d.Mq, (int)d.D, (int)d.Ld, dR, r_w, k.r_wt, dlat, c.lat_heads ? &lh : nullptr),
+         e.weight_grad(d.dt, (int)d.Mq, (int)d.D, (int)d.Ld, dR, k.lat, dr_w, nullptr), d.dt == LLATTN_F32);
   const llattn_tensor dl = c.lat_heads ? view(dlat, 0, d.es, d.Ld * d.nq, d.Ldh, (int64_t)d.nq * d.Ldh)
                                        : view(dlat, 0, d.es, d.nq * d.Ld, d.Ld, d.Ldh);
   const size_t n_lat = llattn_workspace_size(&c.shape, LLATTN_WS_LATENT_BWD);
@@ -322,17 +337,18 @@ void block_fwd(Exec& e, const llattn_block_cfg& c, const llattn_block_params& p,
   casts.launch(e);
   const Weights w = block_weights(c, p, k);
   const llattn_heads_layout hl{d.T, d.Dh, 3 * d.H, c.macro ? 0 : d.Ldh};
-  e.linear(dt, (int)d.M, (int)width, (int)Dm, x, w.qkv, w.b_qkv, k.qkvr, c.heads ? &hl : nullptr);
+  const bool f32 = dt == LLATTN_F32;
   if (c.macro) {
     if (!twin_pools(c)) e.pool(dt, x, k.pq, d.B, d.T, (int)Dm, s.q_block, d.nq, LLATTN_DIV_SEG);
     else e.pool(dt, x, k.pooled, d.B, d.T, (int)Dm, s.chunk, d.nc, LLATTN_DIV_SEG);
-    e.linear(dt, (int)d.Mq, (int)d.Ld, (int)Dm, k.pq, w.rq, p.b_rq, k.rq);
   }
   if (!twin_pools(c)) e.pool(dt, x, k.pooled, d.B, d.T, (int)Dm, s.chunk, d.nc, LLATTN_DIV_COUNT);
-  e.linear(dt, d.B * d.nc, (int)(2 * d.Ld), (int)Dm, k.pooled, w.rkv, p.b_rkv, k.gkgv);
+  e.gemm(e.linear(dt, (int)d.M, (int)width, (int)Dm, x, w.qkv, w.b_qkv, k.qkvr, c.heads ? &hl : nullptr),
+         e.linear(dt, d.B * d.nc, (int)(2 * d.Ld), (int)Dm, k.pooled, w.rkv, p.b_rkv, k.gkgv), f32);
+  if (c.macro) e.gemm(e.linear(dt, (int)d.Mq, (int)d.Ld, (int)Dm, k.pq, w.rq, p.b_rq, k.rq), f32);
   const llattn_tensor y = view(k.y, 0, d.es, d.T * d.D, d.D, d.Dh);
   core_fwd(e, c, block_views(c, k.qkvr, c.heads, k.rq, k.gkgv), p.gate_l, p.gate_r, w.r, p.b_r, k.core, y);
-  e.linear(dt, (int)d.M, (int)Dm, (int)d.D, k.y, w.out, p.b_out, out);
+  e.gemm(e.linear(dt, (int)d.M, (int)Dm, (int)d.D, k.y, w.out, p.b_out, out), f32);
 }
 
 void block_bwd(Exec& e, Arena& a, const llattn_block_cfg& c, const llattn_block_params& p, const void* x,
@@ -345,8 +361,8 @@ void block_bwd(Exec& e, Arena& a, const llattn_block_cfg& c, const llattn_block_
   const Weights w = block_weights(c, p, k);
   void* dyc = a.take(d.M * d.D * d.es);
   const llattn_heads_layout yh{d.T, d.Dh, d.H, 0};
-  e.input_grad(dt, (int)d.M, (int)Dm, (int)d.D, dy, w.out, k.w_outt, dyc, c.dy_heads ? &yh : nullptr);
-  e.weight_grad(dt, (int)d.M, (int)Dm, (int)d.D, dy, k.y, g.w_out, g.b_out);
+  e.gemm(e.input_grad(dt, (int)d.M, (int)Dm, (int)d.D, dy, w.out, k.w_outt, dyc, c.dy_heads ? &yh : nullptr),
+         e.weight_grad(dt, (int)d.M, (int)Dm, (int)d.D, dy, k.y, g.w_out, g.b_out), !bf);
   void* dqkv = a.take(d.M * width * d.es);
   void* drq = c.macro ? a.take(d.Mq * d.Ld * d.es) : nullptr;
   void* dgkgv = a.take((int64_t)d.B * d.nc * 2 * d.Ld * d.es);
@@ -358,29 +374,31 @@ void block_bwd(Exec& e, Arena& a, const llattn_block_cfg& c, const llattn_block_
            g.gate_r, g.w_r, g.b_r);
   const int Mc = d.B * d.nc;
   void* dpooled = dx ? a.take((int64_t)Mc * Dm * d.es) : nullptr;
-  if (dx) e.input_grad(dt, Mc, (int)(2 * d.Ld), (int)Dm, dgkgv, w.rkv, nullptr, dpooled);
-  e.weight_grad(dt, Mc, (int)(2 * d.Ld), (int)Dm, dgkgv, k.pooled, g.w_rkv, g.b_rkv);
+  // an input gradient (where it is wanted) with the weight gradient of the same dy
+  auto grads = [&](const llattn_gemm_desc& di, const llattn_gemm_desc& dw) {
+    if (dx) e.gemm(di, dw, !bf);
+    if (!dx || e.dry) e.gemm(dw, !bf);  // the scratch is sized for both
+  };
+  grads(e.input_grad(dt, Mc, (int)(2 * d.Ld), (int)Dm, dgkgv, w.rkv, nullptr, dpooled),
+        e.weight_grad(dt, Mc, (int)(2 * d.Ld), (int)Dm, dgkgv, k.pooled, g.w_rkv, g.b_rkv));
   void* dpq = dx && c.macro ? a.take(d.Mq * Dm * d.es) : nullptr;
-  if (c.macro) {
-    if (dx) e.input_grad(dt, (int)d.Mq, (int)d.Ld, (int)Dm, drq, w.rq, nullptr, dpq);
-    e.weight_grad(dt, (int)d.Mq, (int)d.Ld, (int)Dm, drq, k.pq, g.w_rq, g.b_rq);
-  }
-  if (dx) {
-    // the poolings' gradients: in bf16 added in the product's epilogue, query blocks first
-    llattn_gemm_rowadd ra[2];
-    int n = 0;
-    static char there;  // a dry run's addends count as present
-    if (e.dry) dpq = dpooled = &there;
-    if (c.macro) ra[n++] = llattn_gemm_rowadd{dpq, Dm, d.T, s.q_block, d.nq, LLATTN_DIV_SEG};
-    ra[n++] = llattn_gemm_rowadd{dpooled, Dm, d.T, s.chunk, d.nc, LLATTN_DIV_COUNT};
-    e.input_grad(dt, (int)d.M, (int)width, (int)Dm, dqkv, w.qkv, k.w_qkvt, dx, nullptr, ra, bf ? n : 0);
-    for (int q = 0; q < n && !bf; ++q)
-      e.run([&] {
-        return llattn_pool_bwd(ra[q].ptr, (int64_t)ra[q].n_seg * Dm, Dm, dx, d.T * Dm, Dm, d.B, d.T, (int)Dm, ra[q].seg,
-                               ra[q].n_seg, ra[q].divisor, 1, dt, e.stream);
-      });
-  }
-  e.weight_grad(dt, (int)d.M, (int)width, (int)Dm, dqkv, x, g.w_qkv, g.b_qkv);
+  if (c.macro)
+    grads(e.input_grad(dt, (int)d.Mq, (int)d.Ld, (int)Dm, drq, w.rq, nullptr, dpq),
+          e.weight_grad(dt, (int)d.Mq, (int)d.Ld, (int)Dm, drq, k.pq, g.w_rq, g.b_rq));
+  // the poolings' gradients join the input gradient: in bf16 in the product's epilogue, query blocks first
+  static char there;  // a dry run's addends count as present
+  if (e.dry) dpq = dpooled = &there;
+  llattn_gemm_rowadd ra[2];
+  int n = 0;
+  if (c.macro) ra[n++] = llattn_gemm_rowadd{dpq, Dm, d.T, s.q_block, d.nq, LLATTN_DIV_SEG};
+  ra[n++] = llattn_gemm_rowadd{dpooled, Dm, d.T, s.chunk, d.nc, LLATTN_DIV_COUNT};
+  grads(e.input_grad(dt, (int)d.M, (int)width, (int)Dm, dqkv, w.qkv, k.w_qkvt, dx, nullptr, ra, bf ? n : 0),
+        e.weight_grad(dt, (int)d.M, (int)width, (int)Dm, dqkv, x, g.w_qkv, g.b_qkv));
+  for (int q = 0; q < n && !bf && dx; ++q)
+    e.run([&] {
+      return llattn_pool_bwd(ra[q].ptr, (int64_t)ra[q].n_seg * Dm, Dm, dx, d.T * Dm, Dm, d.B, d.T, (int)Dm, ra[q].seg,
+                             ra[q].n_seg, ra[q].divisor, 1, dt, e.stream);
+    });
 }
 
 int32_t check_cfg(const char* what, const llattn_block_cfg* c, bool block) {
@@ -478,17 +496,18 @@ void ffn_fwd(Exec& e, const llattn_ffn_cfg& c, const void* x, const float* w1, c
   casts.add(w2, k.w2, c.d_out, c.d_ff, LLATTN_BF16, k.w2t, c.d_out);
   casts.launch(e);
   static char there;
-  e.linear(LLATTN_BF16, c.rows, c.d_ff, c.d, x, k.w1, b1, k.g, nullptr, LLATTN_ACT_GELU, e.dry ? &there : k.gp);
-  e.linear(LLATTN_BF16, c.rows, c.d_out, c.d_ff, k.g, k.w2, b2, y);
+  e.gemm(e.linear(LLATTN_BF16, c.rows, c.d_ff, c.d, x, k.w1, b1, k.g, nullptr, LLATTN_ACT_GELU, e.dry ? &there : k.gp), false);
+  e.gemm(e.linear(LLATTN_BF16, c.rows, c.d_out, c.d_ff, k.g, k.w2, b2, y), false);
 }
 void ffn_bwd(Exec& e, Arena& a, const llattn_ffn_cfg& c, const void* x, const Ffn& k, const void* dy, void* dx,
              float* dw1, float* db1, float* dw2, float* db2) {
   void* dh = a.take((int64_t)c.rows * c.d_ff * 2);
   static char there;
-  e.input_grad(LLATTN_BF16, c.rows, c.d_out, c.d_ff, dy, k.w2, k.w2t, dh, nullptr, nullptr, 0, e.dry ? &there : k.gp);
-  e.weight_grad(LLATTN_BF16, c.rows, c.d_out, c.d_ff, dy, k.g, dw2, db2);
-  if (dx) e.input_grad(LLATTN_BF16, c.rows, c.d_ff, c.d, dh, k.w1, k.w1t, dx);
-  e.weight_grad(LLATTN_BF16, c.rows, c.d_ff, c.d, dh, x, dw1, db1);
+  e.gemm(e.input_grad(LLATTN_BF16, c.rows, c.d_out, c.d_ff, dy, k.w2, k.w2t, dh, nullptr, nullptr, 0, e.dry ? &there : k.gp),
+         e.weight_grad(LLATTN_BF16, c.rows, c.d_out, c.d_ff, dy, k.g, dw2, db2), false);
+  const llattn_gemm_desc dw = e.weight_grad(LLATTN_BF16, c.rows, c.d_ff, c.d, dh, x, dw1, db1);
+  if (dx) e.gemm(e.input_grad(LLATTN_BF16, c.rows, c.d_ff, c.d, dh, k.w1, k.w1t, dx), dw, false);
+  if (!dx || e.dry) e.gemm(dw, false);
 }
 Need ffn_need(const llattn_ffn_cfg& c, bool bwd) {
   return measure([&](Exec& e, Arena& a) {

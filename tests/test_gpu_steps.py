@@ -1,5 +1,6 @@
 """The native steps (one call per direction) against the Python path that issues the same products one by one: the
-same bits for every output and gradient.  The Python path runs while calls are logged."""
+same bits for every output and gradient, or the same values up to the order of a product's sums where two products
+share a launch.  The Python path runs while calls are logged."""
 from __future__ import annotations
 
 import contextlib
@@ -36,6 +37,19 @@ def _both(fn, entry):
         python = fn()
     assert log
     return native, python
+
+
+def _close(native, python, bf16):
+    """Equal up to the order in which a product's fp32 sums are formed.  In fp32 that is 2^-21 of an output's norm; in
+    bf16 a sum on a rounding boundary moves an element by one unit, 2^-8 of it at most, here and there, and what is
+    computed from it by as much: 2^-9 of the norm."""
+    assert len(native) == len(python)
+    for i, (a, b) in enumerate(zip(native, python)):
+        assert (a is None) == (b is None), i
+        if a is not None:
+            assert a.dtype == b.dtype and a.shape == b.shape, i
+            off, norm = float((a.double() - b.double()).norm()), float(b.double().norm())
+            assert off <= (2.0 ** -9 if bf16 else 2.0 ** -21) * norm, (i, off, norm)
 
 
 def _same(native, python):
@@ -85,20 +99,18 @@ def test_block_step_matches_python_path(cfg, bf16, bias):
         y.backward(dy)
         return [y.detach(), xx.grad, *(p.grad for p in m.parameters())]
 
+    # fp32: the Python path forms the poolings' input gradients apart and adds them; here they are added in place
     native, python = _both(train, "llattn_block_bwd")
-    if bf16:
-        _same(native, python)
-    else:  # the Python path forms the poolings' input gradients apart and adds them; here they are added in place
-        _same(native[:1] + native[2:], python[:1] + python[2:])
-        assert float((native[1] - python[1]).norm()) <= 2.0 ** -22 * float(python[1].norm())
-    _same(*_both(lambda: train(False), "llattn_block_bwd"))
+    _close(native, python, bf16)
+    _close(*_both(lambda: train(False), "llattn_block_bwd"), bf16)
+    _same(train(), native)
 
     def infer():
         with torch.no_grad(), cast():
             return [m(x)]
 
     a, b = _both(infer, "llattn_block_fwd")
-    _same(a, b)
+    _close(a, b, bf16)
     assert torch.equal(a[0], native[0])
 
 
@@ -154,12 +166,12 @@ def test_block_step_leaves_other_inputs_to_the_python_path():
             ref = m(x[..., :128].contiguous())
             assert called
             del called[:]
-            assert torch.equal(m(x[..., :128]), ref)
+            _close([m(x[..., :128])], [ref], True)
             wide = m(x[..., :128].float().contiguous())  # pooled in float32 before the rounding
             assert float((wide - ref).float().norm() / ref.float().norm()) < 0.02
             odd = torch.empty(m.out.weight.numel() + 1, device=dev)[1:].view_as(m.out.weight).copy_(m.out.weight)
             m.out.weight = torch.nn.Parameter(odd)
-            assert torch.equal(m(x[..., :128].contiguous()), ref)
+            _close([m(x[..., :128].contiguous())], [ref], True)
         assert not called
     finally:
         steps._call = real
@@ -195,7 +207,7 @@ def test_op_step_matches_python_path(contiguous, dtype, qb, T, per_head):
             assert t.grad.stride() == t.stride()
         return [y.detach(), *(t.grad for t in leaves), b.grad]
 
-    _same(*_both(run, "llattn_core_bwd"))
+    _close(*_both(run, "llattn_core_bwd"), dtype == torch.bfloat16)
 
 
 @pytest.mark.parametrize("shape,d_ff,bias", [((3, 7, 64), 128, True), ((2, 600, 128), 256, False),
@@ -219,5 +231,5 @@ def test_ffn_step_matches_python_path(shape, d_ff, bias):
         y.backward(dy)
         return [y.detach(), xx.grad, *(p.grad for p in (*w1.parameters(), *w2.parameters()))]
 
-    _same(*_both(run, "llattn_ffn_bwd"))
-    _same(*_both(lambda: run(False), "llattn_ffn_fwd"))
+    _close(*_both(run, "llattn_ffn_bwd"), True)
+    _close(*_both(lambda: run(False), "llattn_ffn_fwd"), True)
