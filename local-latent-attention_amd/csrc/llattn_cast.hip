@@ -10,8 +10,7 @@
 // (fp32 rows), written as bf16 rows, and written again transposed through LDS, so W^T costs 2 bytes per
 // element on top of the cast instead of a separate read and write of W.
 // Conversion rounds to nearest even, as a torch .to(torch.bfloat16) does.
-#include "llattn_abi.h"
-#include "llattn_device.h"
+#include "llattn_pool.h"
 
 namespace llattn {
 namespace {
@@ -61,20 +60,20 @@ __device__ __forceinline__ void cast_tile(const float* __restrict__ src, uint16_
   }
 }
 
-__global__ __launch_bounds__(256) void cast_kernel(const CastArgs a) {
-  __shared__ uint16_t t[64][72];
+// Workgroup `block` of `blocks`: a tile of a transposed segment, or its share of the chunks.
+__device__ __forceinline__ void cast_block(const CastArgs& a, int block, int blocks, uint16_t (*t)[72]) {
   const int tiles = a.tile_start[a.nseg];
-  if ((int)blockIdx.x < tiles) {  // a tile of a transposed segment (workgroup-uniform branch)
+  if (block < tiles) {  // a tile of a transposed segment (workgroup-uniform branch)
     int s = 0;
-    while (s + 1 < a.nseg && (int)blockIdx.x >= a.tile_start[s + 1]) ++s;
+    while (s + 1 < a.nseg && block >= a.tile_start[s + 1]) ++s;
     const int rows = a.rows[s];
     cast_tile(a.src[s], static_cast<uint16_t*>(a.dst[s]), a.tdst[s], a.tld[s], rows, (int)(a.n[s] / rows),
-              (int)blockIdx.x - a.tile_start[s], t);
+              block - a.tile_start[s], t);
     return;
   }
   const int64_t total = a.start[a.nseg];
-  const int64_t nblk = (int64_t)gridDim.x - tiles;
-  for (int64_t c = ((int64_t)blockIdx.x - tiles) * 256 + threadIdx.x; c < total; c += nblk * 256) {
+  const int64_t nblk = (int64_t)blocks - tiles;
+  for (int64_t c = ((int64_t)block - tiles) * 256 + threadIdx.x; c < total; c += nblk * 256) {
     int s = 0;
     while (s + 1 < a.nseg && c >= a.start[s + 1]) ++s;
     const int64_t e0 = (c - a.start[s]) * 8;  // first element of the chunk within segment s
@@ -98,6 +97,36 @@ __global__ __launch_bounds__(256) void cast_kernel(const CastArgs a) {
       }
     }
   }
+}
+
+__global__ __launch_bounds__(256) void cast_kernel(const CastArgs a) {
+  __shared__ uint16_t t[64][72];
+  cast_block(a, blockIdx.x, gridDim.x, t);
+}
+
+// The casts with the poolings of the same step: neither reads what the other writes.  At a few thousand tokens a
+// pooling (one pass over a segment's rows per workgroup, ~100 workgroups) is bound by its chain of loads, which hides
+// behind the casts' bytes; at more both are bound by bandwidth and one launch saves the drain between them.  The
+// poolings' workgroups come first: theirs is the longer chain.  Measured (MI355X, bf16, two launches -> one): 1024
+// tokens of 1408 dims 15.3 + 5.0 -> 15.9 us, 3 x 1337 tokens 15.2 + 6.3 -> 16.8, 4 x 8192 of 1024 dims 9.7 + 17 -> 19.8.
+struct PoolList {
+  PoolArgs p[kCastPools];
+  int32_t segs[kCastPools], end[kCastPools];  // segments of all batches; workgroups up to and including this pooling's
+};
+
+template <typename T>
+__global__ __launch_bounds__(256) void cast_pool_kernel(const CastArgs a, const PoolList l) {
+  __shared__ union {
+    uint16_t t[64][72];
+    float red[kPoolLds];
+  } s;
+  const int block = blockIdx.x;
+  if (block >= l.end[kCastPools - 1]) {  // workgroup-uniform
+    cast_block(a, block - l.end[kCastPools - 1], gridDim.x - l.end[kCastPools - 1], s.t);
+    return;
+  }
+  const int q = block >= l.end[0], w = block - (q ? l.end[0] : 0);
+  pool_strip<T>(l.p[q], w % l.segs[q], w / l.segs[q], s.red);
 }
 
 // dst[c][r] = src[r][c] for a bf16 matrix, in 64 x 64 tiles through LDS: 16-byte row reads of src and 16-byte
@@ -146,15 +175,16 @@ extern "C" int32_t llattn_transpose(const void* src, int64_t ld_src, int32_t row
   return check_launch("llattn_transpose");
 }
 
-extern "C" int32_t llattn_cast_transposed(int32_t nseg, const float* const* src, void* const* dst,
-                                          const int64_t* n, const int32_t* dst_dtype, void* const* dst_t,
-                                          const int64_t* ld_t, const int32_t* rows, void* stream) {
+namespace {
+// Checks the segments and fills the kernel's arguments; blocks: its workgroups (0: nothing to do).
+int32_t prepare_cast(int32_t nseg, const float* const* src, void* const* dst, const int64_t* n, const int32_t* dst_dtype,
+                     void* const* dst_t, const int64_t* ld_t, const int32_t* rows, CastArgs* args, int64_t* blocks) {
   if (nseg < 1 || nseg > LLATTN_CAST_MAX_SEGS)
     return fail(LLATTN_ERR_SHAPE, "llattn_cast: %d segments (1 to %d supported)", nseg, LLATTN_CAST_MAX_SEGS);
   if (!src || !dst || !n || !dst_dtype) return fail(LLATTN_ERR_LAYOUT, "llattn_cast: null argument array");
   if (dst_t && (!ld_t || !rows))
     return fail(LLATTN_ERR_LAYOUT, "llattn_cast_transposed: dst_t given without ld_t and rows");
-  CastArgs a{};
+  CastArgs& a = *args;
   a.nseg = nseg;
   int64_t chunks = 0, tiles = 0;
   for (int i = 0; i < nseg; ++i) {
@@ -189,9 +219,51 @@ extern "C" int32_t llattn_cast_transposed(int32_t nseg, const float* const* src,
   }
   a.start[nseg] = chunks;
   a.tile_start[nseg] = (int32_t)tiles;
-  if (chunks == 0 && tiles == 0) return LLATTN_OK;
-  const int64_t blocks = tiles + std::min<int64_t>((chunks + 255) / 256, 4096);
+  *blocks = tiles + std::min<int64_t>((chunks + 255) / 256, 4096);
+  return LLATTN_OK;
+}
+}  // namespace
+
+extern "C" int32_t llattn_cast_transposed(int32_t nseg, const float* const* src, void* const* dst,
+                                          const int64_t* n, const int32_t* dst_dtype, void* const* dst_t,
+                                          const int64_t* ld_t, const int32_t* rows, void* stream) {
+  CastArgs a{};
+  int64_t blocks = 0;
+  const int32_t rc = prepare_cast(nseg, src, dst, n, dst_dtype, dst_t, ld_t, rows, &a, &blocks);
+  if (rc || blocks == 0) return rc;
   hipLaunchKernelGGL(cast_kernel, dim3((unsigned)blocks), dim3(256), 0, static_cast<hipStream_t>(stream), a);
+  return check_launch("llattn_cast");
+}
+
+int32_t llattn::cast_and_pool(int32_t nseg, const float* const* src, void* const* dst, const int64_t* n,
+                              const int32_t* dst_dtype, void* const* dst_t, const int64_t* ld_t, const int32_t* rows,
+                              const PoolArgs* pools, int32_t n_pools, int32_t pool_dtype, void* stream) {
+  CastArgs a{};
+  PoolList l{};
+  int64_t blocks = 0, pool_blocks = 0;
+  if (nseg > 0) {
+    const int32_t rc = prepare_cast(nseg, src, dst, n, dst_dtype, dst_t, ld_t, rows, &a, &blocks);
+    if (rc) return rc;
+  }
+  if (n_pools < 1 || n_pools > kCastPools)
+    return fail(LLATTN_ERR_SHAPE, "cast_and_pool: %d poolings (1 to %d supported)", n_pools, kCastPools);
+  for (int q = 0; q < kCastPools; ++q) {
+    if (q < n_pools) {
+      const int32_t rc = check_pool("llattn_pool_fwd", pools[q], pool_dtype);
+      if (rc) return rc;
+      const dim3 g = pool_grid(pools[q], pool_dtype);
+      l.p[q] = pools[q];
+      l.segs[q] = (int32_t)g.x;
+      pool_blocks += (int64_t)g.x * g.y;
+    }
+    if (blocks + pool_blocks > INT32_MAX) return fail(LLATTN_ERR_SHAPE, "llattn_pool_fwd: too many segments");
+    l.end[q] = (int32_t)pool_blocks;
+  }
+  const dim3 grid((unsigned)(blocks + pool_blocks));
+  if (pool_dtype == LLATTN_F32)
+    hipLaunchKernelGGL(cast_pool_kernel<float>, grid, dim3(256), 0, static_cast<hipStream_t>(stream), a, l);
+  else
+    hipLaunchKernelGGL(cast_pool_kernel<uint16_t>, grid, dim3(256), 0, static_cast<hipStream_t>(stream), a, l);
   return check_launch("llattn_cast");
 }
 

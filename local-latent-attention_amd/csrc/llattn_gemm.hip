@@ -9,7 +9,8 @@
 //   input grad dx = dy W          A = dy [M][K],  B = W stored [K][N]
 //   weight grad dW = dy^T x       A = dy stored [K][M], B = x stored [K][N]
 //
-// Tiling: a 256-thread workgroup (4 waves, 2 x 2) owns a 256 x 256 tile of C;
+// Tiling (this file; products of few such tiles run on the smaller ones of llattn_gemm_tile.hip): a 256-thread
+// workgroup (4 waves, 2 x 2) owns a 256 x 256 tile of C;
 // each wave owns 128 x 128 (64 accumulators of 16 x 16, v_mfma_f32_16x16x32_bf16,
 // held in AGPRs).  K advances in steps of 64 through two LDS stages of 64 KB.
 // Tiles move from HBM to LDS with buffer_load_dwordx4 ... lds (no register

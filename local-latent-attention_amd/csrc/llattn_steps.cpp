@@ -17,6 +17,7 @@
 
 #include "llattn_abi.h"
 #include "llattn_pair.h"
+#include "llattn_pool.h"
 #include "llattn_steps.h"
 
 namespace llattn {
@@ -144,6 +145,18 @@ struct Casts {
     e.run([&] {
       return any_t ? llattn_cast_transposed(n, src, dst, count, dt, dst_t, ld_t, rows, e.stream)
                    : llattn_cast(n, src, dst, count, dt, e.stream);
+    });
+  }
+  // with up to two poolings of x [B][T][D] in the same launch
+  int n_pools = 0;
+  llattn::PoolArgs pools[llattn::kCastPools];
+  void pool(const void* x, void* out, int B, int T, int D, int seg, int segs, int div) {
+    pools[n_pools++] = llattn::PoolArgs{x, (int64_t)T * D, D, out, (int64_t)segs * D, D, B, T, D, seg, segs, div, 0};
+  }
+  void launch_with_pools(Exec& e, int pool_dtype) {
+    e.run([&] {
+      return llattn::cast_and_pool(n, src, dst, count, dt, any_t ? dst_t : nullptr, ld_t, rows, pools, n_pools,
+                                   pool_dtype, e.stream);
     });
   }
 };
@@ -334,15 +347,15 @@ void block_fwd(Exec& e, const llattn_block_cfg& c, const llattn_block_params& p,
     casts.add(p.w_out, k.w_out, Dm, Dm, dt, k.w_outt, Dm);
     casts.add(p.w_r, k.core.r_w, d.D, d.Ld, dt, k.core.r_wt, d.D);
   }
-  casts.launch(e);
+  if (c.macro) {
+    if (!twin_pools(c)) casts.pool(x, k.pq, d.B, d.T, (int)Dm, s.q_block, d.nq, LLATTN_DIV_SEG);
+    else casts.pool(x, k.pooled, d.B, d.T, (int)Dm, s.chunk, d.nc, LLATTN_DIV_SEG);
+  }
+  if (!twin_pools(c)) casts.pool(x, k.pooled, d.B, d.T, (int)Dm, s.chunk, d.nc, LLATTN_DIV_COUNT);
+  casts.launch_with_pools(e, dt);
   const Weights w = block_weights(c, p, k);
   const llattn_heads_layout hl{d.T, d.Dh, 3 * d.H, c.macro ? 0 : d.Ldh};
   const bool f32 = dt == LLATTN_F32;
-  if (c.macro) {
-    if (!twin_pools(c)) e.pool(dt, x, k.pq, d.B, d.T, (int)Dm, s.q_block, d.nq, LLATTN_DIV_SEG);
-    else e.pool(dt, x, k.pooled, d.B, d.T, (int)Dm, s.chunk, d.nc, LLATTN_DIV_SEG);
-  }
-  if (!twin_pools(c)) e.pool(dt, x, k.pooled, d.B, d.T, (int)Dm, s.chunk, d.nc, LLATTN_DIV_COUNT);
   e.gemm(e.linear(dt, (int)d.M, (int)width, (int)Dm, x, w.qkv, w.b_qkv, k.qkvr, c.heads ? &hl : nullptr),
          e.linear(dt, d.B * d.nc, (int)(2 * d.Ld), (int)Dm, k.pooled, w.rkv, p.b_rkv, k.gkgv), f32);
   if (c.macro) e.gemm(e.linear(dt, (int)d.Mq, (int)d.Ld, (int)Dm, k.pq, w.rq, p.b_rq, k.rq), f32);

@@ -233,3 +233,22 @@ def test_ffn_step_matches_python_path(shape, d_ff, bias):
 
     _close(*_both(run, "llattn_ffn_bwd"), True)
     _close(*_both(lambda: run(False), "llattn_ffn_fwd"), True)
+
+
+@pytest.mark.parametrize("seg", [1, 7, 8, 9, 25, 32, 33, 57, 100, 128])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_pool_segment_lengths(seg, dtype):
+    """Segments around the eight row groups and their four rows in flight, the last one short.  fp32 sums of `seg`
+    terms: seg * 2^-24 of the sum of magnitudes; a bf16 result rounds by at most 2^-8 of itself on top."""
+    from llattn_amd import DIV_COUNT, pool
+    dev = require_cuda()
+    print("case: pool", seg, dtype, flush=True)
+    n, B, D = 5, 2, 264
+    T = n * seg - seg // 3
+    x = torch.randn(B, T, D, device=dev, generator=torch.Generator(device=dev).manual_seed(seg)).to(dtype)
+    got = pool(x, seg, n, DIV_COUNT).double().cpu()
+    for i in range(n):
+        rows = x[:, i * seg:(i + 1) * seg].double().cpu()
+        ref, mag = rows.mean(1), rows.abs().mean(1)
+        tol = (seg + 2) * 2.0 ** -24 * mag + (2.0 ** -8 * ref.abs() if dtype == torch.bfloat16 else 0)
+        assert ((got[:, i] - ref).abs() <= tol).all(), i
