@@ -231,8 +231,8 @@ struct TilePlan { int mb, nb, kg; };
 TilePlan tile_plan(const llattn_gemm_desc* d, double* us = nullptr);  // us: the time it expects
 void launch_tile(const GemmArgs& a, const TilePlan& p, bool a_kmaj, bool b_kmaj, int c_dtype, hipStream_t st);
 // Two independent products in one launch: x Wᵀ or dy W into bf16, and then dyᵀ x into fp32 or (after x Wᵀ) another x Wᵀ.
-int pair_plan(const llattn_gemm_desc* d0, const llattn_gemm_desc* d1);
-void launch_pair(GemmArgs a0, GemmArgs a1, int mb, bool b_kmaj0, bool weight1, hipStream_t st);
+TilePlan pair_plan(const llattn_gemm_desc* d0, const llattn_gemm_desc* d1);
+void launch_pair(GemmArgs a0, GemmArgs a1, const TilePlan& p, bool b_kmaj0, bool weight1, hipStream_t st);
 
 }  // namespace gemm
 }  // namespace llattn

@@ -924,21 +924,21 @@ namespace llattn {
 namespace gemm {
 
 size_t pair_workspace(const llattn_gemm_desc* d0, const llattn_gemm_desc* d1) {
-  if (pair_plan(d0, d1)) return 0;
+  if (pair_plan(d0, d1).mb) return 0;
   return std::max(llattn_gemm_workspace_size(d0), llattn_gemm_workspace_size(d1));
 }
 
 int32_t run_pair(const llattn_gemm_desc* d0, const llattn_gemm_desc* d1, void* workspace, size_t workspace_bytes,
                  void* stream) {
-  const int mb = pair_plan(d0, d1);
-  if (!mb) {
+  const TilePlan p = pair_plan(d0, d1);
+  if (!p.mb) {
     if (const int32_t rc = llattn_gemm(d0, workspace, workspace_bytes, stream)) return rc;
     return llattn_gemm(d1, workspace, workspace_bytes, stream);
   }
   GemmArgs a0, a1;
   if (const int32_t rc = prepare(d0, nullptr, 0, true, a0)) return rc;
   if (const int32_t rc = prepare(d1, nullptr, 0, true, a1)) return rc;
-  launch_pair(a0, a1, mb, !d0->b_trans, d1->a_trans, static_cast<hipStream_t>(stream));
+  launch_pair(a0, a1, p, !d0->b_trans, d1->a_trans, static_cast<hipStream_t>(stream));
   return check_launch("llattn_gemm");
 }
 

@@ -114,9 +114,9 @@ __device__ __forceinline__ void finish4(const GemmArgs& a, int row, int col, f32
 
 constexpr int stage_bytes(int mb, int nb) { return 32 * (mb + nb) * 128; }
 
-// Workgroup `block` of `blocks` of a product; smem: KG NST stages, rsl: [KG][32 MB].
+// Workgroup `block` of `blocks` of a product; smem: KG NST stages.
 template <bool AK, bool BKM, int EPI, int MB, int NB, int KG, int NST>
-__device__ __forceinline__ void tile_product(const GemmArgs& a, int block, int blocks, unsigned char* smem, float* rsl) {
+__device__ __forceinline__ void tile_product(const GemmArgs& a, int block, int blocks, unsigned char* smem) {
   constexpr int TM = 32 * MB, TN = 32 * NB;
   typedef TileOp<AK, false, TM> OpA;
   typedef TileOp<BKM, false, TN> OpB;
@@ -195,6 +195,12 @@ __device__ __forceinline__ void tile_product(const GemmArgs& a, int block, int b
     }
   }
   __builtin_amdgcn_s_waitcnt(wait_vm_lgkm0(0));  // no DMA in flight past this point
+  // [KG][32 MB] row sums: behind the partial sums of the k groups where the stages leave room; for one k group, which
+  // has none, in the stages themselves (five 64 x 64 workgroups then fill a CU's LDS to the byte)
+  constexpr bool OWN = KG > 1 && NST * STAGE == MB * NB * 4096;
+  __shared__ float own[OWN ? KG * TM : 1];
+  float* rsl = OWN ? own : reinterpret_cast<float*>(smem + (KG > 1 ? KG * MB * NB * 4096 : 0));
+  if (!OWN && a.rowsum && n0 == 0) __syncthreads();  // every wave's loads have landed and its fragments are read
   if (rs) {  // the four lane groups hold the row's four 8-wide k slices
 #pragma unroll
     for (int i = 0; i < MB; ++i) {
@@ -238,32 +244,33 @@ __device__ __forceinline__ void tile_product(const GemmArgs& a, int block, int b
 template <bool AK, bool BKM, int EPI, int MB, int NB, int KG, int NST>
 __global__ __launch_bounds__(256 * KG) void gemm_tile_kernel(const GemmArgs a) {
   __shared__ __align__(1024) unsigned char smem[KG * NST * stage_bytes(MB, NB)];
-  __shared__ float rsl[KG * 32 * MB];
-  tile_product<AK, BKM, EPI, MB, NB, KG, NST>(a, blockIdx.x, gridDim.x, smem, rsl);
+  tile_product<AK, BKM, EPI, MB, NB, KG, NST>(a, blockIdx.x, gridDim.x, smem);
 }
 
 // Two independent products in one launch: the first n0 workgroups (a multiple of 8, so that both see their XCD) take
 // the first one.  An input and a weight gradient of the same dy, or two projections, each fill the chip badly at a
 // few thousand rows; together they share its last round and one launch.
-template <bool AK0, bool BK0, int EPI0, bool AK1, bool BK1, int EPI1, int MB>
-__global__ __launch_bounds__(256) void gemm_tile_pair_kernel(const GemmArgs a0, const GemmArgs a1, int n0) {
-  __shared__ __align__(1024) unsigned char smem[2 * stage_bytes(MB, MB)];
-  __shared__ float rsl[32 * MB];
+template <bool AK0, bool BK0, int EPI0, bool AK1, bool BK1, int EPI1, int MB, int KG>
+__global__ __launch_bounds__(256 * KG) void gemm_tile_pair_kernel(const GemmArgs a0, const GemmArgs a1, int n0) {
+  __shared__ __align__(1024) unsigned char smem[KG * 2 * stage_bytes(MB, MB)];
   const int b = blockIdx.x, c0 = a0.tiles_m * a0.tiles_n, c1 = a1.tiles_m * a1.tiles_n;
   if (b < n0) {
-    if (b < c0) tile_product<AK0, BK0, EPI0, MB, MB, 1, 2>(a0, b, c0, smem, rsl);
+    if (b < c0) tile_product<AK0, BK0, EPI0, MB, MB, KG, 2>(a0, b, c0, smem);
   } else if (b - n0 < c1) {
-    tile_product<AK1, BK1, EPI1, MB, MB, 1, 2>(a1, b - n0, c1, smem, rsl);
+    tile_product<AK1, BK1, EPI1, MB, MB, KG, 2>(a1, b - n0, c1, smem);
   }
 }
 
-// 128 x 128 tiles run two workgroups per CU with one k group, 64 x 64 tiles four; with more k groups one.
+// 128 x 128 tiles run two workgroups per CU with one k group, one with two; 64 x 64 tiles five with one, and with two k
+// groups one of four stages each, or two of two stages where there are more tiles than CUs (1024 x 1408 x 4096, 352
+// tiles: two rounds of the first 31 us, one of the second 26; 333 x 1408 x 4096, 132 tiles: 17 against 24).
 template <bool AK, bool BKM, int EPI>
 void launch_epi(const GemmArgs& a, const TilePlan& p, hipStream_t st) {
   const dim3 grid(a.tiles_m * a.tiles_n);
   if (p.mb == 4 && p.kg == 1) hipLaunchKernelGGL((gemm_tile_kernel<AK, BKM, EPI, 4, 4, 1, 2>), grid, dim3(256), 0, st, a);
   else if (p.mb == 4) hipLaunchKernelGGL((gemm_tile_kernel<AK, BKM, EPI, 4, 4, 2, 2>), grid, dim3(512), 0, st, a);
   else if (p.kg == 1) hipLaunchKernelGGL((gemm_tile_kernel<AK, BKM, EPI, 2, 2, 1, 2>), grid, dim3(256), 0, st, a);
+  else if (grid.x > 256) hipLaunchKernelGGL((gemm_tile_kernel<AK, BKM, EPI, 2, 2, 2, 2>), grid, dim3(512), 0, st, a);
   else hipLaunchKernelGGL((gemm_tile_kernel<AK, BKM, EPI, 2, 2, 2, 4>), grid, dim3(512), 0, st, a);
 }
 template <bool AK, bool BKM>
@@ -274,7 +281,7 @@ void launch_dt(const GemmArgs& a, const TilePlan& p, int c_dtype, hipStream_t st
 
 }  // namespace
 
-// Time in us of the 256 x 256 kernels with S k splits: rounds of (tile, split) workgroups over 256 CUs, 1.2 us per
+// Time in us of the 256 x 256 kernels with S k splits: 6 us to fill and drain, rounds of (tile, split) workgroups over 256 CUs, 1.2 us per
 // 64-k step of a workgroup alone up to 1.75 with every CU at work, and for S > 1 the ordered reduction with its fp32
 // partials written and read at 7 TB/s.  (1024 x 4736 x 1408, 76 tiles: 32 us; 8192 x 4096 x 1408, 512: 83;
 // 1536 x 1536 x 4011, 36 tiles in 7 splits: 41.)
@@ -282,21 +289,25 @@ static double big_us(int64_t M, int64_t N, int steps, int S) {
   const int64_t n = ((M + BM - 1) / BM) * ((N + BN - 1) / BN) * S;
   const double last = (double)(n % 256) / 256.0;
   const double per = (double)(n / 256) * 1.75 + (n % 256 ? 1.2 + 0.55 * last * last : 0.0);
-  return 4.0 + (double)((steps + S - 1) / S) * per + (S > 1 ? 7.0 + 8.0 * S * (double)M * (double)N / 7e6 : 0.0);
+  return 6.0 + (double)((steps + S - 1) / S) * per + (S > 1 ? 7.0 + 8.0 * S * (double)M * (double)N / 7e6 : 0.0);
 }
 
-// The tiles that a product takes, fitted to a sweep of 42 products (16 x 1024 x 1408 to 32768 x 1408 x 512; all layouts):
-//   128 x 128, one k group: rounds of two tiles per CU, 1.27 us per 64-k step (1.1 for a last round of up to two, 0.75
-//   for one), 4 us once;  two k groups: rounds of one, 3.4 us each and 1.0 to 1.22 us per step of a group;
-//   64 x 64, one k group: rounds of four tiles per CU, 0.85 us per step (0.35 for a last round of one, 0.44 of two, 0.6
-//   of three; a fifth more for one or two over a long contraction), 3 us once;  two k groups: rounds of one, 2.4 us
-//   each and 0.45 per step of a group.  (Four k groups: within 3% of two.)
+// The tiles that a product takes, fitted to the times of 38 products (16 x 1024 x 1408 to 3000 x 4736 x 1408; all
+// layouts) whose operands the launches before had just written, as a step finds them: 2-5 us longer than on operands
+// left in L2 by the same product.
+//   128 x 128, one k group: rounds of two tiles per CU, 1.27 us per 64-k step (1.02 for a last round of up to two, 0.75
+//   for one), 8.5 us once;  two k groups: rounds of one, 5.5 us each and 0.95 per step of a group;
+//   64 x 64, one k group: rounds of four tiles per CU, 0.85 us per step (0.5 for a last round of one, 0.52 of two, 0.68
+//   of three), 4.5 us once;  two k groups: 0.44 us per step of a group for up to one tile per CU, 0.68 for up to two.
+//   (Four k groups: no faster.)
 // Only where 256 x 256 tiles leave CUs idle (below 224 of them): from there on
 // those tiles' half as large operand traffic wins (4011 x 4992 x 1536: 69 us against 81).  Neither the epilogue nor
 // the layouts enter, so a product has the same bits whichever way it is stored.
-// Measured against the 256 x 256 kernels and the register-staged 64 x 64 tiles that this replaced:
-//   333 x 4736 x 1408: 30 -> 12.5 us;  1024 x 4096 x 1408: 30 -> 17;  1536 x 384 x 4011 (dyT x): 52 -> 18;
-//   4011 x 384 x 1536 (dy W): 25 -> 13;  32768 x 64 x 1024: 24 -> 13;  1024 x 1408 x 1408: 15 -> 12.
+// Measured on operands just written, in us: 333 x 4736 x 1408 13.5, 1024 x 1408 x 1408 13.3,
+// 1024 x 1408 x 4096 26.8, 1024 x 4096 x 1408 18.7, 4011 x 384 x 1536 (dy W) 14.3, 1536 x 384 x 4011 (dyT x) 18.5;
+// with L2-resident operands against the 256 x 256 kernels and the register-staged 64 x 64 tiles that this replaced:
+//   333 x 4736 x 1408: 30 -> 12.5;  1024 x 4096 x 1408: 30 -> 17;  1536 x 384 x 4011: 52 -> 18;  32768 x 64 x 1024:
+//   24 -> 13.
 TilePlan tile_plan(const llattn_gemm_desc* d, double* us) {
   const TilePlan none{0, 0, 0};
   if (d->split_k > 0 || d->M <= 0 || d->N <= 0 || d->K <= 0) return none;
@@ -314,12 +325,12 @@ TilePlan tile_plan(const llattn_gemm_desc* d, double* us) {
   const int64_t t128 = ((M + 127) / 128) * ((N + 127) / 128), t64 = ((M + 63) / 64) * ((N + 63) / 64);
   const auto split = [&](int kg) { return (double)((steps + kg - 1) / kg); };
   const int64_t r128 = t128 % 512, r64 = (t64 % 1024 + 255) / 256;
-  take(4.0 + steps * ((double)(t128 / 512) * 1.27 + (r128 == 0 ? 0.0 : r128 <= 256 ? 0.75 : 1.1)), 4, 1);
-  const auto rounds = [](int64_t t) { return (double)((t + 255) / 256); };
-  if (steps >= 4) take(0.6 + rounds(t128) * (3.4 + split(2) * (1.0 + 0.22 * std::min(1.0, (double)t128 / 256.0))), 4, 2);
-  const double lengthy = 1.0 + 0.2 * std::min(1.0, steps / 48.0), last[] = {0.0, 0.35 * lengthy, 0.44 * lengthy, 0.6, 0.82};
-  take(3.0 + steps * ((double)(t64 / 1024) * 0.85 + last[r64]), 2, 1);
-  if (steps >= 4) take(0.6 + rounds(t64) * (2.4 + split(2) * 0.45), 2, 2);
+  take(8.5 + steps * ((double)(t128 / 512) * 1.27 + (r128 == 0 ? 0.0 : r128 <= 256 ? 0.75 : 1.02)), 4, 1);
+  if (steps >= 4) take(3.0 + (double)((t128 + 255) / 256) * (5.5 + split(2) * 0.95), 4, 2);
+  const double last[] = {0.0, 0.5, 0.52, 0.68, 0.82};
+  take(4.5 + steps * ((double)(t64 / 1024) * 0.85 + last[r64]), 2, 1);
+  if (steps >= 4 && t64 <= 256) take(3.8 + split(2) * 0.44, 2, 2);
+  if (steps >= 4 && t64 > 256 && t64 <= 512) take(5.6 + split(2) * 0.68, 2, 2);
   if (us) *us = best_t;
   return best;
 }
@@ -345,56 +356,67 @@ double alone_us(const llattn_gemm_desc* d) {
   return t;
 }
 
-template <int MB>
-void launch_pair_mb(const GemmArgs& a0, const GemmArgs& a1, bool nt0, bool nt1, int n0, dim3 grid, hipStream_t st) {
-  const dim3 block(256);
-  if (nt1) hipLaunchKernelGGL((gemm_tile_pair_kernel<true, true, EPI_BF16, true, true, EPI_BF16, MB>), grid, block, 0, st, a0, a1, n0);
-  else if (nt0) hipLaunchKernelGGL((gemm_tile_pair_kernel<true, true, EPI_BF16, false, false, EPI_F32, MB>), grid, block, 0, st, a0, a1, n0);
-  else hipLaunchKernelGGL((gemm_tile_pair_kernel<true, false, EPI_BF16, false, false, EPI_F32, MB>), grid, block, 0, st, a0, a1, n0);
+template <int MB, int KG>
+void launch_pair_as(const GemmArgs& a0, const GemmArgs& a1, bool nt0, bool nt1, int n0, dim3 grid, hipStream_t st) {
+  const dim3 block(256 * KG);
+  if (nt1)
+    hipLaunchKernelGGL((gemm_tile_pair_kernel<true, true, EPI_BF16, true, true, EPI_BF16, MB, KG>), grid, block, 0, st,
+                       a0, a1, n0);
+  else if (nt0)
+    hipLaunchKernelGGL((gemm_tile_pair_kernel<true, true, EPI_BF16, false, false, EPI_F32, MB, KG>), grid, block, 0, st,
+                       a0, a1, n0);
+  else
+    hipLaunchKernelGGL((gemm_tile_pair_kernel<true, false, EPI_BF16, false, false, EPI_F32, MB, KG>), grid, block, 0, st,
+                       a0, a1, n0);
 }
 
 }  // namespace
 
-// Tile of two products in one launch (32 mb squared, one k group), or 0 where they are better run one by one: the
-// work of all tiles at a full chip's rate per (tile, step), or the longest tile at the rate of the tiles that share
-// its CU, and a third of a shorter one for the ragged end; taken where that saves 5%.  (q|k|v and the latents' keys and
-// values of a 0.55b layer over 333 tokens: 18 us in one launch, 17 + 8 in two; the latent projections' two gradients of
-// 4 x 8192 tokens with 64-token query blocks 11.5 us, 5 + 10.  The gradients of a few thousand tokens' large projections stay apart: the weight
-// gradient's long contraction wants its own k split.)
-int pair_plan(const llattn_gemm_desc* d0, const llattn_gemm_desc* d1) {
+// Tiles of two products in one launch, or none where they are better run one by one: the work of all tiles at a full
+// chip's rate per (tile, step), or the longest tile at the rate of the tiles that share its CU, and part of a shorter
+// one for the ragged end; taken where that saves 5%.  (q|k|v and the latents' keys and values of a 0.55b layer over 333
+// tokens: 17 + 8 us in two launches, 18 in one of one k group, 14 of two; the latent projections' two gradients of
+// 4 x 8192 tokens with 64-token query blocks 5 + 10 us in two, 11.5 in one.  The gradients of a few thousand tokens'
+// large projections stay apart: the weight gradient's long contraction wants its own k split.)
+TilePlan pair_plan(const llattn_gemm_desc* d0, const llattn_gemm_desc* d1) {
+  const TilePlan none{0, 0, 0};
   for (const llattn_gemm_desc* d : {d0, d1})
-    if (d->split_k > 0 || d->M <= 0 || d->N <= 0 || d->K <= 0) return 0;
+    if (d->split_k > 0 || d->M <= 0 || d->N <= 0 || d->K <= 0) return none;
   const bool bf0 = d0->c_dtype == LLATTN_BF16 && !d0->a_trans, nt1 = d1->c_dtype == LLATTN_BF16 && !d1->a_trans && !d1->b_trans;
   const bool tn1 = d1->c_dtype == LLATTN_F32 && d1->a_trans && d1->b_trans;
-  if (!bf0 || !(tn1 || (nt1 && !d0->b_trans))) return 0;
+  if (!bf0 || !(tn1 || (nt1 && !d0->b_trans))) return none;
   const double s0 = (d0->K + SK - 1) / SK, s1 = (d1->K + SK - 1) / SK;
   double best_t = 0.95 * (alone_us(d0) + alone_us(d1));
-  int best = 0;
-  for (int mb : {4, 2}) {
+  TilePlan best = none;
+  const auto take = [&](int mb, int kg, double fill, double rate, const auto& alone) {
     const int64_t T = 32 * mb;
-    const double t0 = (double)(((d0->M + T - 1) / T) * ((d0->N + T - 1) / T)), t1 = (double)(((d1->M + T - 1) / T) * ((d1->N + T - 1) / T));
-    const double n = t0 + t1, most = std::max(s0, s1), least = std::min(s0, s1);
-    double t;
-    if (mb == 4) t = 4.0 + std::max((t0 * s0 + t1 * s1) * 1.27 / 512.0, (n <= 256 ? 0.75 : 1.1) * most) + 0.3 * least;
-    else t = 3.0 + std::max((t0 * s0 + t1 * s1) * 0.85 / 1024.0, (n <= 256 ? 0.38 : n <= 512 ? 0.5 : n <= 768 ? 0.6 : 0.82) * most) + 0.15 * least;
+    const double t0 = (double)(((d0->M + T - 1) / T) * ((d0->N + T - 1) / T));
+    const double t1 = (double)(((d1->M + T - 1) / T) * ((d1->N + T - 1) / T));
+    const double most = std::max(s0, s1), least = std::min(s0, s1), step = alone(t0 + t1);
+    if (step == 0.0) return;
+    const double t = fill + std::max((t0 * s0 + t1 * s1) * rate, step * most) + 0.18 * step * least;
     if (t < best_t) {
       best_t = t;
-      best = mb;
+      best = TilePlan{mb, mb, kg};
     }
-  }
+  };
+  take(4, 1, 8.5, 1.27 / 512.0, [](double n) { return n <= 256 ? 0.75 : 1.02; });
+  take(2, 1, 4.5, 0.85 / 1024.0, [](double n) { return n <= 512 ? 0.52 : n <= 768 ? 0.68 : 0.82; });
+  if (s0 >= 4 && s1 >= 4) take(2, 2, 5.6, 0.8 / 1024.0, [](double n) { return n <= 512 ? 0.34 : 0.0; });
   return best;
 }
 
-void launch_pair(GemmArgs a0, GemmArgs a1, int mb, bool b_kmaj0, bool weight1, hipStream_t st) {
-  const int T = 32 * mb;
+void launch_pair(GemmArgs a0, GemmArgs a1, const TilePlan& p, bool b_kmaj0, bool weight1, hipStream_t st) {
+  const int T = 32 * p.mb;
   for (GemmArgs* a : {&a0, &a1}) {
     a->tiles_m = (a->M + T - 1) / T;
     a->tiles_n = (a->N + T - 1) / T;
   }
   const int n0 = (a0.tiles_m * a0.tiles_n + 7) / 8 * 8;
   const dim3 grid(n0 + a1.tiles_m * a1.tiles_n);
-  if (mb == 4) launch_pair_mb<4>(a0, a1, b_kmaj0, !weight1, n0, grid, st);
-  else launch_pair_mb<2>(a0, a1, b_kmaj0, !weight1, n0, grid, st);
+  if (p.mb == 4) launch_pair_as<4, 1>(a0, a1, b_kmaj0, !weight1, n0, grid, st);
+  else if (p.kg == 1) launch_pair_as<2, 1>(a0, a1, b_kmaj0, !weight1, n0, grid, st);
+  else launch_pair_as<2, 2>(a0, a1, b_kmaj0, !weight1, n0, grid, st);
 }
 
 }  // namespace gemm

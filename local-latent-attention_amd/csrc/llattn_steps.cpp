@@ -1,10 +1,11 @@
 // Whole steps of the attention block, its core and the feed-forward (include/llattn_steps.h): the launches of the
 // single entry points in a row.  A training pass of the block is ~25 launches whose kernels take 5-50 us each at a
 // few thousand tokens; issued one by one from Python (a call of 15-25 us each: argument structs, workspace queries,
-// output tensors) the GPU waited for the host.  One call issues them in about 4 us each.  Measured (MI355X, a pass,
-// before -> now): a 0.55b layer's forward over 333 tokens 267 -> 100 us, its fwd + bwd over 3 x 1337 tokens (0.60b)
-// 905 -> 640 us, the op at head dim 128 over 2 x 3001 tokens 488 -> 293 us (53 us of it gradients laid out as their
-// inputs, which autograd then need not copy), the 0.55b model over 1024 tokens 9.4 -> 4.9 ms.
+// output tensors) the GPU waited for the host.  One call issues them in about 4 us each.  Measured (MI355X, a pass
+// before -> with these calls; in brackets with the kernels for small products since): a 0.55b layer's forward over 333
+// tokens 267 -> 100 us (56), its fwd + bwd over 3 x 1337 tokens (0.60b) 905 -> 640 us (574), the op at head dim 128 over
+// 2 x 3001 tokens 488 -> 293 us (270; 53 us of it gradients laid out as their inputs, which autograd then need not
+// copy), the 0.55b model over 1024 tokens 9.4 -> 4.9 ms (3.9).
 //
 // The sequences are those of the Python path (module.py, ops.py, linear.py, ffn.py: kept for profiling and for
 // parameters this path does not take), product by product with the same operands and roundings.  Two products that do

@@ -639,7 +639,8 @@ def test_scaled_input_grad_through_the_transpose(M, K, N):
 
 
 @pytest.mark.parametrize("M,N,K", [(8, 8, 8), (64, 64, 64), (264, 136, 72), (72, 136, 200), (1000, 520, 328),
-                                   (1000, 4104, 264), (1000, 4104, 1032), (1024, 4096, 1408), (1288, 72, 4008)])
+                                   (1000, 1416, 328), (1000, 4104, 264), (1000, 4104, 1032), (1024, 4096, 1408),
+                                   (1288, 72, 4008)])
 def test_gemm_tiles_layouts_and_epilogues(M, N, K):
     """The smaller tiles (64 x 64 and 128 x 128, one and two k groups): every operand layout at strides of its own,
     into bf16 and fp32, with bias, accumulation, row addends, the activations, split-head storage and row sums,

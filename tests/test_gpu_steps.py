@@ -65,6 +65,7 @@ BLOCKS = [  # B, T, d_model, heads, latent width, latent heads, window, latents,
     (1, 1, 128, 4, 64, 2, 64, 16, 0),     # one token
     (1, 1, 128, 4, 64, 2, 64, 16, 64),    # one token, one query block
     (3, 333, 128, 4, 64, 2, 64, 16, 0),
+    (1, 333, 1408, 16, 512, 8, 64, 16, 0),  # two projections in one launch with two k groups
     (2, 640, 256, 4, 32, 2, 128, 10, 64),  # query blocks that are the latent chunks: one pooling
     (2, 650, 256, 4, 32, 2, 300, 10, 48),  # others
     (2, 2100, 256, 4, 128, 2, 64, 16, 0),  # transposed weights (4200 rows), split-head storage
