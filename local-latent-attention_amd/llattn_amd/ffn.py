@@ -20,7 +20,7 @@ import torch
 from . import _lib as L
 from . import gemm, ops
 from .linear import pack_params, weight_grad
-from .steps import Ffn, ffn_forward, plain
+from .steps import Ffn, plain
 
 BF16 = torch.bfloat16
 
@@ -80,5 +80,5 @@ def feed_forward(x: torch.Tensor, w1: torch.nn.Linear, w2: torch.nn.Linear) -> t
             and all(p is None or plain(p, dev) for p in ps):
         saved = torch.is_grad_enabled() and (x.requires_grad or any(p is not None and p.requires_grad for p in ps))
         cfg = L.LlattnFfnCfg(rows, d, d_ff, d_out, int(saved))
-        return Ffn.apply(x, cfg, *ps) if saved else ffn_forward(x, cfg, *ps)[0]
+        return Ffn.apply(x, cfg, *ps)
     return _FeedForward.apply(x, *ps)

@@ -188,7 +188,7 @@ class LocalLatentAttentionTriton(nn.Module):
                                int(bf16 and heads_layout_ok(lay, D, not macro)), int(ops._remote_heads(lay, dt)),
                                int(bf16 and grad_heads_ok(B * T, D, D, lay.Dh)),
                                int(bf16 and ops._latent_grad_heads(lay)))
-        return steps.Block.apply(x, cfg, *params) if saved else steps.block_forward(x, cfg, params)[0]
+        return steps.Block.apply(x, cfg, *params)
 
     def _packed_weights(self, macro: bool) -> dict:
         """The bf16 copies of every projection weight that this forward multiplies with (what bf16 autocast casts

@@ -4,7 +4,8 @@ Each autograd function here is the whole of a step that :mod:`llattn_amd.module`
 :mod:`llattn_amd.ffn` otherwise issue product by product from Python: the same products with what the backward
 reads in one buffer (two independent ones may share a launch).  The calls that take this path have parameters in fp32, whole, 16-byte aligned and
 on the activations' device, activations in the compute dtype, and nobody looking at the single calls
-(:func:`llattn_amd.ops.observed`).  The others, and profiling, stay on the Python path.
+(:func:`llattn_amd.ops.observed`).  The others, and profiling, stay on the Python path.  Forward-only calls are
+applied as functions too: a tangent, a batched tensor or a tracer is then met as by any other autograd function.
 """
 from __future__ import annotations
 
@@ -73,6 +74,8 @@ _BWD_F32_MACRO = (0, 2, 4, 6, 8, 10, 11)
 class Block(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, cfg, *params):
+        if not cfg.saved:
+            return block_forward(x, cfg, params)[0]
         params = [None if p is None else p.detach() for p in params]
         out, kept = block_forward(x.detach(), cfg, params)
         which = _BWD_BF16 if cfg.shape.dtype == L.BF16 else _BWD_F32_MACRO if cfg.macro else _BWD_F32
@@ -156,6 +159,8 @@ def ffn_forward(x, cfg, w1, b1, w2, b2):
 class Ffn(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, cfg, w1, b1, w2, b2):
+        if not cfg.saved:
+            return ffn_forward(x, cfg, w1, b1, w2, b2)[0]
         y, kept = ffn_forward(x.detach(), cfg, w1, b1, w2, b2)
         ctx.save_for_backward(x, kept)
         ctx.cfg, ctx.bias = cfg, (b1 is not None, b2 is not None)

@@ -253,3 +253,23 @@ def test_pool_segment_lengths(seg, dtype):
         ref, mag = rows.mean(1), rows.abs().mean(1)
         tol = (seg + 2) * 2.0 ** -24 * mag + (2.0 ** -8 * ref.abs() if dtype == torch.bfloat16 else 0)
         assert ((got[:, i] - ref).abs() <= tol).all(), i
+
+
+@pytest.mark.parametrize("entry", ["block", "ffn"])
+def test_forward_only_steps_refuse_tangents_and_vmap(entry):
+    """A forward that keeps nothing for a backward is still an autograd function: a forward-mode tangent or a batched
+    input raises instead of being dropped."""
+    import torch.autograd.forward_ad as fwad
+    from llattn_amd import LocalLatentAttentionTriton
+    from llattn_amd.ffn import feed_forward
+    dev = require_cuda()
+    m = LocalLatentAttentionTriton(128, 4, 2, 64, 16, 64).to(dev).requires_grad_(False)
+    w1, w2 = (torch.nn.Linear(*s).to(dev).requires_grad_(False) for s in ((128, 256), (256, 128)))
+    fn = m if entry == "block" else lambda t: feed_forward(t, w1, w2)
+    x = torch.randn(2, 64, 128, device=dev).bfloat16()
+    with torch.no_grad(), torch.autocast("cuda", dtype=torch.bfloat16):
+        fn(x)
+        with fwad.dual_level(), pytest.raises(RuntimeError):
+            fn(fwad.make_dual(x, torch.ones_like(x)))
+        with pytest.raises(RuntimeError):
+            torch.func.vmap(fn)(x[None])
