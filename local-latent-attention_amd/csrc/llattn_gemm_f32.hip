@@ -531,9 +531,12 @@ extern "C" int32_t llattn_gemm_f32(const llattn_gemm_desc* d, void* stream) {
   const int64_t a_bytes = (d->a_trans ? (int64_t)(d->K - 1) * d->lda + d->M : (int64_t)(d->M - 1) * d->lda + d->K) * 4;
   const int64_t b_bytes = (d->b_trans ? (int64_t)(d->K - 1) * d->ldb + d->N : (int64_t)(d->N - 1) * d->ldb + d->K) * 4;
   const auto vec = [](const void* p, int64_t ld) { return (int)(aligned16(p) && ld % 4 == 0); };
-  // the LDS kernel moves 16-byte pieces by 32-bit offsets: none may straddle the end of a contiguous dimension
+  // the LDS kernel moves 16-byte pieces by 32-bit offsets: none may straddle the end of a contiguous dimension, and
+  // the rows of a stage that lie past K must be past the extent, not wrapped around into it (SK ld 4 < 2^32)
+  const auto span = [](int32_t trans, int64_t ld) { return !trans || ld < (int64_t(1) << 32) / (4 * SK); };
   const bool lds_ok = vec(d->A, d->lda) && vec(d->B, d->ldb) && (d->a_trans ? d->M : d->K) % 4 == 0 &&
-                      (d->b_trans ? d->N : d->K) % 4 == 0 && a_bytes <= (int64_t)kPast && b_bytes <= (int64_t)kPast;
+                      (d->b_trans ? d->N : d->K) % 4 == 0 && span(d->a_trans, d->lda) && span(d->b_trans, d->ldb) &&
+                      a_bytes <= (int64_t)kPast && b_bytes <= (int64_t)kPast;
   const F32Plan plan = plan_f32(d->M, d->N, d->K, lds_ok);
   const int TM = plan.nb ? 64 : 32, TN = plan.nb ? 32 * plan.nb : 32;
   const int64_t tiles = (int64_t)((d->M + TM - 1) / TM) * ((d->N + TN - 1) / TN);

@@ -619,6 +619,23 @@ def test_gemm_f32_kernels_and_layouts(M, N, K):
                 assert torch.equal(out, again)
 
 
+def test_gemm_f32_wide_strides():
+    """Rows past K at a stride whose byte offsets pass 2^32 within a stage of 32 k do not come back as other rows:
+    the row sums of A are those of its K rows."""
+    from llattn_amd import gemm
+    dev = require_cuda()
+    M, N, K, ld = 3072, 1024, 20, 50_000_000
+    print("case: gemm f32 wide strides", flush=True)
+    g = torch.Generator(device=dev).manual_seed(1)
+    a = torch.ones((K - 1) * ld + M, device=dev).as_strided((K, M), (ld, 1))
+    a.copy_(torch.randn(K, M, device=dev, generator=g))
+    b = torch.randn(K, N, device=dev, generator=g)
+    out, rs = torch.empty(M, N, device=dev), torch.empty(M, device=dev)
+    gemm._run_f32(M, N, K, a, True, b, True, out, rowsum=rs)
+    assert _err(out, (a.double().T @ b.double()).float()) < 1e-5
+    assert _err(rs, a.double().sum(0).float()) < 1e-5
+
+
 @pytest.mark.parametrize("M,K,N", [(4096, 72, 8), (4099, 128, 264), (8200, 256, 1040), (16384, 64, 2048), (4096, 4096, 4096)])
 def test_scaled_input_grad_through_the_transpose(M, K, N):
     """``matmul_nn_scaled`` with the transposed copy (the persistent kernel's MUL_AUX epilogue, or its split-K
