@@ -56,12 +56,17 @@ def block_forward(x, cfg, params):
     """``(out, kept)`` of the block on ``x [B, T, D]``; ``params``: the twelve parameters of ``L.BLOCK_PARAMS``
     (biases None without)."""
     dev = x.device
-    kept = _bytes(_size("llattn_block_bytes", cfg, 0), dev)
-    n = _size("llattn_block_bytes", cfg, 1)
-    ws = _bytes(n, dev)
+    k, n = _size("llattn_block_bytes", cfg, 0), _size("llattn_block_bytes", cfg, 1)
+    if cfg.saved:
+        kept, ws = _bytes(k, dev), _bytes(n, dev)
+        at = _ptr(ws)
+    else:  # nothing outlives the call: one buffer
+        k = (k + 255) & ~255
+        kept = _bytes(k + n, dev)
+        at = kept.data_ptr() + k if n else None
     out = torch.empty_like(x)
     _call("llattn_block_fwd", _ref(cfg), _ref(L.LlattnBlockParams(*[_ptr(p) for p in params])), x.data_ptr(),
-          kept.data_ptr(), _ptr(ws), n, out.data_ptr(), L.stream_ptr(dev))
+          kept.data_ptr(), at, n, out.data_ptr(), L.stream_ptr(dev))
     return out, kept
 
 
