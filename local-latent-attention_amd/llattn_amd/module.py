@@ -194,6 +194,9 @@ class LocalLatentAttentionTriton(nn.Module):
             return None
         macro = self.latent_query_block_size > 1
         saved = torch.is_grad_enabled() and (x.requires_grad or any(p is not None and p.requires_grad for p in params))
+        # one call forms every gradient; with parts frozen ahead of what trains the single products stop early
+        if saved and not x.requires_grad and not all(p is None or p.requires_grad for p in params):
+            return None
         cfg = L.LlattnBlockCfg(lay.shape(dt), D, int(macro), int(biases[0]), int(saved),
                                int(bf16 and heads_layout_ok(lay, D, not macro)), int(ops._remote_heads(lay, dt)),
                                int(bf16 and grad_heads_ok(B * T, D, D, lay.Dh)),

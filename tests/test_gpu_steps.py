@@ -273,3 +273,33 @@ def test_forward_only_steps_refuse_tangents_and_vmap(entry):
             fn(fwad.make_dual(x, torch.ones_like(x)))
         with pytest.raises(RuntimeError):
             torch.func.vmap(fn)(x[None])
+
+
+def test_block_with_frozen_parts_stops_its_backward_early():
+    """Only ``out`` trains and the input needs no gradient: the backward forms that projection's gradients alone."""
+    from llattn_amd import LocalLatentAttentionTriton, steps
+    dev = require_cuda()
+    torch.manual_seed(6)
+    m = LocalLatentAttentionTriton(128, 4, 2, 64, 16, 64).to(dev)
+    x, dy = (torch.randn(2, 96, 128, device=dev).bfloat16() for _ in range(2))
+
+    def grads(frozen):
+        m.zero_grad(set_to_none=True)
+        for n, p in m.named_parameters():
+            p.requires_grad_(not frozen or n.startswith("out."))
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            y = m(x)
+        y.backward(dy)
+        return [m.out.weight.grad, m.out.bias.grad]
+
+    called, real = [], steps._call
+    steps._call = lambda name, *a: (called.append(name), real(name, *a))[1]
+    try:
+        ref = grads(False)
+        assert "llattn_block_bwd" in called
+        del called[:]
+        got = grads(True)
+    finally:
+        steps._call = real
+    assert not called
+    _close(got, ref, True)
