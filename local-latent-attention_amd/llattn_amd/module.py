@@ -192,6 +192,14 @@ class LocalLatentAttentionTriton(nn.Module):
                 return None
         if bf16 and (D % 8 or lay.Dh % 8 or lay.Ldh % 8):
             return None
+        # the native call takes pointers: another width of a replaced projection, or gates per head, run (or are
+        # refused) product by product
+        Ld = lay.Lh * lay.Ldh
+        shapes = ((3 * D, D), (3 * D,), (Ld, D), (Ld,), (2 * Ld, D), (2 * Ld,), (D, Ld), (D,), (D, D), (D,),
+                  (1, lay.Dh), (1, lay.Dh))
+        for p, s in zip(params, shapes):
+            if p is not None and p.shape != s:
+                return None
         macro = self.latent_query_block_size > 1
         saved = torch.is_grad_enabled() and (x.requires_grad or any(p is not None and p.requires_grad for p in params))
         # one call forms every gradient; with parts frozen ahead of what trains the single products stop early

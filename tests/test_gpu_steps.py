@@ -303,3 +303,68 @@ def test_block_with_frozen_parts_stops_its_backward_early():
         steps._call = real
     assert not called
     _close(got, ref, True)
+
+
+@pytest.mark.parametrize("bf16", [True, False])
+def test_block_with_other_projection_widths_and_gates(bf16):
+    """Replaced projections: a wider and a narrower ``out`` give the columns that their rows give one by one, another
+    width of ``rkv_proj`` is refused, and gates per head act on their own heads."""
+    from llattn_amd import LocalLatentAttentionTriton
+    dev = require_cuda()
+    torch.manual_seed(7)
+    D, H = 128, 4
+    m = LocalLatentAttentionTriton(D, H, 2, 64, 16, 64).to(dev)
+    x = torch.randn(2, 200, D, device=dev).to(torch.bfloat16 if bf16 else torch.float32)
+    w, b = torch.randn(2 * D, D, device=dev) * 0.1, torch.randn(2 * D, device=dev)
+
+    def out_linear(rows):
+        lin = torch.nn.Linear(D, len(w[rows])).to(dev)
+        with torch.no_grad():
+            lin.weight.copy_(w[rows])
+            lin.bias.copy_(b[rows])
+        return lin
+
+    def run(dy):
+        m.zero_grad(set_to_none=True)
+        with torch.autocast("cuda", dtype=torch.bfloat16, enabled=bf16):
+            y = m(x)
+        y.backward(dy.to(y.dtype))
+        return y.detach(), m.out.weight.grad, m.out.bias.grad
+
+    dy = torch.randn(2, 200, 2 * D, device=dev)
+    parts = []
+    for i in range(2):
+        m.out = out_linear(slice(i * D, (i + 1) * D))
+        parts.append(run(dy[..., i * D:(i + 1) * D]))
+    for rows in (slice(0, 2 * D), slice(0, D // 2)):
+        m.out = out_linear(rows)
+        got = run(dy[..., rows])
+        _close(got, [torch.cat([p[0] for p in parts], -1)[..., rows], torch.cat([p[1] for p in parts])[rows],
+                     torch.cat([p[2] for p in parts])[rows]], bf16)
+
+    m.out = torch.nn.Linear(D, D, bias=True).to(dev)
+    with torch.no_grad():
+        m.out.weight.copy_(torch.eye(D, device=dev))
+        m.out.bias.zero_()
+    gates = [torch.randn(1, D // H, device=dev) for _ in range(2)]
+
+    def heads(gate):
+        m.gate_local.weight, m.gate_remote.weight = torch.nn.Parameter(gate), torch.nn.Parameter(gate.flip(-1))
+        m.zero_grad(set_to_none=True)
+        with torch.autocast("cuda", dtype=torch.bfloat16, enabled=bf16):
+            y = m(x)
+        y.backward(dy[..., :D].to(y.dtype))
+        return y.detach().view(2, 200, H, D // H), m.gate_local.weight.grad
+
+    (y0, g0), (y1, g1) = heads(gates[0]), heads(gates[1])
+    y, g = heads(torch.cat([gates[0], gates[1], gates[1], gates[1]]))
+    _close([y], [torch.cat([y0[:, :, :1], y1[:, :, 1:]], 2)], bf16)
+    same, gs = heads(gates[1].expand(H, -1).contiguous())
+    _close([same, gs[1:]], [y1, g[1:]], bf16)
+    # the shared gate's gradient is the heads' sum: fp32 sums of B T H = 1600 terms in another order, 1600 * 2^-24 of
+    # their magnitudes, which the signed sum is taken to be a tenth of
+    assert float((gs.sum(0) - g1[0]).norm()) <= 1e-3 * float(g1.norm())
+
+    m.rkv_proj = torch.nn.Linear(D, 64).to(dev)
+    with pytest.raises(ValueError):
+        heads(gates[0])

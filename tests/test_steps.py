@@ -58,3 +58,25 @@ def test_step_sizes_and_refusals():
     assert lib.llattn_block_fwd(None, ref(p), buf, buf, None, 0, buf, None) == L.ERR_SHAPE
     f = L.LlattnFfnCfg(0, 64, 128, 64, 1)
     assert lib.llattn_ffn_bytes(ref(f), 0) == 0 and b"positive" in lib.llattn_last_error()
+
+
+@pytest.mark.parametrize("name,change", [
+    ("none", None), ("wider out", ("out", 128, 256)), ("narrower out", ("out", 128, 64)),
+    ("narrower rkv_proj", ("rkv_proj", 128, 64)), ("wider rq_proj", ("rq_proj", 128, 128)),
+    ("other r_out", ("r_out", 32, 128)), ("short qkv_proj", ("qkv_proj", 128, 128)), ("gates per head", None),
+    ("short bias", None)])
+def test_block_step_takes_only_the_layouts_shapes(name, change, monkeypatch):
+    """A parameter of another shape than the layout's never reaches the native call, which sees pointers alone."""
+    import torch
+    from llattn_amd import LocalLatentAttentionTriton, steps
+    taken = object()
+    monkeypatch.setattr(steps, "Block", type("Taken", (), {"apply": staticmethod(lambda *a: taken)}))
+    m = LocalLatentAttentionTriton(128, 4, 2, 64, 16, 64)
+    if change is not None:
+        setattr(m, change[0], torch.nn.Linear(*change[1:]))
+    elif name == "gates per head":
+        m.gate_local.weight = torch.nn.Parameter(torch.randn(4, 32))
+    elif name == "short bias":
+        m.out.bias = torch.nn.Parameter(torch.zeros(64))
+    x = torch.randn(2, 96, 128)
+    assert m._forward_native(x, m.layout(2, 96)) is (taken if name == "none" else None)
