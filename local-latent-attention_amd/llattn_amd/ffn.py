@@ -69,16 +69,23 @@ class _FeedForward(torch.autograd.Function):
                 None if db1 is None else db1.to(b1dt), dw2.to(w2dt), None if db2 is None else db2.to(b2dt))
 
 
+def _step_cfg(x: torch.Tensor, ps) -> L.LlattnFfnCfg | None:
+    """The native step's configuration for ``x`` and ``(w1, b1, w2, b2)``, or None where it does not take them: it
+    sees pointers alone, so every shape is compared here."""
+    dev, d = x.device, x.shape[-1]
+    rows = x.numel() // max(1, d)
+    d_ff, d_out = ps[0].shape[0], ps[2].shape[0]
+    if not 0 < rows < 1 << 31 or d % 8 or d_ff % 8 or d_out % 8 or not plain(x, dev, BF16):
+        return None
+    for p, s in zip(ps, ((d_ff, d), (d_ff,), (d_out, d_ff), (d_out,))):
+        if p is not None and (p.shape != s or not plain(p, dev)):
+            return None
+    saved = torch.is_grad_enabled() and (x.requires_grad or any(p is not None and p.requires_grad for p in ps))
+    return L.LlattnFfnCfg(rows, d, d_ff, d_out, int(saved))
+
+
 def feed_forward(x: torch.Tensor, w1: torch.nn.Linear, w2: torch.nn.Linear) -> torch.Tensor:
     """bf16 ``w2(gelu(w1(x)))`` on the GEMM kernels (GPU only; widths multiples of 8)."""
     ps = (w1.weight, w1.bias, w2.weight, w2.bias)
-    dev = x.device
-    rows = x.numel() // max(1, x.shape[-1])
-    d, d_ff, d_out = x.shape[-1], ps[0].shape[0], ps[2].shape[0]
-    if x.is_cuda and not ops.observed() and 0 < rows < 1 << 31 and d % 8 == 0 and d_ff % 8 == 0 and d_out % 8 == 0 \
-            and ps[0].shape[1] == d and ps[2].shape[1] == d_ff and plain(x, dev, BF16) \
-            and all(p is None or plain(p, dev) for p in ps):
-        saved = torch.is_grad_enabled() and (x.requires_grad or any(p is not None and p.requires_grad for p in ps))
-        cfg = L.LlattnFfnCfg(rows, d, d_ff, d_out, int(saved))
-        return Ffn.apply(x, cfg, *ps)
-    return _FeedForward.apply(x, *ps)
+    cfg = _step_cfg(x, ps) if x.is_cuda and not ops.observed() else None
+    return _FeedForward.apply(x, *ps) if cfg is None else Ffn.apply(x, cfg, *ps)

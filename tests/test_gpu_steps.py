@@ -368,3 +368,15 @@ def test_block_with_other_projection_widths_and_gates(bf16):
     m.rkv_proj = torch.nn.Linear(D, 64).to(dev)
     with pytest.raises(ValueError):
         heads(gates[0])
+
+
+def test_ffn_with_a_short_bias_is_refused():
+    from llattn_amd.ffn import feed_forward
+    dev = require_cuda()
+    w1, w2 = torch.nn.Linear(128, 256).to(dev), torch.nn.Linear(256, 128).to(dev)
+    x = torch.randn(2, 64, 128, device=dev).bfloat16()
+    for lin in (w1, w2):
+        full, lin.bias = lin.bias, torch.nn.Parameter(torch.zeros(64, device=dev))
+        with pytest.raises(ValueError), torch.autocast("cuda", dtype=torch.bfloat16):
+            feed_forward(x, w1, w2)
+        lin.bias = full

@@ -80,3 +80,17 @@ def test_block_step_takes_only_the_layouts_shapes(name, change, monkeypatch):
         m.out.bias = torch.nn.Parameter(torch.zeros(64))
     x = torch.randn(2, 96, 128)
     assert m._forward_native(x, m.layout(2, 96)) is (taken if name == "none" else None)
+
+
+@pytest.mark.parametrize("which,shape", [(None, None), (0, (256, 64)), (1, (128,)), (2, (128, 128)), (3, (64,)), (3, (1, 128))])
+def test_ffn_step_takes_only_matching_shapes(which, shape):
+    """A weight or a bias of another shape never reaches the native call."""
+    import torch
+    from llattn_amd import ffn
+    ps = [torch.zeros(s) for s in ((256, 128), (256,), (128, 256), (128,))]
+    if which is not None:
+        ps[which] = torch.zeros(shape)
+    cfg = ffn._step_cfg(torch.zeros(3, 7, 128, dtype=torch.bfloat16), ps)
+    assert (cfg is None) == (which is not None)
+    if cfg is not None:
+        assert [cfg.rows, cfg.d, cfg.d_ff, cfg.d_out, cfg.saved] == [21, 128, 256, 128, 0]
