@@ -68,6 +68,17 @@ def _aligned_f32(t: torch.Tensor) -> torch.Tensor:
     return t
 
 
+def _gates(gate_l: torch.Tensor, gate_r: torch.Tensor, H: int, Dh: int):
+    """The two gate vectors as the kernels read them, both shared by the heads ([Dh] or [1, Dh]) or both per head
+    ([H, Dh]).  ``gate_l`` decides which, so another size of either would be read past its end."""
+    per_head = gate_l.dim() == 2 and gate_l.shape[0] > 1
+    n = H * Dh if per_head else Dh
+    if gate_l.numel() != n or gate_r.numel() != n:
+        raise ValueError(f"the gates must both be [1, {Dh}] or both [{H}, {Dh}], got {tuple(gate_l.shape)} and "
+                         f"{tuple(gate_r.shape)}")
+    return _aligned_f32(gate_l), _aligned_f32(gate_r)
+
+
 def _contig(t: torch.Tensor) -> torch.Tensor:
     t = t.contiguous()
     if t.data_ptr() % 16:
@@ -335,7 +346,7 @@ class LLAttnCore(torch.autograd.Function):
         gkgv = _contig(gkgv.to(dt))
         if tuple(gkgv.shape) != (lay.B, lay.n_chunks, 2 * Ld):
             raise ValueError(f"gkgv must be [B, {lay.n_chunks}, {2 * Ld}], got {tuple(gkgv.shape)}")
-        gl, gr = _aligned_f32(gate_l), _aligned_f32(gate_r)
+        gl, gr = _gates(gate_l, gate_r, H, Dh)
         q, k, v, rqv = _qkv_views(lay, qkv, rq is None, heads)
         if rq is not None:
             rqv = L.view(rq, rq.stride(0), rq.stride(1), Ldh)
@@ -432,12 +443,12 @@ class LLAttnFunction(torch.autograd.Function):
                 local_block_size=256, q_block=0):
         L.require_gpu(Q, K, V, GQ, GK, GV)
         B, H, S, Dh = Q.shape
-        _, Lh, nq, Ldh = GQ.shape
+        Bq, Lh, nq, Ldh = GQ.shape
         n_chunks = GK.shape[2]
         if K.shape != Q.shape or V.shape != Q.shape:
             raise ValueError("Q, K, V must share the shape [B, Nh, S, Dh]")
-        if GK.shape != GV.shape or GK.shape[:2] != (B, Lh) or GK.shape[3] != Ldh:
-            raise ValueError("GK, GV must be [B, Lh, Nc, Ldh] matching GQ")
+        if Bq != B or GK.shape != GV.shape or GK.shape[:2] != (B, Lh) or GK.shape[3] != Ldh:
+            raise ValueError("GQ must be [B, Lh, Q, Ldh] and GK, GV [B, Lh, Nc, Ldh] matching it")
         if chunk_size <= 0 or n_chunks != -(-S // chunk_size):
             raise ValueError(f"GK has {n_chunks} latents but ceil(S / chunk_size) = {-(-S // max(chunk_size, 1))}")
         if window <= 0:
@@ -448,7 +459,7 @@ class LLAttnFunction(torch.autograd.Function):
         lay = L.Layout(B, S, H, Dh, Lh, Ldh, window, min(S, max(window, local_block_size)), chunk_size, n_chunks, qb, nq)
         dt, device = Q.dtype, Q.device
         Q, K, V, GQ, GK, GV = (_contig_last(t.to(dt)) for t in (Q, K, V, GQ, GK, GV))
-        gl, gr = _aligned_f32(gate_local_w), _aligned_f32(gate_remote_w)
+        gl, gr = _gates(gate_local_w, gate_remote_w, H, Dh)
         ctx.lay, ctx.has_rb = lay, r_out_b is not None
         ctx.like = (gate_local_w, gate_remote_w)
         ctx.r_b_dtype = None if r_out_b is None else r_out_b.dtype

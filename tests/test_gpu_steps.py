@@ -380,3 +380,15 @@ def test_ffn_with_a_short_bias_is_refused():
         with pytest.raises(ValueError), torch.autocast("cuda", dtype=torch.bfloat16):
             feed_forward(x, w1, w2)
         lin.bias = full
+
+
+def test_op_refuses_other_batches_and_mixed_gates():
+    from llattn_amd import LLAttnFunction
+    dev = require_cuda()
+    B, H, T, Dh, Lh, Ldh, chunk = 2, 4, 64, 32, 2, 32, 16
+    q = torch.randn(B, H, T, Dh, device=dev)
+    gq, gk = torch.randn(B, Lh, T, Ldh, device=dev), torch.randn(B, Lh, T // chunk, Ldh, device=dev)
+    shared, per_head, r_w = (torch.randn(*s, device=dev) for s in ((1, Dh), (H, Dh), (H * Dh, Lh * Ldh)))
+    for a in ((gq[:1], shared, shared), (gq, per_head, shared), (gq, shared, per_head)):
+        with pytest.raises(ValueError):
+            LLAttnFunction.apply(q, q, q, a[0], gk, gk, a[1], a[2], r_w, 16, chunk)

@@ -94,3 +94,18 @@ def test_ffn_step_takes_only_matching_shapes(which, shape):
     assert (cfg is None) == (which is not None)
     if cfg is not None:
         assert [cfg.rows, cfg.d, cfg.d_ff, cfg.d_out, cfg.saved] == [21, 128, 256, 128, 0]
+
+
+def test_gates_of_two_forms_are_refused():
+    """Both shared by the heads or both per head: the kernels read them by one rule."""
+    import torch
+    from llattn_amd import ops
+    H, Dh = 4, 32
+    shared, per_head = torch.randn(1, Dh), torch.randn(H, Dh)
+    for a, b in ((shared, shared), (shared[0], shared), (per_head, per_head), (shared.expand(H, Dh), per_head)):
+        gl, gr = ops._gates(a, b, H, Dh)
+        assert torch.equal(gl, a) and torch.equal(gr, b) and gl.is_contiguous() and gr.is_contiguous()
+    for a, b in ((per_head, shared), (shared, per_head), (per_head[:2], per_head[:2]), (shared[:, :16], shared),
+                 (per_head, per_head[:3])):
+        with pytest.raises(ValueError, match="gates"):
+            ops._gates(a, b, H, Dh)
