@@ -145,6 +145,9 @@ constexpr int wait_vm_lgkm0(int n) { return (n & 15) | ((n >> 4) << 14) | 0x0070
 
 // An offset past every operand extent (operands are below 4 GiB - 16 bytes): the lane reads zero.
 constexpr uint32_t kOffPastK = 0xFFFFFFF0u;
+// A lane's 32-bit offset within a step.  The rows of an m/n-contiguous stage that lie past K must read zero; with wide
+// strides (64 ld 2 >= 2^32 bytes) their offsets pass 32 bits, and cut short they would fall inside the operand again.
+__device__ __forceinline__ uint32_t step_off(int64_t bytes) { return (uint32_t)min(bytes, (int64_t)kOffPastK); }
 // A k-contiguous lane's offset for a step whose K tail starts `klim` elements in, its chunk starting at kc.
 __device__ __forceinline__ uint32_t kmask(uint32_t off, int kc, int klim) { return kc < klim ? off : kOffPastK; }
 
@@ -193,7 +196,7 @@ __device__ __forceinline__ void tile_offsets64(uint32_t (&off)[PDMA], int (&kc)[
     } else {
       const int k = 2 * bi + (lane >> 5);
       const int c = (lane & 31) ^ (2 * (k & 3));
-      off[i] = (uint32_t)(((int64_t)k * ld + min(o0 + 8 * c, omax - 8)) * 2);
+      off[i] = step_off(((int64_t)k * ld + min(o0 + 8 * c, omax - 8)) * 2);
       kc[i] = 0;
     }
   }

@@ -42,7 +42,7 @@ struct TileOp {
       } else {
         constexpr int PER = O / 8;
         const int q = bi * 64 + lane, k = q / PER, c = (q % PER) ^ (2 * (k & 3));
-        off[i] = (uint32_t)(((int64_t)k * ld + min(o0 + 8 * c, omax - 8)) * 2);
+        off[i] = step_off(((int64_t)k * ld + min(o0 + 8 * c, omax - 8)) * 2);
         kc[i] = 0;
       }
     }

@@ -636,6 +636,32 @@ def test_gemm_f32_wide_strides():
     assert _err(rs, a.double().sum(0).float()) < 1e-5
 
 
+def test_gemm_wide_strides():
+    """The same for the bf16 kernels (64 k rows per stage; 64 x 64 and 128 x 128 tiles, 256 x 256 ones with row sums of
+    their own or from a column of ones): NaN everywhere between the operands' rows reaches neither the products nor
+    the row sums.  fp32 sums of K = 24 terms: K * 2^-24 of the sum of magnitudes."""
+    from llattn_amd import gemm
+    dev = require_cuda()
+    K, ld = 24, 50_000_000
+    base = torch.full(((K - 1) * ld + 16384,), float("nan"), device=dev, dtype=torch.bfloat16)
+    g = torch.Generator(device=dev).manual_seed(1)
+    for M, N in ((512, 320), (3072, 1024), (3072, 2056), (4096, 4096), (4096, 4104)):
+        print("case: gemm wide strides", M, N, flush=True)
+        a, b = base.as_strided((K, M), (ld, 1)), base.as_strided((K, N), (ld, 1), 8192)
+        for t in (a, b):
+            t.copy_(torch.randn(t.shape, device=dev, generator=g))
+        A, B = a.double(), b.double()
+        rs = torch.empty(M, device=dev)
+        out = gemm.matmul_tn(a, b, rowsum=rs)
+        assert ((out - A.T @ B).abs() <= K * 2.0 ** -24 * (A.abs().T @ B.abs())).all()
+        assert ((rs - A.sum(0)).abs() <= K * 2.0 ** -24 * A.abs().sum(0)).all()
+        x = torch.randn(M, K, device=dev, generator=g).bfloat16()
+        X = x.double()
+        tol = (2.0 ** -8) * (X @ B).abs() + 2 * K * 2.0 ** -24 * (X.abs() @ B.abs())
+        assert ((gemm.matmul_nn(x, b) - X @ B).abs() <= tol).all()
+        base.as_strided((K, 16384), (ld, 1)).fill_(float("nan"))
+
+
 @pytest.mark.parametrize("M,K,N", [(4096, 72, 8), (4099, 128, 264), (8200, 256, 1040), (16384, 64, 2048), (4096, 4096, 4096)])
 def test_scaled_input_grad_through_the_transpose(M, K, N):
     """``matmul_nn_scaled`` with the transposed copy (the persistent kernel's MUL_AUX epilogue, or its split-K
