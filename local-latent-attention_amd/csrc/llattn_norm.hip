@@ -111,7 +111,7 @@ __global__ __launch_bounds__(256, NCH <= 6 ? 2 : 1) void rmsnorm_bwd_kernel(cons
                                                           int64_t lddx16) {
 #pragma clang fp contract(off)
   constexpr bool WL = RES && NCH <= 8;  // weights in LDS
-  extern __shared__ float red[];        // [4][D] dw of the four waves; with WL then the [D] weights
+  extern __shared__ float red[];        // [4][D] dw of the four waves; with WL then the weights, zero past the row
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int nq = D >> 2;
   const int nw = gridDim.x * 4, gw = blockIdx.x * 4 + wave;
@@ -125,8 +125,9 @@ __global__ __launch_bounds__(256, NCH <= 6 ? 2 : 1) void rmsnorm_bwd_kernel(cons
   float wv[WL ? 1 : NCH][4], dw[NCH][4];
   float* wl = red + 4 * D;
   if constexpr (WL) {
-    for (int c = threadIdx.x; c < nq; c += 256)
-      *reinterpret_cast<float4*>(wl + 4 * c) = *reinterpret_cast<const float4*>(w + 4 * c);
+    for (int c = threadIdx.x; c < 64 * NCH; c += 256)
+      *reinterpret_cast<float4*>(wl + 4 * c) = c < nq ? *reinterpret_cast<const float4*>(w + 4 * c)
+                                                      : make_float4(0.f, 0.f, 0.f, 0.f);
     __syncthreads();
   }
 #pragma unroll
@@ -144,8 +145,8 @@ __global__ __launch_bounds__(256, NCH <= 6 ? 2 : 1) void rmsnorm_bwd_kernel(cons
     for (int e = 0; e < 4; ++e) dw[i][e] = 0.f;
   }
   auto weights = [&](int i, float (&o)[4]) {
-    if constexpr (WL) {  // values past the row meet dy = 0
-      const float4 w4 = *reinterpret_cast<const float4*>(wl + 4 * min(lane + 64 * i, nq - 1));
+    if constexpr (WL) {
+      const float4 w4 = *reinterpret_cast<const float4*>(wl + 4 * (lane + 64 * i));
       o[0] = w4.x; o[1] = w4.y; o[2] = w4.z; o[3] = w4.w;
     } else {
 #pragma unroll
@@ -314,7 +315,7 @@ struct BwdArgs {
 template <typename XT, typename DYT, int NCH>
 void launch_bwd_n(const BwdArgs& a, hipStream_t st) {
   const dim3 grid(kBwdBlocks), block(256);
-  const size_t lds = (size_t)(a.dres && NCH <= 8 ? 5 : 4) * a.D * sizeof(float);
+  const size_t lds = (size_t)(4 * a.D + (a.dres && NCH <= 8 ? 256 * NCH : 0)) * sizeof(float);
   const DYT* dy = static_cast<const DYT*>(a.dy);
   const XT* x = static_cast<const XT*>(a.x);
   const XT* dres = static_cast<const XT*>(a.dres);

@@ -157,3 +157,24 @@ def test_residual_gradient_copy(M, D):
         y2 = rms_norm(s2, w2, 1e-6)
     y2.backward(dy)
     assert torch.equal(x.grad, s2.grad + ds) and torch.equal(w.grad, w2.grad)
+
+
+@pytest.mark.parametrize("D", [260, 1408, 1540, 2052])
+@pytest.mark.parametrize("last", [float("inf"), float("nan")])
+def test_residual_backward_with_a_non_finite_weight(D, last):
+    """A weight that is not finite at the end of the row acts where it stands: the residual instance gives what the
+    plain one gives, plus the residual path's gradient."""
+    from llattn_amd.norm import add_rms_norm, rms_norm
+    dev = require_cuda()
+    print("case: residual backward, non-finite weight", D, last, flush=True)
+    g = torch.Generator(device=dev).manual_seed(D)
+    x, res, ds, dy = (torch.randn(37, D, device=dev, generator=g) for _ in range(4))
+    w = torch.randn(D, device=dev, generator=g)
+    w[-1] = last
+    x.requires_grad_()
+    s, y = add_rms_norm(x, res, w.requires_grad_(), 1e-6)
+    torch.autograd.backward([s, y], [ds, dy])
+    s2, w2 = s.detach().requires_grad_(), w.detach().requires_grad_()
+    rms_norm(s2, w2, 1e-6).backward(dy)
+    for a, b in ((x.grad, s2.grad + ds), (w.grad, w2.grad)):
+        assert ((a == b) | (a.isnan() & b.isnan())).all()
