@@ -114,6 +114,8 @@ struct PoolList {
   int32_t segs[kCastPools], end[kCastPools];  // segments of all batches; workgroups up to and including this pooling's
 };
 
+constexpr int64_t kMaxGrid = ((int64_t(1) << 32) - 1) / 256;  // workgroups of 256 in a row: 32 bits of threads
+
 template <typename T>
 __global__ __launch_bounds__(256) void cast_pool_kernel(const CastArgs a, const PoolList l) {
   __shared__ union {
@@ -256,8 +258,20 @@ int32_t llattn::cast_and_pool(int32_t nseg, const float* const* src, void* const
       l.segs[q] = (int32_t)g.x;
       pool_blocks += (int64_t)g.x * g.y;
     }
-    if (blocks + pool_blocks > INT32_MAX) return fail(LLATTN_ERR_SHAPE, "llattn_pool_fwd: too many segments");
-    l.end[q] = (int32_t)pool_blocks;
+    l.end[q] = (int32_t)std::min<int64_t>(pool_blocks, INT32_MAX);
+  }
+  if (blocks + pool_blocks > kMaxGrid) {  // more workgroups than one row of them may hold: a pooling has two dimensions
+    if (blocks) {
+      const int32_t rc = llattn_cast_transposed(nseg, src, dst, n, dst_dtype, dst_t, ld_t, rows, stream);
+      if (rc) return rc;
+    }
+    for (int q = 0; q < n_pools; ++q) {
+      const PoolArgs& p = pools[q];
+      const int32_t rc = llattn_pool_fwd(p.x, p.x_sb, p.x_st, p.out, p.o_sb, p.o_sn, p.B, p.T, p.D, p.seg, p.n_seg,
+                                         p.divisor, pool_dtype, stream);
+      if (rc) return rc;
+    }
+    return LLATTN_OK;
   }
   const dim3 grid((unsigned)(blocks + pool_blocks));
   if (pool_dtype == LLATTN_F32)

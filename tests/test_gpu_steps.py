@@ -392,3 +392,19 @@ def test_op_refuses_other_batches_and_mixed_gates():
     for a in ((gq[:1], shared, shared), (gq, per_head, shared), (gq, shared, per_head)):
         with pytest.raises(ValueError):
             LLAttnFunction.apply(q, q, q, a[0], gk, gk, a[1], a[2], r_w, 16, chunk)
+
+
+def test_block_step_with_more_poolings_than_one_launch_holds():
+    """A million short sequences: the two poolings' workgroups pass 2^32 threads in a row, so that they are launched
+    apart from the weight casts.  Sequences do not see each other: the first ones equal a small batch's."""
+    from llattn_amd import LocalLatentAttentionTriton
+    dev = require_cuda()
+    torch.manual_seed(8)
+    B, T, D = 1 << 20, 12, 64
+    m = LocalLatentAttentionTriton(D, 2, 2, 16, T, 16, latent_query_block_size=2).to(dev)
+    assert B * (T + T // 2) * 256 >= 1 << 32
+    x = torch.randn(B, T, D, device=dev, dtype=torch.bfloat16)
+    with torch.no_grad(), torch.autocast("cuda", dtype=torch.bfloat16):
+        (a,), (b,) = _both(lambda: [m(x)], "llattn_block_fwd")
+        _close([a[:64], a[-64:]], [m(x[:64]), m(x[-64:])], True)
+        _close([a[B // 2:B // 2 + 64]], [b[B // 2:B // 2 + 64]], True)
