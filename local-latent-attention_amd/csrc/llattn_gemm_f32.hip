@@ -481,8 +481,8 @@ F32Plan plan_f32(int M, int N, int K, bool lds_ok) {
   };
   const int chunks = (K + FK - 1) / FK;
   for (int wk : {1, 2, 4, 8}) {
-    if (wk > 1 && chunks < 2 * wk) break;
     const int64_t tiles = (int64_t)((M + 31) / 32) * ((N + 31) / 32), per_simd = (tiles * wk + 1023) / 1024;
+    if (wk > 1 && (chunks < 2 * wk || tiles * wk >= (int64_t(1) << 32) / 64)) break;  // a grid holds 2^32 threads
     take(((chunks + wk - 1) / wk) * std::max(0.28, 0.45 * (double)per_simd) + 2.0, 0, wk);
   }
   if (!lds_ok) return best;

@@ -636,6 +636,21 @@ def test_gemm_f32_wide_strides():
     assert _err(rs, a.double().sum(0).float()) < 1e-5
 
 
+def test_gemm_f32_grid_of_many_register_tiles():
+    """Nine million 32 x 32 tiles (an odd stride keeps them off the LDS tiles): with eight waves each they would pass
+    the 2^32 threads that a grid holds, and the last tiles would stay unwritten."""
+    from llattn_amd import gemm
+    dev = require_cuda()
+    M, N, K = 8_700_000, 1025, 255
+    print("case: gemm f32 many tiles", flush=True)
+    g = torch.Generator(device=dev).manual_seed(1)
+    a, b = torch.randn(M, K, device=dev, generator=g), torch.randn(N, K, device=dev, generator=g)
+    out = gemm.linear_f32(a, b)
+    for r in (slice(0, 64), slice(M // 2, M // 2 + 64), slice(M - 64, M)):
+        ref, mag = a[r].double() @ b.double().T, a[r].double().abs() @ b.double().abs().T
+        assert ((out[r] - ref).abs() <= K * 2.0 ** -24 * mag).all()
+
+
 def test_gemm_wide_strides():
     """The same for the bf16 kernels (64 k rows per stage; 64 x 64 and 128 x 128 tiles, 256 x 256 ones with row sums of
     their own or from a column of ones): NaN everywhere between the operands' rows reaches neither the products nor
