@@ -6,7 +6,7 @@
 // A[k * lda + m] (a_trans = 1); B(n, k) is B[n * ldb + k] (b_trans = 0) or B[k * ldb + n] (b_trans = 1).
 //
 // What bounds it: the fp32 matrix rate (64 flop per clock and SIMD, a sixteenth of bf16's) where there are tiles
-// enough for every CU, and otherwise the latency of a chain of loads and the last round of tiles.  Two kernels:
+// enough for every CU, and otherwise the latency of a chain of loads and the last round of tiles.  Three kernels:
 //
 // * gemm_f32_lds_kernel, 64 x 64 or 64 x 32 output tiles: four waves (2 x 2) share the tile's operands through LDS,
 //   two stages of 32 k filled by direct-to-LDS loads (whole 128-byte lines), a stage's loads in flight during the
@@ -15,8 +15,11 @@
 // * gemm_f32_kernel, 32 x 32 tiles: a wave owns the tile for a range of k and loads its MFMA operands straight into
 //   registers (nothing is shared, so LDS would add a round trip); WK waves share a tile.  For products of a few
 //   tiles, and for operands that are not 16-byte aligned or whose edges cut a 16-byte piece.
+// * gemm_f32_staged_kernel, 64 x 64 tiles staged through registers and LDS: for many tiles of operands that the
+//   direct loads do not take (not 16-byte aligned, a 16-byte piece cut by an edge, 4 GiB and more); the register tiles
+//   load each element twice as often.
 //
-// In both, the k ranges of a tile are added through LDS in order: deterministic, no atomics, no workspace.
+// In the first two, the k ranges of a tile are added through LDS in order: deterministic, no atomics, no workspace.
 //
 // MFMA operands of a 16-k chunk for lane (r, g): rows MB r + i (i < MB) of the wave's 16 MB, k = 4 g + s of product
 // s (s < 4).  A k-contiguous operand supplies them as one 16-byte piece per i, an m/n-contiguous one as one piece of
@@ -462,6 +465,92 @@ __global__ __launch_bounds__(256 * KG) void gemm_f32_lds_kernel(const GemmF32Arg
   }
 }
 
+// ---- staged tiles: operands that the direct-to-LDS loads do not take ----------------------------------------
+constexpr int ST = 64, SP = ST + 4;  // tile, padded LDS row (floats)
+
+// 4 elements of a 64 x 16 operand tile into the k-major LDS tile s[k][o]: thread t takes row o = t / 4 and
+// k = 4 (t % 4) .. + 3 of k-contiguous storage, else k = t / 16 and o = 4 (t % 16) .. + 3.  Zero past the matrix.
+// (The layout as an argument: as a template parameter of the kernel it took 5% longer.)
+__device__ __forceinline__ void stage_tile(const float* __restrict__ p, int64_t ld, bool kc, int o0, int k0, int O, int K,
+                                           int t, float (*s)[SP]) {
+  float v[4];
+  if (kc) {
+    const int o = t >> 2, k = 4 * (t & 3), go = o0 + o, gk = k0 + k;
+    const float* q = p + (int64_t)go * ld + gk;
+    if (go < O && gk + 3 < K && ((uintptr_t)q & 15) == 0) {
+      const float4 x = *reinterpret_cast<const float4*>(q);
+      v[0] = x.x; v[1] = x.y; v[2] = x.z; v[3] = x.w;
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = (go < O && gk + e < K) ? q[e] : 0.f;
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) s[k + e][o] = v[e];
+  } else {
+    const int o = 4 * (t & 15), k = t >> 4, go = o0 + o, gk = k0 + k;
+    const float* q = p + (int64_t)gk * ld + go;
+    if (gk < K && go + 3 < O && ((uintptr_t)q & 15) == 0) {
+      const float4 x = *reinterpret_cast<const float4*>(q);
+      v[0] = x.x; v[1] = x.y; v[2] = x.z; v[3] = x.w;
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = (gk < K && go + e < O) ? q[e] : 0.f;
+    }
+    *reinterpret_cast<float4*>(&s[k][o]) = make_float4(v[0], v[1], v[2], v[3]);
+  }
+}
+
+// Four waves of 32 x 32 (2 x 2); a 16-k chunk is staged and multiplied at a time.
+__global__ __launch_bounds__(256) void gemm_f32_staged_kernel(const GemmF32Args a, int kc_a, int kc_b) {
+  __shared__ __align__(16) float As[FK][SP];
+  __shared__ __align__(16) float Bs[FK][SP];
+  const int tid = threadIdx.x, lane = tid & 63, r = lane & 15, g = lane >> 4;
+  const int wave = tid >> 6, wm = wave >> 1, wn = wave & 1;
+  const int m0 = (blockIdx.x / a.tiles_n) * ST, n0 = (blockIdx.x % a.tiles_n) * ST;
+  const bool rs = a.rowsum != nullptr && n0 == 0;  // workgroup-uniform
+  f32x4 acc[2][2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float rsum = 0.f;  // rs: thread t < 64 sums row m0 + t of A over k
+  for (int k0 = 0; k0 < a.K; k0 += FK) {
+    stage_tile(a.A, a.lda, kc_a, m0, k0, a.M, a.K, tid, As);
+    stage_tile(a.B, a.ldb, kc_b, n0, k0, a.N, a.K, tid, Bs);
+    __syncthreads();
+    if (rs && tid < ST) {
+#pragma unroll
+      for (int k = 0; k < FK; ++k) rsum += As[k][tid];
+    }
+#pragma unroll
+    for (int kk = 0; kk < FK; kk += 4) {  // lane (r, g) supplies A[m = r][k = g] and B[n = r][k = g]
+      float av[2], bv[2];
+#pragma unroll
+      for (int i = 0; i < 2; ++i) av[i] = As[kk + g][wm * 32 + 16 * i + r];
+#pragma unroll
+      for (int j = 0; j < 2; ++j) bv[j] = Bs[kk + g][wn * 32 + 16 * j + r];
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[i], bv[j], acc[i][j], 0, 0, 0);
+    }
+    __syncthreads();
+  }
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)  // lane (r, g) holds C[m = 16 i + 4 g + e][n = 16 j + r] of the wave's block
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int m = m0 + wm * 32 + 16 * i + 4 * g + e, n = n0 + wn * 32 + 16 * j + r;
+        if (m >= a.M || n >= a.N) continue;
+        float* c = a.C + (int64_t)m * a.ldc + n;
+        const float v = acc[i][j][e] + (a.bias ? a.bias[n] : 0.f);
+        *c = a.accumulate ? *c + v : v;
+      }
+  if (rs && tid < ST && m0 + tid < a.M) a.rowsum[m0 + tid] = rsum;
+}
+
 // Kernel, tile and k split: the least of a time model in us, fitted to a sweep of 20 products (16 x 64 x 256 to
 // 4096 x 3072 x 1024, each layout; within 15% of the best configuration on all of them).
 //   LDS tiles: rounds of tiles over 256 CUs at 256 flop per clock and CU and 2.25 GHz, times the share that a round
@@ -469,8 +558,13 @@ __global__ __launch_bounds__(256 * KG) void gemm_f32_lds_kernel(const GemmF32Arg
 //   64 x 64, 5 rounds: 117 us against 100), plus 3 us to fill and drain.
 //   32 x 32 register tiles: a chunk of 16 k takes 0.28 us of load latency with one chunk ahead, or 0.45 us per wave
 //   that shares the SIMD (twice the operand bytes of a 64 x 64 tile: 1000 x 4736 x 1408 takes 186 us), plus 2 us.
-struct F32Plan { int nb, k; };  // LDS tiles of 64 x 32 nb with k groups; nb = 0: register tiles with k waves
-F32Plan plan_f32(int M, int N, int K, bool lds_ok) {
+//   Operands that are not 16-byte aligned: the register tiles load by the element, 2.8 times as long.
+//   Staged tiles: 1.3 us per chunk of 16 k (1.7 by the element), or 0.40 (0.62) us per tile of a CU where that is more,
+//   plus 3 us.  Measured, register against staged tiles, in rows padded to 16 bytes: 1000 x 1409 x 1409 65 against
+//   120 us, 20000 x 1025 x 255 167 against 121, 1 200 000 x 1024 x 1024 (4.9 GB) 37.0 against 22.3 ms; by the element:
+//   333 x 1409 x 1407 62 against 147, 1000 x 1409 x 1409 177 against 155, 4096 x 3073 x 1025 1020 against 490.
+struct F32Plan { int nb, k; };  // LDS tiles of 64 x 32 nb with k groups (0: staged); nb = 0: register tiles with k waves
+F32Plan plan_f32(int M, int N, int K, bool lds_ok, bool aligned) {
   F32Plan best{0, 1};
   double best_t = 1e30;
   const auto take = [&](double t, int nb, int k) {
@@ -483,8 +577,11 @@ F32Plan plan_f32(int M, int N, int K, bool lds_ok) {
   for (int wk : {1, 2, 4, 8}) {
     const int64_t tiles = (int64_t)((M + 31) / 32) * ((N + 31) / 32), per_simd = (tiles * wk + 1023) / 1024;
     if (wk > 1 && (chunks < 2 * wk || tiles * wk >= (int64_t(1) << 32) / 64)) break;  // a grid holds 2^32 threads
-    take(((chunks + wk - 1) / wk) * std::max(0.28, 0.45 * (double)per_simd) + 2.0, 0, wk);
+    take(((chunks + wk - 1) / wk) * std::max(0.28, 0.45 * (double)per_simd) * (aligned ? 1.0 : 2.8) + 2.0, 0, wk);
   }
+  const int64_t staged = (int64_t)((M + ST - 1) / ST) * ((N + ST - 1) / ST);
+  if (!lds_ok && staged < (int64_t(1) << 24))
+    take(chunks * (aligned ? std::max(1.3, 0.40 * (double)staged / 256.0) : std::max(1.7, 0.62 * (double)staged / 256.0)) + 3.0, 2, 0);
   if (!lds_ok) return best;
   struct { int nb, kg; double one, more; } const opt[] = {{2, 1, 1.43, 1.18}, {2, 2, 1.28, 1.22}, {1, 2, 1.45, 1.31}, {1, 4, 1.35, 1.55}};
   for (const auto& o : opt) {
@@ -499,7 +596,8 @@ template <bool AK, bool BKM>
 void launch_f32(const GemmF32Args& a, const F32Plan& p, hipStream_t st) {
   const dim3 grid(a.tiles_m * a.tiles_n);
   if (p.nb == 2) {
-    if (p.k == 1) hipLaunchKernelGGL((gemm_f32_lds_kernel<AK, BKM, 2, 2, 1>), grid, dim3(256), 0, st, a);
+    if (p.k == 0) hipLaunchKernelGGL(gemm_f32_staged_kernel, grid, dim3(256), 0, st, a, AK, BKM);
+    else if (p.k == 1) hipLaunchKernelGGL((gemm_f32_lds_kernel<AK, BKM, 2, 2, 1>), grid, dim3(256), 0, st, a);
     else hipLaunchKernelGGL((gemm_f32_lds_kernel<AK, BKM, 2, 2, 2>), grid, dim3(512), 0, st, a);
   } else if (p.nb == 1) {
     if (p.k == 2) hipLaunchKernelGGL((gemm_f32_lds_kernel<AK, BKM, 2, 1, 2>), grid, dim3(512), 0, st, a);
@@ -537,7 +635,7 @@ extern "C" int32_t llattn_gemm_f32(const llattn_gemm_desc* d, void* stream) {
   const bool lds_ok = vec(d->A, d->lda) && vec(d->B, d->ldb) && (d->a_trans ? d->M : d->K) % 4 == 0 &&
                       (d->b_trans ? d->N : d->K) % 4 == 0 && span(d->a_trans, d->lda) && span(d->b_trans, d->ldb) &&
                       a_bytes <= (int64_t)kPast && b_bytes <= (int64_t)kPast;
-  const F32Plan plan = plan_f32(d->M, d->N, d->K, lds_ok);
+  const F32Plan plan = plan_f32(d->M, d->N, d->K, lds_ok, vec(d->A, d->lda) && vec(d->B, d->ldb));
   const int TM = plan.nb ? 64 : 32, TN = plan.nb ? 32 * plan.nb : 32;
   const int64_t tiles = (int64_t)((d->M + TM - 1) / TM) * ((d->N + TN - 1) / TN);
   if (tiles > 0x7fffffff) return fail(LLATTN_ERR_UNSUPPORTED, "llattn_gemm_f32: too many output tiles");

@@ -583,9 +583,10 @@ def test_gemm_f32_products(M, N, K):
     (1, 1, 1), (3, 5, 7), (31, 33, 17), (32, 32, 16), (65, 130, 257), (128, 1, 48),  # register tiles, every edge
     (40, 24, 600), (33, 2, 4100),                                # split over waves; pieces of 16 bytes cut by N = 2
     (1024, 800, 256), (260, 1028, 100), (2052, 516, 36),          # LDS tiles of 64 x 64, k tails of 4 in 32
-    (1000, 512, 1408), (1000, 1412, 520), (1400, 516, 1000)])     # two and four k groups, 64 x 32 tiles
+    (1000, 512, 1408), (1000, 1412, 520), (1400, 516, 1000),      # two and four k groups, 64 x 32 tiles
+    (2049, 1089, 70), (1500, 2000, 65)])                          # at odd strides: staged 64 x 64 tiles
 def test_gemm_f32_kernels_and_layouts(M, N, K):
-    """Both fp32 kernels and every operand layout (A and B k- or m/n-contiguous, aligned and at odd strides and
+    """The fp32 kernels and every operand layout (A and B k- or m/n-contiguous, aligned and at odd strides and
     offsets) against float64.  The K roundings of partial sums of unit products, each up to 2^-24 of a partial of
     size sqrt(k), add up to about 2^-24 K / 2, where the terms' absolute values sum to 0.64 K: an error of about
     2^-24 of that sum, which (unlike the result) cannot cancel.  Four times that is allowed."""
@@ -636,15 +637,15 @@ def test_gemm_f32_wide_strides():
     assert _err(rs, a.double().sum(0).float()) < 1e-5
 
 
-def test_gemm_f32_grid_of_many_register_tiles():
-    """Nine million 32 x 32 tiles (an odd stride keeps them off the LDS tiles): with eight waves each they would pass
-    the 2^32 threads that a grid holds, and the last tiles would stay unwritten."""
+def test_gemm_f32_grid_of_many_tiles():
+    """An output of nine million 32 x 32 tiles (the odd K in rows of 256 keeps it off the direct-to-LDS ones): with
+    eight waves each they would pass the 2^32 threads that a grid holds, and the last tiles would stay unwritten."""
     from llattn_amd import gemm
     dev = require_cuda()
     M, N, K = 8_700_000, 1025, 255
     print("case: gemm f32 many tiles", flush=True)
     g = torch.Generator(device=dev).manual_seed(1)
-    a, b = torch.randn(M, K, device=dev, generator=g), torch.randn(N, K, device=dev, generator=g)
+    a, b = torch.randn(M, K + 1, device=dev, generator=g)[:, :K], torch.randn(N, K + 1, device=dev, generator=g)[:, :K]
     out = gemm.linear_f32(a, b)
     for r in (slice(0, 64), slice(M // 2, M // 2 + 64), slice(M - 64, M)):
         ref, mag = a[r].double() @ b.double().T, a[r].double().abs() @ b.double().abs().T
