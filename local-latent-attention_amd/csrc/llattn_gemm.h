@@ -229,8 +229,9 @@ __device__ __forceinline__ bf16x8 frag64(const unsigned char* tile, int o16, int
 // Number of K splits of a product on 256 x 256 tiles (llattn_gemm.hip).
 int resolve_split(const llattn_gemm_desc* d);
 
-// Tile (32 mb x 32 nb) and k groups of a product on the smaller tiles; mb = 0: not taken (llattn_gemm_tile.hip).
-struct TilePlan { int mb, nb, kg; };
+// Tile (32 mb x 32 nb), k groups and k splits over workgroups of a product on the smaller tiles; mb = 0: not taken
+// (llattn_gemm_tile.hip).
+struct TilePlan { int mb, nb, kg, splits; };
 TilePlan tile_plan(const llattn_gemm_desc* d, double* us = nullptr);  // us: the time it expects
 void launch_tile(const GemmArgs& a, const TilePlan& p, bool a_kmaj, bool b_kmaj, int c_dtype, hipStream_t st);
 // Two independent products in one launch: x Wᵀ or dy W into bf16, and then dyᵀ x into fp32 or (after x Wᵀ) another x Wᵀ.

@@ -722,7 +722,8 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const GemmArgs a, in
     }
     *reinterpret_cast<float4*>(c) = make_float4(v[0], v[1], v[2], v[3]);
   } else {
-    uint16_t* c = static_cast<uint16_t*>(a.C) + (int64_t)row * a.ldc + col;
+    const int64_t off = a.ch.T ? (int64_t)heads_off(a.ch, (uint32_t)row, (uint32_t)col) : (int64_t)row * a.ldc + col;
+    uint16_t* c = static_cast<uint16_t*>(a.C) + off;
     if (a.accumulate) {
       float o[4];
       load4<uint16_t>(c, o);
@@ -747,6 +748,15 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const GemmArgs a, in
   }
 }
 
+void launch_reduce(const GemmArgs& a, int S, int c_dtype, hipStream_t st) {
+  const int64_t quads = (int64_t)a.M * (a.N / 4) + (a.rowsum ? a.M : 0);
+  const dim3 rg((unsigned)((quads + 255) / 256)), block(256);
+  if (c_dtype == LLATTN_F32)
+    hipLaunchKernelGGL((splitk_reduce_kernel<EPI_F32>), rg, block, 0, st, a, S);
+  else
+    hipLaunchKernelGGL((splitk_reduce_kernel<EPI_BF16>), rg, block, 0, st, a, S);
+}
+
 template <bool AK, bool BKM>
 void launch(const GemmArgs& a, int S, int c_dtype, hipStream_t st) {
   const dim3 grid(a.tiles_m * a.tiles_n * S), block(256);
@@ -755,12 +765,7 @@ void launch(const GemmArgs& a, int S, int c_dtype, hipStream_t st) {
   if (S > 1) {
     if (rs) hipLaunchKernelGGL((gemm_kernel<AK, BKM, EPI_PART, !AK && !BKM>), grid, block, 0, st, a);
     else hipLaunchKernelGGL((gemm_kernel<AK, BKM, EPI_PART>), grid, block, 0, st, a);
-    const int64_t quads = (int64_t)a.M * (a.N / 4) + (a.rowsum ? a.M : 0);
-    const dim3 rg((unsigned)((quads + 255) / 256));
-    if (c_dtype == LLATTN_F32)
-      hipLaunchKernelGGL((splitk_reduce_kernel<EPI_F32>), rg, block, 0, st, a, S);
-    else
-      hipLaunchKernelGGL((splitk_reduce_kernel<EPI_BF16>), rg, block, 0, st, a, S);
+    launch_reduce(a, S, c_dtype, st);
   } else if (c_dtype == LLATTN_F32) {
     if (rs) hipLaunchKernelGGL((gemm_kernel<AK, BKM, EPI_F32, !AK && !BKM>), grid, block, 0, st, a);
     else hipLaunchKernelGGL((gemm_kernel<AK, BKM, EPI_F32>), grid, block, 0, st, a);
@@ -816,8 +821,8 @@ using namespace llattn::gemm;
 
 extern "C" size_t llattn_gemm_workspace_size(const llattn_gemm_desc* d) {
   if (!d) return 0;
-  if (tile_plan(d).mb) return 0;
-  const int S = resolve_split(d);
+  const TilePlan tp = tile_plan(d);
+  const int S = tp.mb ? tp.splits : resolve_split(d);
   return S > 1 ? (size_t)S * d->M * (d->N + (d->a_rowsum ? 1 : 0)) * sizeof(float) : 0;
 }
 
@@ -953,6 +958,7 @@ extern "C" int32_t llattn_gemm(const llattn_gemm_desc* d, void* workspace, size_
   hipStream_t st = static_cast<hipStream_t>(stream);
   if (const TilePlan tp = tile_plan(d); tp.mb) {
     launch_tile(a, tp, !d->a_trans, !d->b_trans, d->c_dtype, st);
+    if (tp.splits > 1) launch_reduce(a, tp.splits, d->c_dtype, st);
     return check_launch("llattn_gemm");
   }
   // bf16 x Wᵀ (+ bias) (+ row addends) without K split or accumulation: the persistent kernel, one workgroup

@@ -1,8 +1,9 @@
 // bf16 GEMM on 128 x 128 and 64 x 64 output tiles for gfx950: the products whose 256 x 256 tiles (llattn_gemm.hip)
 // are too few for the chip, i.e. a few thousand rows and less -- prompts, micro-batches, the pooled latents.
 //
-// C[m][n] = sum_k A(m, k) B(n, k) with every operand layout, output and epilogue of llattn_gemm except partial sums:
-// the k split here is inside the workgroup.
+// C[m][n] = sum_k A(m, k) B(n, k) with every operand layout, output and epilogue of llattn_gemm; the k split is inside
+// the workgroup, and over workgroups (EPI_PART, the ordered reduction of llattn_gemm.hip behind it) only where a long
+// contraction has a few tiles.
 //
 // Four waves (2 x 2), each 16 MB x 16 NB, share a tile's operands through NST LDS stages of 64 k filled by
 // direct-to-LDS loads (as in llattn_gemm.hip), NST - 1 steps ahead; one barrier per step.  KG groups of four waves
@@ -70,9 +71,14 @@ struct TileOp {
 
 // C[row][col .. col + 4) = v with the epilogue of the 256 x 256 kernels: bias, accumulation or row addends in fp32,
 // one rounding, then the activation on the rounded value.
+// EPI_PART: the plain sums into the partials of split `split`.
 template <int EPI>
-__device__ __forceinline__ void finish4(const GemmArgs& a, int row, int col, f32x4 x) {
+__device__ __forceinline__ void finish4(const GemmArgs& a, int split, int row, int col, f32x4 x) {
   if (row >= a.M || col >= a.N) return;
+  if constexpr (EPI == EPI_PART) {
+    *reinterpret_cast<f32x4*>(a.part + ((int64_t)split * a.M + row) * a.N + col) = x;
+    return;
+  }
   float v[4] = {x[0], x[1], x[2], x[3]};
   if (a.bias) {
     const float4 b = *reinterpret_cast<const float4*>(a.bias + col);
@@ -114,7 +120,7 @@ __device__ __forceinline__ void finish4(const GemmArgs& a, int row, int col, f32
 
 constexpr int stage_bytes(int mb, int nb) { return 32 * (mb + nb) * 128; }
 
-// Workgroup `block` of `blocks` of a product; smem: KG NST stages.
+// Workgroup `block` of `blocks` of a product (EPI_PART: of a.n_split times its tiles); smem: KG NST stages.
 template <bool AK, bool BKM, int EPI, int MB, int NB, int KG, int NST>
 __device__ __forceinline__ void tile_product(const GemmArgs& a, int block, int blocks, unsigned char* smem) {
   constexpr int TM = 32 * MB, TN = 32 * NB;
@@ -126,13 +132,25 @@ __device__ __forceinline__ void tile_product(const GemmArgs& a, int block, int b
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), w4 = wave & 3, kg = wave >> 2;
   const int wm = w4 >> 1, wn = w4 & 1;
   // contiguous tile ranges per XCD, then groups of 8 tile rows
-  const int t = xcd_remap(block, blocks);
+  int t = xcd_remap(block, blocks);
+  int split = 0;
+  int64_t a_bytes = a.a_bytes, b_bytes = a.b_bytes;
+  int K = a.K, steps = a.k_pairs;
+  if constexpr (EPI == EPI_PART) {  // k steps [split steps, + steps): the product of a shorter K and operands that end there
+    const int tiles = a.tiles_m * a.tiles_n;
+    split = t / tiles;
+    t -= split * tiles;
+    steps = (a.k_pairs + a.n_split - 1) / a.n_split;
+    K = min(K, (split + 1) * steps * SK);
+    if (!AK) a_bytes = min(a_bytes, ((int64_t)(K - 1) * a.lda + a.M) * 2);
+    if (!BKM) b_bytes = min(b_bytes, ((int64_t)(K - 1) * a.ldb + a.N) * 2);
+  }
   constexpr int GM = 8;
   const int group = t / (GM * a.tiles_n), first_m = group * GM, gm = min(a.tiles_m - first_m, GM);
   const int m0 = (first_m + (t % (GM * a.tiles_n)) % gm) * TM, n0 = (t % (GM * a.tiles_n)) / gm * TN;
   const bool rs = a.rowsum != nullptr && n0 == 0 && wn == 0;  // wave-uniform
   // every k group runs the same number of steps; those past K read zeros
-  const int nk = (a.k_pairs + KG - 1) / KG, kbeg = kg * nk * SK;
+  const int nk = (steps + KG - 1) / KG, kbeg = (split * steps + kg * nk) * SK;
   unsigned char* sm = smem + kg * NST * STAGE;
 
   OpA oa;
@@ -140,8 +158,8 @@ __device__ __forceinline__ void tile_product(const GemmArgs& a, int block, int b
   oa.init(a.lda, m0, a.M, w4, lane);
   ob.init(a.ldb, n0, a.N, w4, lane);
   auto fetch = [&](int kt) {  // step kt (the last one again past the end: never read) into stage kt % NST
-    const int k0 = kbeg + min(kt, nk - 1) * SK, klim = a.K - k0;
-    const i32x4 ra = step_rsrc<AK>(a.A, a.lda, a.a_bytes, k0), rb = step_rsrc<BKM>(a.B, a.ldb, a.b_bytes, k0);
+    const int k0 = kbeg + min(kt, nk - 1) * SK, klim = K - k0;
+    const i32x4 ra = step_rsrc<AK>(a.A, a.lda, a_bytes, k0), rb = step_rsrc<BKM>(a.B, a.ldb, b_bytes, k0);
     unsigned char* st = sm + (kt % NST) * STAGE;
 #pragma unroll
     for (int i = 0; i < OpA::NB; ++i) oa.dma(ra, st, w4, i, klim);
@@ -216,7 +234,7 @@ __device__ __forceinline__ void tile_product(const GemmArgs& a, int block, int b
 #pragma unroll
     for (int i = 0; i < MB; ++i)
 #pragma unroll
-      for (int j = 0; j < NB; ++j) finish4<EPI>(a, rowb + 16 * i, colb + 16 * j, acc[i][j]);
+      for (int j = 0; j < NB; ++j) finish4<EPI>(a, split, rowb + 16 * i, colb + 16 * j, acc[i][j]);
   } else {
     f32x4* red = reinterpret_cast<f32x4*>(smem);  // [KG][4 waves][MB][NB][64]
 #pragma unroll
@@ -230,14 +248,15 @@ __device__ __forceinline__ void tile_product(const GemmArgs& a, int block, int b
       f32x4 v = red[(w4 * MB * NB + u) * 64 + lane];
 #pragma unroll
       for (int w = 1; w < KG; ++w) v += red[((4 * w + w4) * MB * NB + u) * 64 + lane];
-      finish4<EPI>(a, rowb + 16 * (u / NB), colb + 16 * (u % NB), v);
+      finish4<EPI>(a, split, rowb + 16 * (u / NB), colb + 16 * (u % NB), v);
     }
   }
   if (a.rowsum && n0 == 0 && threadIdx.x < TM && m0 + (int)threadIdx.x < a.M) {
     float v = rsl[threadIdx.x];
 #pragma unroll
     for (int w = 1; w < KG; ++w) v += rsl[w * TM + threadIdx.x];
-    a.rowsum[m0 + threadIdx.x] = v;
+    float* out = EPI == EPI_PART ? a.part + ((int64_t)a.n_split * a.N + split) * a.M : a.rowsum;
+    out[m0 + threadIdx.x] = v;
   }
 }
 
@@ -267,7 +286,9 @@ __global__ __launch_bounds__(256 * KG) void gemm_tile_pair_kernel(const GemmArgs
 template <bool AK, bool BKM, int EPI>
 void launch_epi(const GemmArgs& a, const TilePlan& p, hipStream_t st) {
   const dim3 grid(a.tiles_m * a.tiles_n);
-  if (p.mb == 4 && p.kg == 1) hipLaunchKernelGGL((gemm_tile_kernel<AK, BKM, EPI, 4, 4, 1, 2>), grid, dim3(256), 0, st, a);
+  if constexpr (EPI == EPI_PART) {
+    hipLaunchKernelGGL((gemm_tile_kernel<AK, BKM, EPI, 2, 2, 1, 2>), dim3(grid.x * a.n_split), dim3(256), 0, st, a);
+  } else if (p.mb == 4 && p.kg == 1) hipLaunchKernelGGL((gemm_tile_kernel<AK, BKM, EPI, 4, 4, 1, 2>), grid, dim3(256), 0, st, a);
   else if (p.mb == 4) hipLaunchKernelGGL((gemm_tile_kernel<AK, BKM, EPI, 4, 4, 2, 2>), grid, dim3(512), 0, st, a);
   else if (p.kg == 1) hipLaunchKernelGGL((gemm_tile_kernel<AK, BKM, EPI, 2, 2, 1, 2>), grid, dim3(256), 0, st, a);
   else if (grid.x > 256) hipLaunchKernelGGL((gemm_tile_kernel<AK, BKM, EPI, 2, 2, 2, 2>), grid, dim3(512), 0, st, a);
@@ -275,7 +296,8 @@ void launch_epi(const GemmArgs& a, const TilePlan& p, hipStream_t st) {
 }
 template <bool AK, bool BKM>
 void launch_dt(const GemmArgs& a, const TilePlan& p, int c_dtype, hipStream_t st) {
-  if (c_dtype == LLATTN_F32) launch_epi<AK, BKM, EPI_F32>(a, p, st);
+  if (a.n_split > 1) launch_epi<AK, BKM, EPI_PART>(a, p, st);
+  else if (c_dtype == LLATTN_F32) launch_epi<AK, BKM, EPI_F32>(a, p, st);
   else launch_epi<AK, BKM, EPI_BF16>(a, p, st);
 }
 
@@ -283,13 +305,13 @@ void launch_dt(const GemmArgs& a, const TilePlan& p, int c_dtype, hipStream_t st
 
 // Time in us of the 256 x 256 kernels with S k splits: 6 us to fill and drain, rounds of (tile, split) workgroups over 256 CUs, 1.2 us per
 // 64-k step of a workgroup alone up to 1.75 with every CU at work, and for S > 1 the ordered reduction with its fp32
-// partials written and read at 7 TB/s.  (1024 x 4736 x 1408, 76 tiles: 32 us; 8192 x 4096 x 1408, 512: 83;
+// partials written and read at 9 TB/s.  (1024 x 4736 x 1408, 76 tiles: 32 us; 8192 x 4096 x 1408, 512: 83;
 // 1536 x 1536 x 4011, 36 tiles in 7 splits: 41.)
 static double big_us(int64_t M, int64_t N, int steps, int S) {
   const int64_t n = ((M + BM - 1) / BM) * ((N + BN - 1) / BN) * S;
   const double last = (double)(n % 256) / 256.0;
   const double per = (double)(n / 256) * 1.75 + (n % 256 ? 1.2 + 0.55 * last * last : 0.0);
-  return 6.0 + (double)((steps + S - 1) / S) * per + (S > 1 ? 7.0 + 8.0 * S * (double)M * (double)N / 7e6 : 0.0);
+  return 6.0 + (double)((steps + S - 1) / S) * per + (S > 1 ? 7.0 + 8.0 * S * (double)M * (double)N / 9e6 : 0.0);
 }
 
 // The tiles that a product takes, fitted to the times of 38 products (16 x 1024 x 1408 to 3000 x 4736 x 1408; all
@@ -300,6 +322,10 @@ static double big_us(int64_t M, int64_t N, int steps, int S) {
 //   64 x 64, one k group: rounds of four tiles per CU, 0.85 us per step (0.5 for a last round of one, 0.52 of two, 0.68
 //   of three), 4.5 us once;  two k groups: 0.44 us per step of a group for up to one tile per CU, 0.68 for up to two.
 //   (Four k groups: no faster.)
+//   64 x 64 split over workgroups: 5.2 us and 0.07 per split with the reduction's launch, the same steps (from memory 2.8 TB/s at most, in
+//   pieces of 128 bytes a k row), partials written and read at 4.2 TB/s.
+//   (128 x 128 x 4096: 8.2 us in 16 splits against 16 in two k groups and 20 on 256 x 256 tiles in 16 splits;
+//   512 x 512 x 4096 15.3 in 8 splits against 19; 333 x 1408 x 4096, 132 tiles, 20 in 4 splits against 18.)
 // Only where 256 x 256 tiles leave CUs idle (below 224 of them): from there on
 // those tiles' half as large operand traffic wins (4011 x 4992 x 1536: 69 us against 81).  Neither the epilogue nor
 // the layouts enter, so a product has the same bits whichever way it is stored.
@@ -309,17 +335,17 @@ static double big_us(int64_t M, int64_t N, int steps, int S) {
 //   333 x 4736 x 1408: 30 -> 12.5;  1024 x 4096 x 1408: 30 -> 17;  1536 x 384 x 4011: 52 -> 18;  32768 x 64 x 1024:
 //   24 -> 13.
 TilePlan tile_plan(const llattn_gemm_desc* d, double* us) {
-  const TilePlan none{0, 0, 0};
+  const TilePlan none{0, 0, 0, 1};
   if (d->split_k > 0 || d->M <= 0 || d->N <= 0 || d->K <= 0) return none;
   const int64_t M = d->M, N = d->N;
   if (((M + BM - 1) / BM) * ((N + BN - 1) / BN) >= 224) return none;
   const int steps = (d->K + SK - 1) / SK;
   TilePlan best = none;
   double best_t = 0.97 * big_us(M, N, steps, resolve_split(d));
-  const auto take = [&](double t, int mb, int kg) {
+  const auto take = [&](double t, int mb, int kg, int S = 1) {
     if (t < best_t) {
       best_t = t;
-      best = TilePlan{mb, mb, kg};
+      best = TilePlan{mb, mb, kg, S};
     }
   };
   const int64_t t128 = ((M + 127) / 128) * ((N + 127) / 128), t64 = ((M + 63) / 64) * ((N + 63) / 64);
@@ -331,6 +357,15 @@ TilePlan tile_plan(const llattn_gemm_desc* d, double* us) {
   take(4.5 + steps * ((double)(t64 / 1024) * 0.85 + last[r64]), 2, 1);
   if (steps >= 4 && t64 <= 256) take(3.8 + split(2) * 0.44, 2, 2);
   if (steps >= 4 && t64 > 256 && t64 <= 512) take(5.6 + split(2) * 0.68, 2, 2);
+  // a few tiles of a long contraction (from K = 2048 on; below, it gains a microsecond at most): 64 x 64 tiles over S
+  // ranges of at least two steps, their partials reduced in order
+  const double stream = 2.0 * (double)(M + N) * (double)d->K / 2.8e6;
+  for (int S = 2; S <= 32 && steps >= 32; S *= 2) {
+    const int64_t per = (steps + S - 1) / S, parts = (steps + per - 1) / per, n = t64 * parts;  // no range is empty
+    if (per < 2 || n > 2048) break;
+    take(5.2 + 0.07 * (double)parts + std::max(stream, (double)per * ((double)(n / 1024) * 0.85 + last[(n % 1024 + 255) / 256])) +
+             8.0 * (double)parts * (double)M * (double)N / 4.2e6, 2, 1, (int)parts);
+  }
   if (us) *us = best_t;
   return best;
 }
@@ -339,6 +374,7 @@ void launch_tile(const GemmArgs& a0, const TilePlan& p, bool a_kmaj, bool b_kmaj
   GemmArgs a = a0;
   a.tiles_m = (a.M + 32 * p.mb - 1) / (32 * p.mb);
   a.tiles_n = (a.N + 32 * p.nb - 1) / (32 * p.nb);
+  a.n_split = p.splits;
   if (a_kmaj && b_kmaj) launch_dt<true, true>(a, p, c_dtype, st);
   else if (a_kmaj) launch_dt<true, false>(a, p, c_dtype, st);
   else if (!b_kmaj) launch_dt<false, false>(a, p, c_dtype, st);
@@ -379,7 +415,7 @@ void launch_pair_as(const GemmArgs& a0, const GemmArgs& a1, bool nt0, bool nt1, 
 // 4 x 8192 tokens with 64-token query blocks 5 + 10 us in two, 11.5 in one.  The gradients of a few thousand tokens'
 // large projections stay apart: the weight gradient's long contraction wants its own k split.)
 TilePlan pair_plan(const llattn_gemm_desc* d0, const llattn_gemm_desc* d1) {
-  const TilePlan none{0, 0, 0};
+  const TilePlan none{0, 0, 0, 1};
   for (const llattn_gemm_desc* d : {d0, d1})
     if (d->split_k > 0 || d->M <= 0 || d->N <= 0 || d->K <= 0) return none;
   const bool bf0 = d0->c_dtype == LLATTN_BF16 && !d0->a_trans, nt1 = d1->c_dtype == LLATTN_BF16 && !d1->a_trans && !d1->b_trans;
@@ -397,7 +433,7 @@ TilePlan pair_plan(const llattn_gemm_desc* d0, const llattn_gemm_desc* d1) {
     const double t = fill + std::max((t0 * s0 + t1 * s1) * rate, step * most) + 0.18 * step * least;
     if (t < best_t) {
       best_t = t;
-      best = TilePlan{mb, mb, kg};
+      best = TilePlan{mb, mb, kg, 1};
     }
   };
   take(4, 1, 8.5, 1.27 / 512.0, [](double n) { return n <= 256 ? 0.75 : 1.02; });
