@@ -25,8 +25,9 @@ int32_t llattn_rmsnorm_bwd_residual(const void* dy, int32_t dy_dtype, int64_t ld
  * host language between them.  The caller passes memory: `kept` holds what the
  * forward leaves for the backward (llattn_*_bytes, which = 0; without a
  * backward it is the forward's scratch), `ws` the scratch of one call
- * (which = 1: forward, 2: backward; may be NULL where that is 0 bytes).
- * Everything is 16-byte aligned. */
+ * (which = 1: forward, 2: backward, 3: backward without dx; may be NULL where
+ * that is 0 bytes).  Outputs also serve as scratch before they are written:
+ * out and dx overlap no input.  Everything is 16-byte aligned. */
 
 /* The block: x [B][T][d_model] in shape.dtype, fp32 parameters.  `saved`: a
  * backward will follow.  The layout flags choose split-head storage

@@ -26,24 +26,25 @@ namespace {
 
 constexpr size_t up(size_t n) { return (n + 255) & ~size_t(255); }
 
-// Hands out 256-byte aligned pieces of a buffer; base null: only counts.
+// Hands out 256-byte aligned pieces of a buffer as a stack; base null: only counts.  What was given back is handed out
+// again: the launches of a step run in order on one stream.
 struct Arena {
   char* base;
-  size_t used = 0;
+  size_t used = 0, peak = 0;
   template <typename T = void>
   T* take(size_t bytes) {
     char* p = base ? base + used : nullptr;
     used += up(bytes);
+    peak = std::max(peak, used);
     return reinterpret_cast<T*>(p);
   }
 };
 
-// Runs launches until one fails (its status is `rc`); dry: nothing runs, `need` is the largest GEMM workspace.
+// Runs launches until one fails (its status is `rc`), with scratch from `a`; dry: nothing runs, a.peak is what it takes.
 struct Exec {
   void* stream = nullptr;
   bool dry = true;
-  void* gemm_ws = nullptr;
-  size_t gemm_bytes = 0, need = 0;
+  Arena a{nullptr};
   int32_t rc = LLATTN_OK;
 
   template <typename F>
@@ -56,9 +57,10 @@ struct Exec {
       run([&] { return llattn_gemm_f32(&d, stream); });
       return;
     }
-    const size_t n = llattn_gemm_workspace_size(&d);
-    need = std::max(need, n);
-    run([&] { return llattn_gemm(&d, n ? gemm_ws : nullptr, n ? gemm_bytes : 0, stream); });
+    const size_t n = llattn_gemm_workspace_size(&d), mark = a.used;
+    void* ws = n ? a.take(n) : nullptr;
+    run([&] { return llattn_gemm(&d, ws, n, stream); });
+    a.used = mark;
   }
   // two products that do not depend on each other
   void gemm(const llattn_gemm_desc& d0, const llattn_gemm_desc& d1, bool f32) {
@@ -67,9 +69,10 @@ struct Exec {
       gemm(d1, true);
       return;
     }
-    const size_t n = llattn::gemm::pair_workspace(&d0, &d1);
-    need = std::max(need, n);
-    run([&] { return llattn::gemm::run_pair(&d0, &d1, n ? gemm_ws : nullptr, n ? gemm_bytes : 0, stream); });
+    const size_t n = llattn::gemm::pair_workspace(&d0, &d1), mark = a.used;
+    void* ws = n ? a.take(n) : nullptr;
+    run([&] { return llattn::gemm::run_pair(&d0, &d1, ws, n, stream); });
+    a.used = mark;
   }
   // y [M][N] = x [M][K] w [N][K]ᵀ (+ b)
   static llattn_gemm_desc linear(int dt, int M, int N, int K, const void* x, const void* w, const float* b, void* y,
@@ -186,14 +189,15 @@ struct Dims {
   bool macro() const { return nq != T; }
 };
 
-Core core_layout(const llattn_block_cfg& c, Arena& a) {
+// lat_at, R_at: where these lie if not in the arena
+Core core_layout(const llattn_block_cfg& c, Arena& a, void* lat_at = nullptr, void* R_at = nullptr) {
   const Dims d(c.shape);
   const bool bf = d.dt == LLATTN_BF16;
   Core k{};
   if (bf) k.r_w = a.take(d.D * d.Ld * 2);
   if (bf && c.saved && persistent_grad(d.Mq, d.D, d.Ld)) k.r_wt = a.take(d.D * d.Ld * 2);
-  k.lat = a.take(d.Mq * d.Ld * d.es);
-  k.R = a.take(d.Mq * d.D * d.es);
+  k.lat = lat_at ? lat_at : a.take(d.Mq * d.Ld * d.es);
+  k.R = R_at ? R_at : a.take(d.Mq * d.D * d.es);
   if (c.saved) {
     k.lse_lat = a.take<float>((size_t)d.B * d.Lh * d.nq * 4);
     k.ol = a.take(d.M * d.D * d.es);
@@ -225,12 +229,13 @@ void core_fwd(Exec& e, const llattn_block_cfg& c, const llattn_core_views& in, c
   });
 }
 
-void core_bwd(Exec& e, Arena& a, const llattn_block_cfg& c, const llattn_core_views& in, const float* gl,
+void core_bwd(Exec& e, const llattn_block_cfg& c, const llattn_core_views& in, const float* gl,
               const float* gr, const void* r_w, const Core& k, const llattn_tensor& dy, const llattn_core_views& out,
               float* dgl, float* dgr, float* dr_w, float* dr_b) {
   const Dims d(c.shape);
+  Arena& a = e.a;
   void* drem = a.take(d.M * d.D * d.es);
-  const size_t n_local = llattn_workspace_size(&c.shape, LLATTN_WS_LOCAL_BWD);
+  const size_t mark = a.used, n_local = llattn_workspace_size(&c.shape, LLATTN_WS_LOCAL_BWD);
   void* ws_local = a.take(n_local);
   const llattn_tensor R = remote_view(c, d, k.R), dr = view(drem, 0, d.es, d.T * d.D, d.D, d.Dh);
   const llattn_tensor ol = view(k.ol, 0, d.es, (int64_t)d.H * d.T * d.Dh, d.Dh, (int64_t)d.T * d.Dh);
@@ -238,6 +243,7 @@ void core_bwd(Exec& e, Arena& a, const llattn_block_cfg& c, const llattn_core_vi
     return llattn_local_gate_bwd(&c.shape, &in.q, &in.k, &in.v, &R, gl, gr, &ol, k.lse, k.w, &dy, &out.q, &out.k,
                                  &out.v, &dr, dgl, dgr, dr_b, ws_local, n_local, e.stream);
   });
+  a.used = mark;
   void* dR = drem;
   if (c.shape.q_block > 1 || d.macro()) {
     dR = a.take(d.Mq * d.D * d.es);
@@ -271,14 +277,27 @@ bool twin_pools(const llattn_block_cfg& c) {
   return c.macro && s.q_block == s.chunk && s.n_q == s.n_chunks && (int64_t)s.n_q * s.q_block <= s.T;
 }
 
-Block block_layout(const llattn_block_cfg& c, Arena& a) {
+// out: the output's buffer.  With no backward to follow it holds R until the product that writes it (R has no more
+// rows than the output), and y lies over the projection's weights and the latent output, which nothing reads any more
+// when the local kernel writes it.
+Block block_layout(const llattn_block_cfg& c, Arena& a, void* out) {
   const Dims d(c.shape);
   const int64_t Dm = c.d_model, width = 3 * Dm + (c.macro ? 0 : d.Ld);
   const bool bf = d.dt == LLATTN_BF16;
   Block k{};
+  const size_t mark = a.used;
   if (bf || !c.macro) {
     k.w_qkv = a.take(width * Dm * d.es);
     if (c.has_bias) k.b_qkv = a.take<float>(width * 4);
+  }
+  void* lat = nullptr;
+  if (!c.saved) {
+    lat = a.take(d.Mq * d.Ld * d.es);
+    if (!lat) lat = &a;  // a dry run's counts as placed
+    const size_t end = a.used;
+    a.used = mark;
+    k.y = a.take(d.M * d.D * d.es);
+    a.used = std::max(a.used, end);
   }
   if (bf) {
     if (c.saved && persistent_grad(d.M, width, Dm)) k.w_qkvt = a.take(width * Dm * 2);
@@ -294,8 +313,8 @@ Block block_layout(const llattn_block_cfg& c, Arena& a) {
     k.rq = a.take(d.Mq * d.Ld * d.es);
   }
   k.gkgv = a.take((int64_t)d.B * d.nc * 2 * d.Ld * d.es);
-  k.y = a.take(d.M * d.D * d.es);
-  k.core = core_layout(c, a);
+  if (c.saved) k.y = a.take(d.M * d.D * d.es);
+  k.core = core_layout(c, a, lat, c.saved ? nullptr : out);
   return k;
 }
 
@@ -365,7 +384,7 @@ void block_fwd(Exec& e, const llattn_block_cfg& c, const llattn_block_params& p,
   e.gemm(e.linear(dt, (int)d.M, (int)Dm, (int)d.D, k.y, w.out, p.b_out, out), f32);
 }
 
-void block_bwd(Exec& e, Arena& a, const llattn_block_cfg& c, const llattn_block_params& p, const void* x,
+void block_bwd(Exec& e, const llattn_block_cfg& c, const llattn_block_params& p, const void* x,
                const Block& k, const void* dy, void* dx, const llattn_block_grads& g) {
   const Dims d(c.shape);
   const llattn_shape& s = c.shape;
@@ -373,25 +392,29 @@ void block_bwd(Exec& e, Arena& a, const llattn_block_cfg& c, const llattn_block_
   const int dt = d.dt;
   const bool bf = dt == LLATTN_BF16;
   const Weights w = block_weights(c, p, k);
-  void* dyc = a.take(d.M * d.D * d.es);
-  const llattn_heads_layout yh{d.T, d.Dh, d.H, 0};
-  e.gemm(e.input_grad(dt, (int)d.M, (int)Dm, (int)d.D, dy, w.out, k.w_outt, dyc, c.dy_heads ? &yh : nullptr),
-         e.weight_grad(dt, (int)d.M, (int)Dm, (int)d.D, dy, k.y, g.w_out, g.b_out), !bf);
+  Arena& a = e.a;
   void* dqkv = a.take(d.M * width * d.es);
   void* drq = c.macro ? a.take(d.Mq * d.Ld * d.es) : nullptr;
   void* dgkgv = a.take((int64_t)d.B * d.nc * 2 * d.Ld * d.es);
+  const size_t mark = a.used;
+  // the core's output gradient lies in dx, which the last product writes, long after its last reader
+  void* dyc = dx ? dx : a.take(d.M * d.D * d.es);
+  const llattn_heads_layout yh{d.T, d.Dh, d.H, 0};
+  e.gemm(e.input_grad(dt, (int)d.M, (int)Dm, (int)d.D, dy, w.out, k.w_outt, dyc, c.dy_heads ? &yh : nullptr),
+         e.weight_grad(dt, (int)d.M, (int)Dm, (int)d.D, dy, k.y, g.w_out, g.b_out), !bf);
   // the gradient in plain rows whatever the storage of qkv: the projection's backward reads it row-major
   const llattn_core_views out = block_views(c, dqkv, false, drq, dgkgv);
   const llattn_tensor dyv = c.dy_heads ? view(dyc, 0, d.es, (int64_t)d.T * d.D, d.Dh, (int64_t)d.T * d.Dh)
                                        : view(dyc, 0, d.es, d.T * d.D, d.D, d.Dh);
-  core_bwd(e, a, c, block_views(c, k.qkvr, c.heads, k.rq, k.gkgv), p.gate_l, p.gate_r, w.r, k.core, dyv, out, g.gate_l,
+  core_bwd(e, c, block_views(c, k.qkvr, c.heads, k.rq, k.gkgv), p.gate_l, p.gate_r, w.r, k.core, dyv, out, g.gate_l,
            g.gate_r, g.w_r, g.b_r);
+  a.used = mark;
   const int Mc = d.B * d.nc;
   void* dpooled = dx ? a.take((int64_t)Mc * Dm * d.es) : nullptr;
   // an input gradient (where it is wanted) with the weight gradient of the same dy
   auto grads = [&](const llattn_gemm_desc& di, const llattn_gemm_desc& dw) {
     if (dx) e.gemm(di, dw, !bf);
-    if (!dx || e.dry) e.gemm(dw, !bf);  // the scratch is sized for both
+    else e.gemm(dw, !bf);
   };
   grads(e.input_grad(dt, Mc, (int)(2 * d.Ld), (int)Dm, dgkgv, w.rkv, nullptr, dpooled),
         e.weight_grad(dt, Mc, (int)(2 * d.Ld), (int)Dm, dgkgv, k.pooled, g.w_rkv, g.b_rkv));
@@ -429,31 +452,28 @@ int32_t check_cfg(const char* what, const llattn_block_cfg* c, bool block) {
   return LLATTN_OK;
 }
 
-// The scratch of a call: the GEMM workspace, then the arena.
-int32_t begin(Exec& e, Arena& a, const char* what, size_t need, size_t gemm, void* ws, size_t ws_bytes, void* stream) {
+int32_t begin(Exec& e, const char* what, size_t need, void* ws, size_t ws_bytes, void* stream) {
   if (need && (!ws || ws_bytes < need || !aligned16(ws)))
     return fail(LLATTN_ERR_WORKSPACE, "%s needs %zu scratch bytes (got %zu)", what, need, ws_bytes);
   e.stream = stream;
   e.dry = false;
-  e.gemm_ws = ws;
-  e.gemm_bytes = gemm;
-  a = Arena{static_cast<char*>(ws) + up(gemm)};
+  e.a = Arena{static_cast<char*>(ws)};
   return LLATTN_OK;
 }
 
-struct Need { size_t gemm, arena, total; };
 template <typename F>
-Need measure(F f) {
+size_t measure(F f) {
   Exec e;
-  Arena a{nullptr};
-  f(e, a);
-  return Need{e.need, a.used, e.need || a.used ? up(e.need) + a.used : 0};
+  f(e);
+  return e.a.peak;
 }
 
-Need block_need(const llattn_block_cfg& c, bool bwd) {
-  return measure([&](Exec& e, Arena& a) {
+enum Pass { FWD = 1, BWD = 2, BWD_NO_DX = 3 };  // what a size is asked for (llattn_*_bytes)
+
+size_t block_need(const llattn_block_cfg& c, int pass) {
+  return measure([&](Exec& e) {
     Arena none{nullptr};
-    const Block k = block_layout(c, none);
+    const Block k = block_layout(c, none, nullptr);
     // a dry run reads no pointer, but the routes follow from which transposed copies exist
     Block with = k;
     static char there;
@@ -464,18 +484,18 @@ Need block_need(const llattn_block_cfg& c, bool bwd) {
     if (bf && c.saved && persistent_grad(d.M, c.d_model, c.d_model)) with.w_outt = &there;
     if (bf && c.saved && persistent_grad(d.Mq, d.D, d.Ld)) with.core.r_wt = &there;
     const llattn_block_params p{};
-    if (!bwd) {
+    if (pass == FWD) {
       block_fwd(e, c, p, nullptr, with, nullptr);
     } else {
       llattn_block_grads g{};
       if (c.has_bias) g.b_qkv = g.b_rq = g.b_rkv = g.b_out = reinterpret_cast<float*>(&there);
-      block_bwd(e, a, c, p, nullptr, with, nullptr, &there, g);
+      block_bwd(e, c, p, nullptr, with, nullptr, pass == BWD ? &there : nullptr, g);
     }
   });
 }
 
-Need core_need(const llattn_block_cfg& c, bool bwd) {
-  return measure([&](Exec& e, Arena& a) {
+size_t core_need(const llattn_block_cfg& c, int pass) {
+  return measure([&](Exec& e) {
     Arena none{nullptr};
     Core k = core_layout(c, none);
     static char there;
@@ -483,8 +503,8 @@ Need core_need(const llattn_block_cfg& c, bool bwd) {
     if (d.dt == LLATTN_BF16 && c.saved && persistent_grad(d.Mq, d.D, d.Ld)) k.r_wt = &there;
     const llattn_core_views v{};
     const llattn_tensor t{};
-    if (!bwd) core_fwd(e, c, v, nullptr, nullptr, nullptr, nullptr, k, t);
-    else core_bwd(e, a, c, v, nullptr, nullptr, nullptr, k, t, v, nullptr, nullptr, nullptr, nullptr);
+    if (pass == FWD) core_fwd(e, c, v, nullptr, nullptr, nullptr, nullptr, k, t);
+    else core_bwd(e, c, v, nullptr, nullptr, nullptr, k, t, v, nullptr, nullptr, nullptr, nullptr);
   });
 }
 
@@ -513,26 +533,26 @@ void ffn_fwd(Exec& e, const llattn_ffn_cfg& c, const void* x, const float* w1, c
   e.gemm(e.linear(LLATTN_BF16, c.rows, c.d_ff, c.d, x, k.w1, b1, k.g, nullptr, LLATTN_ACT_GELU, e.dry ? &there : k.gp), false);
   e.gemm(e.linear(LLATTN_BF16, c.rows, c.d_out, c.d_ff, k.g, k.w2, b2, y), false);
 }
-void ffn_bwd(Exec& e, Arena& a, const llattn_ffn_cfg& c, const void* x, const Ffn& k, const void* dy, void* dx,
+void ffn_bwd(Exec& e, const llattn_ffn_cfg& c, const void* x, const Ffn& k, const void* dy, void* dx,
              float* dw1, float* db1, float* dw2, float* db2) {
-  void* dh = a.take((int64_t)c.rows * c.d_ff * 2);
+  void* dh = e.a.take((int64_t)c.rows * c.d_ff * 2);
   static char there;
   e.gemm(e.input_grad(LLATTN_BF16, c.rows, c.d_out, c.d_ff, dy, k.w2, k.w2t, dh, nullptr, nullptr, 0, e.dry ? &there : k.gp),
          e.weight_grad(LLATTN_BF16, c.rows, c.d_out, c.d_ff, dy, k.g, dw2, db2), false);
   const llattn_gemm_desc dw = e.weight_grad(LLATTN_BF16, c.rows, c.d_ff, c.d, dh, x, dw1, db1);
   if (dx) e.gemm(e.input_grad(LLATTN_BF16, c.rows, c.d_ff, c.d, dh, k.w1, k.w1t, dx), dw, false);
-  if (!dx || e.dry) e.gemm(dw, false);
+  else e.gemm(dw, false);
 }
-Need ffn_need(const llattn_ffn_cfg& c, bool bwd) {
-  return measure([&](Exec& e, Arena& a) {
+size_t ffn_need(const llattn_ffn_cfg& c, int pass) {
+  return measure([&](Exec& e) {
     Arena none{nullptr};
     Ffn k = ffn_layout(c, none);
     static char there;
     if (c.saved && persistent_grad(c.rows, c.d_ff, c.d)) k.w1t = &there;
     if (c.saved && persistent_grad(c.rows, c.d_out, c.d_ff)) k.w2t = &there;
     float* bias = reinterpret_cast<float*>(&there);
-    if (!bwd) ffn_fwd(e, c, nullptr, nullptr, nullptr, nullptr, nullptr, k, nullptr);
-    else ffn_bwd(e, a, c, nullptr, k, nullptr, &there, nullptr, bias, nullptr, bias);
+    if (pass == FWD) ffn_fwd(e, c, nullptr, nullptr, nullptr, nullptr, nullptr, k, nullptr);
+    else ffn_bwd(e, c, nullptr, k, nullptr, pass == BWD ? &there : nullptr, nullptr, bias, nullptr, bias);
   });
 }
 int32_t check_ffn(const char* what, const llattn_ffn_cfg* c) {
@@ -550,9 +570,10 @@ extern "C" {
 
 size_t llattn_block_bytes(const llattn_block_cfg* c, int32_t which) {
   if (check_cfg("llattn_block_bytes", c, true)) return 0;
-  if (which != 0) return block_need(*c, which == 2).total;
+  if (which != 0) return block_need(*c, which);
   Arena a{nullptr};
-  block_layout(*c, a);
+  static char there;
+  block_layout(*c, a, &there);
   return a.used;
 }
 
@@ -561,12 +582,10 @@ int32_t llattn_block_fwd(const llattn_block_cfg* c, const llattn_block_params* p
   const char* what = "llattn_block_fwd";
   if (const int32_t rc = check_cfg(what, c, true)) return rc;
   if (!p || !x || !kept || !out || !aligned16(kept)) return fail(LLATTN_ERR_LAYOUT, "%s: null or misaligned buffer", what);
-  const Need n = block_need(*c, false);
   Exec e;
-  Arena a{nullptr};
-  if (const int32_t rc = begin(e, a, what, n.total, n.gemm, ws, ws_bytes, stream)) return rc;
+  if (const int32_t rc = begin(e, what, block_need(*c, FWD), ws, ws_bytes, stream)) return rc;
   Arena ka{static_cast<char*>(kept)};
-  block_fwd(e, *c, *p, x, block_layout(*c, ka), out);
+  block_fwd(e, *c, *p, x, block_layout(*c, ka, out), out);
   return e.rc;
 }
 
@@ -576,18 +595,16 @@ int32_t llattn_block_bwd(const llattn_block_cfg* c, const llattn_block_params* p
   const char* what = "llattn_block_bwd";
   if (const int32_t rc = check_cfg(what, c, true)) return rc;
   if (!p || !x || !kept || !dy || !g || !c->saved) return fail(LLATTN_ERR_LAYOUT, "%s: null buffer or nothing kept", what);
-  const Need n = block_need(*c, true);
   Exec e;
-  Arena a{nullptr};
-  if (const int32_t rc = begin(e, a, what, n.total, n.gemm, ws, ws_bytes, stream)) return rc;
+  if (const int32_t rc = begin(e, what, block_need(*c, dx ? BWD : BWD_NO_DX), ws, ws_bytes, stream)) return rc;
   Arena ka{static_cast<char*>(const_cast<void*>(kept))};
-  block_bwd(e, a, *c, *p, x, block_layout(*c, ka), dy, dx, *g);
+  block_bwd(e, *c, *p, x, block_layout(*c, ka, nullptr), dy, dx, *g);
   return e.rc;
 }
 
 size_t llattn_core_bytes(const llattn_block_cfg* c, int32_t which) {
   if (check_cfg("llattn_core_bytes", c, false)) return 0;
-  if (which != 0) return core_need(*c, which == 2).total;
+  if (which != 0) return core_need(*c, which);
   Arena a{nullptr};
   core_layout(*c, a);
   return a.used;
@@ -599,10 +616,8 @@ int32_t llattn_core_fwd(const llattn_block_cfg* c, const llattn_core_views* in, 
   const char* what = "llattn_core_fwd";
   if (const int32_t rc = check_cfg(what, c, false)) return rc;
   if (!in || !r_w || !kept || !y || !aligned16(kept)) return fail(LLATTN_ERR_LAYOUT, "%s: null or misaligned buffer", what);
-  const Need n = core_need(*c, false);
   Exec e;
-  Arena a{nullptr};
-  if (const int32_t rc = begin(e, a, what, n.total, n.gemm, ws, ws_bytes, stream)) return rc;
+  if (const int32_t rc = begin(e, what, core_need(*c, FWD), ws, ws_bytes, stream)) return rc;
   Arena ka{static_cast<char*>(kept)};
   const Core k = core_layout(*c, ka);
   const Dims d(c->shape);
@@ -620,19 +635,17 @@ int32_t llattn_core_bwd(const llattn_block_cfg* c, const llattn_core_views* in, 
   const char* what = "llattn_core_bwd";
   if (const int32_t rc = check_cfg(what, c, false)) return rc;
   if (!in || !r_w || !kept || !dy || !dv || !c->saved) return fail(LLATTN_ERR_LAYOUT, "%s: null buffer or nothing kept", what);
-  const Need n = core_need(*c, true);
   Exec e;
-  Arena a{nullptr};
-  if (const int32_t rc = begin(e, a, what, n.total, n.gemm, ws, ws_bytes, stream)) return rc;
+  if (const int32_t rc = begin(e, what, core_need(*c, BWD), ws, ws_bytes, stream)) return rc;
   Arena ka{static_cast<char*>(const_cast<void*>(kept))};
   const Core k = core_layout(*c, ka);
-  core_bwd(e, a, *c, *in, gate_l, gate_r, k.r_w ? k.r_w : r_w, k, *dy, *dv, dgate_l, dgate_r, dr_w, dr_b);
+  core_bwd(e, *c, *in, gate_l, gate_r, k.r_w ? k.r_w : r_w, k, *dy, *dv, dgate_l, dgate_r, dr_w, dr_b);
   return e.rc;
 }
 
 size_t llattn_ffn_bytes(const llattn_ffn_cfg* c, int32_t which) {
   if (check_ffn("llattn_ffn_bytes", c)) return 0;
-  if (which != 0) return ffn_need(*c, which == 2).total;
+  if (which != 0) return ffn_need(*c, which);
   Arena a{nullptr};
   ffn_layout(*c, a);
   return a.used;
@@ -643,10 +656,8 @@ int32_t llattn_ffn_fwd(const llattn_ffn_cfg* c, const void* x, const float* w1, 
   const char* what = "llattn_ffn_fwd";
   if (const int32_t rc = check_ffn(what, c)) return rc;
   if (!x || !w1 || !w2 || !kept || !y || !aligned16(kept)) return fail(LLATTN_ERR_LAYOUT, "%s: null or misaligned buffer", what);
-  const Need n = ffn_need(*c, false);
   Exec e;
-  Arena a{nullptr};
-  if (const int32_t rc = begin(e, a, what, n.total, n.gemm, ws, ws_bytes, stream)) return rc;
+  if (const int32_t rc = begin(e, what, ffn_need(*c, FWD), ws, ws_bytes, stream)) return rc;
   Arena ka{static_cast<char*>(kept)};
   ffn_fwd(e, *c, x, w1, b1, w2, b2, ffn_layout(*c, ka), y);
   return e.rc;
@@ -657,12 +668,10 @@ int32_t llattn_ffn_bwd(const llattn_ffn_cfg* c, const void* x, const void* kept,
   const char* what = "llattn_ffn_bwd";
   if (const int32_t rc = check_ffn(what, c)) return rc;
   if (!x || !kept || !dy || !dw1 || !dw2 || !c->saved) return fail(LLATTN_ERR_LAYOUT, "%s: null buffer or nothing kept", what);
-  const Need n = ffn_need(*c, true);
   Exec e;
-  Arena a{nullptr};
-  if (const int32_t rc = begin(e, a, what, n.total, n.gemm, ws, ws_bytes, stream)) return rc;
+  if (const int32_t rc = begin(e, what, ffn_need(*c, dx ? BWD : BWD_NO_DX), ws, ws_bytes, stream)) return rc;
   Arena ka{static_cast<char*>(const_cast<void*>(kept))};
-  ffn_bwd(e, a, *c, x, ffn_layout(*c, ka), dy, dx, dw1, db1, dw2, db2);
+  ffn_bwd(e, *c, x, ffn_layout(*c, ka), dy, dx, dw1, db1, dw2, db2);
   return e.rc;
 }
 

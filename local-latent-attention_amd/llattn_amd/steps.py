@@ -110,7 +110,7 @@ class Block(torch.autograd.Function):
             grads = [w[:n], None if b is None else b[:n], w[n:], None if b is None else b[n:]]
             grads += [None if s is None else new(s) for s in shapes[4:]]
             ptrs = [w.data_ptr(), _ptr(b), None, None] + [_ptr(g) for g in grads[4:]]
-        n = _size("llattn_block_bytes", cfg, 2)
+        n = _size("llattn_block_bytes", cfg, 3 if dx is None else 2)
         ws = _bytes(n, dev)
         _call("llattn_block_bwd", _ref(cfg), _ref(p), x.data_ptr(), kept.data_ptr(), dy.data_ptr(), _ptr(dx),
               _ref(L.LlattnBlockParams(*ptrs)), _ptr(ws), n, L.stream_ptr(dev))
@@ -180,7 +180,7 @@ class Ffn(torch.autograd.Function):
         dx = torch.empty_like(x) if ctx.needs_input_grad[0] else None
         dw1, dw2 = new(cfg.d_ff, cfg.d), new(cfg.d_out, cfg.d_ff)
         db1, db2 = (new(n) if has else None for has, n in zip(ctx.bias, (cfg.d_ff, cfg.d_out)))
-        n = _size("llattn_ffn_bytes", cfg, 2)
+        n = _size("llattn_ffn_bytes", cfg, 3 if dx is None else 2)
         ws = _bytes(n, dev)
         _call("llattn_ffn_bwd", _ref(cfg), x.data_ptr(), kept.data_ptr(), dy.data_ptr(), _ptr(dx), dw1.data_ptr(),
               _ptr(db1), dw2.data_ptr(), _ptr(db2), _ptr(ws), n, L.stream_ptr(dev))

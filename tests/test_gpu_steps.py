@@ -408,3 +408,39 @@ def test_block_step_with_more_poolings_than_one_launch_holds():
         (a,), (b,) = _both(lambda: [m(x)], "llattn_block_fwd")
         _close([a[:64], a[-64:]], [m(x[:64]), m(x[-64:])], True)
         _close([a[B // 2:B // 2 + 64]], [b[B // 2:B // 2 + 64]], True)
+
+
+@pytest.mark.parametrize("qb", [0, 64])
+@pytest.mark.parametrize("bf16", [True, False])
+def test_block_step_peak_memory(qb, bf16):
+    """The native step's peak: a forward alone takes no more than the products one by one; a training pass at most the
+    attention output that its one node keeps to the end and the parameter gradients that it allocates together."""
+    from llattn_amd import LocalLatentAttentionTriton
+    dev = require_cuda()
+    torch.manual_seed(9)
+    D = 512
+    m = LocalLatentAttentionTriton(D, 8, 4, 128, 16, 64, latent_query_block_size=qb).to(dev)
+    x = torch.randn(4, 2048, D, device=dev).to(torch.bfloat16 if bf16 else torch.float32)
+
+    def peak(grad):
+        for _ in range(2):
+            m.zero_grad(set_to_none=True)
+            xx = x.detach().requires_grad_(grad)
+            torch.cuda.synchronize()
+            before = torch.cuda.memory_allocated()
+            torch.cuda.reset_peak_memory_stats()
+            with torch.set_grad_enabled(grad), torch.autocast("cuda", dtype=torch.bfloat16, enabled=bf16):
+                y = m(xx)
+            if grad:
+                y.backward(x)
+            torch.cuda.synchronize()
+            got = torch.cuda.max_memory_allocated() - before
+            del xx, y
+        return got
+
+    for grad in (False, True):
+        native = peak(grad)
+        with _logged():
+            single = peak(grad)
+        more = x.numel() * x.element_size() + 4 * sum(p.numel() for p in m.parameters()) if grad else 0
+        assert native <= single + more + (1 << 20), (grad, native, single, more)
