@@ -19,6 +19,14 @@ int32_t llattn_rmsnorm_bwd_residual(const void* dy, int32_t dy_dtype, int64_t ld
                                     void* dx16, int64_t lddx16, void* workspace, size_t workspace_bytes,
                                     void* stream);
 
+/* Two bf16 products that do not depend on each other: in one launch where that
+ * is expected to pay (d0: x W^T or dy W into bf16; d1: dy^T x into fp32, or
+ * another x W^T after x W^T), else one after the other.  The k order of the
+ * sums can then differ from the single products'. */
+size_t llattn_gemm_pair_workspace_size(const llattn_gemm_desc* d0, const llattn_gemm_desc* d1);
+int32_t llattn_gemm_pair(const llattn_gemm_desc* d0, const llattn_gemm_desc* d1, void* workspace,
+                         size_t workspace_bytes, void* stream);
+
 /* ---- whole steps ---------------------------------------------------------
  * The attention block, its core and the feed-forward as one call per
  * direction: the launches of the entry points of llattn.h in a row, without a

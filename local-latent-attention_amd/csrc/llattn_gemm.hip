@@ -39,7 +39,7 @@
 // (K a multiple of 8) masks the lanes whose 8 k values start at or past K with an out-of-range
 // offset (kmask), so no lane reads the next row's elements.
 #include "llattn_gemm.h"
-#include "llattn_pair.h"
+#include "llattn_steps.h"
 
 namespace llattn {
 namespace gemm {
@@ -925,16 +925,15 @@ int32_t prepare(const llattn_gemm_desc* d, void* workspace, size_t workspace_byt
 
 }  // namespace
 
-namespace llattn {
-namespace gemm {
-
-size_t pair_workspace(const llattn_gemm_desc* d0, const llattn_gemm_desc* d1) {
+extern "C" size_t llattn_gemm_pair_workspace_size(const llattn_gemm_desc* d0, const llattn_gemm_desc* d1) {
+  if (!d0 || !d1) return 0;
   if (pair_plan(d0, d1).mb) return 0;
   return std::max(llattn_gemm_workspace_size(d0), llattn_gemm_workspace_size(d1));
 }
 
-int32_t run_pair(const llattn_gemm_desc* d0, const llattn_gemm_desc* d1, void* workspace, size_t workspace_bytes,
-                 void* stream) {
+extern "C" int32_t llattn_gemm_pair(const llattn_gemm_desc* d0, const llattn_gemm_desc* d1, void* workspace,
+                                    size_t workspace_bytes, void* stream) {
+  if (!d0 || !d1) return fail(LLATTN_ERR_SHAPE, "llattn_gemm_pair: null descriptor");
   const TilePlan p = pair_plan(d0, d1);
   if (!p.mb) {
     if (const int32_t rc = llattn_gemm(d0, workspace, workspace_bytes, stream)) return rc;
@@ -944,11 +943,8 @@ int32_t run_pair(const llattn_gemm_desc* d0, const llattn_gemm_desc* d1, void* w
   if (const int32_t rc = prepare(d0, nullptr, 0, true, a0)) return rc;
   if (const int32_t rc = prepare(d1, nullptr, 0, true, a1)) return rc;
   launch_pair(a0, a1, p, !d0->b_trans, d1->a_trans, static_cast<hipStream_t>(stream));
-  return check_launch("llattn_gemm");
+  return check_launch("llattn_gemm_pair");
 }
-
-}  // namespace gemm
-}  // namespace llattn
 
 extern "C" int32_t llattn_gemm(const llattn_gemm_desc* d, void* workspace, size_t workspace_bytes, void* stream) {
   GemmArgs a;

@@ -9,7 +9,7 @@
 //
 // The sequences are those of the Python path (module.py, ops.py, linear.py, ffn.py: kept for profiling and for
 // parameters this path does not take), product by product with the same operands and roundings.  Two products that do
-// not depend on each other share a launch where that pays (llattn_pair.h); the k order of their sums can then differ
+// not depend on each other share a launch where that pays (llattn_gemm_pair); the k order of their sums can then differ
 // from the single products', otherwise both paths give the same bits.
 //
 // Every step is one function run twice: by the size query with a null base, where buffers only count and launches
@@ -17,7 +17,6 @@
 #include <algorithm>
 
 #include "llattn_abi.h"
-#include "llattn_pair.h"
 #include "llattn_pool.h"
 #include "llattn_steps.h"
 
@@ -69,9 +68,9 @@ struct Exec {
       gemm(d1, true);
       return;
     }
-    const size_t n = llattn::gemm::pair_workspace(&d0, &d1), mark = a.used;
+    const size_t n = llattn_gemm_pair_workspace_size(&d0, &d1), mark = a.used;
     void* ws = n ? a.take(n) : nullptr;
-    run([&] { return llattn::gemm::run_pair(&d0, &d1, ws, n, stream); });
+    run([&] { return llattn_gemm_pair(&d0, &d1, ws, n, stream); });
     a.used = mark;
   }
   // y [M][N] = x [M][K] w [N][K]ᵀ (+ b)

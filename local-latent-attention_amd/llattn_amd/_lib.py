@@ -119,6 +119,8 @@ _BC, _BP, _CV, _FC = (ctypes.POINTER(t) for t in (LlattnBlockCfg, LlattnBlockPar
 STEP_SIGNATURES = {
     "llattn_rmsnorm_bwd_residual": (_I32, [_P, _I32, _I64, _P, _I32, _I64, _P, _P, _I32, _I32, _P, _I64, _P, _P, _I64,
                                            _P, _I64, _P, _SZ, _P]),
+    "llattn_gemm_pair_workspace_size": (_SZ, [_G, _G]),
+    "llattn_gemm_pair": (_I32, [_G, _G, _P, _SZ, _P]),
     "llattn_block_bytes": (_SZ, [_BC, _I32]),
     "llattn_block_fwd": (_I32, [_BC, _BP, _P, _P, _P, _SZ, _P, _P]),
     "llattn_block_bwd": (_I32, [_BC, _BP, _P, _P, _P, _P, _BP, _P, _SZ, _P]),

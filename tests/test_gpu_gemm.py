@@ -775,3 +775,79 @@ def test_gemm_tiles_layouts_and_epilogues(M, N, K):
                 if heads:
                     tail = flat[M * cols:].view(2, -1, M // 2, 8).transpose(1, 2).reshape(M, N - cols)
                     assert torch.equal(tail, plain[:, cols:])
+
+
+# (layouts, first product (M, N, K), second): two shapes of each tile and k-group plan, in this order: 64 x 64 with one k
+# group, with two, 128 x 128
+PAIRS = [("fwd", (401, 24, 8), (155, 1112, 8)), ("fwd", (1066, 1960, 296), (265, 1176, 296)),
+         ("fwd", (29, 192, 376), (165, 16, 376)), ("fwd", (1088, 288, 800), (318, 696, 800)),
+         ("fwd", (2003, 3720, 928), (391, 80, 928)),
+         ("w_t", (27, 64, 32), (32, 64, 27)), ("w_t", (706, 2400, 720), (720, 2400, 706)),
+         ("w_t", (493, 8, 200), (200, 8, 493)), ("w_t", (619, 880, 448), (448, 880, 619)),
+         ("w_t", (1029, 2944, 1080), (1080, 2944, 1029)),
+         ("w", (660, 8, 8), (8, 8, 660)), ("w", (710, 2184, 776), (776, 2184, 710)),
+         ("w", (309, 16, 472), (472, 16, 309)), ("w", (1327, 872, 224), (224, 872, 1327)),
+         ("w", (1203, 2704, 1096), (1096, 2704, 1203)), ("w", (4096, 4096, 64), (64, 4096, 4096))]  # the last: one by one
+
+
+@pytest.mark.parametrize("kind,s0,s1", PAIRS)
+def test_gemm_pair(kind, s0, s1):
+    """Two independent products in one launch: two x W^T, or an input gradient (through W^T or W) with the weight
+    gradient and its row sums, at ragged sizes and strides of their own, with bias, row addends, an elementwise factor
+    and split-head storage, element by element against float64 (bounds as for the smaller tiles above)."""
+    import ctypes
+    from llattn_amd import _lib as L
+    dev = require_cuda()
+    g = torch.Generator(device=dev).manual_seed(sum(s0) + 3 * sum(s1))
+    ref = ctypes.byref
+
+    def rnd(rows, cols, pad=8):
+        return torch.randn(rows, cols + pad, device=dev, generator=g).bfloat16()[:, :cols]
+
+    def near(got, want, terms, roundings):
+        return bool(((got.double() - want).abs() <= roundings * 2.0 ** -8 * want.abs() + 2.0 ** -20 * terms).all())
+
+    def product(s, a_trans, b_trans, dtype, bias=None):
+        M, N, K = s
+        a, b = rnd(K, M) if a_trans else rnd(M, K), rnd(K, N) if b_trans else rnd(N, K)
+        out = torch.full((M, N), float("nan"), device=dev, dtype=dtype)
+        d = L.LlattnGemmDesc(M, N, K, int(a_trans), int(b_trans), a.data_ptr(), a.stride(0), b.data_ptr(), b.stride(0),
+                             out.data_ptr(), N, L.dtype_code(dtype), 0, None if bias is None else bias.data_ptr(), 0, None)
+        A, B = (a.t() if a_trans else a).double(), (b if b_trans else b.t()).double()
+        want, terms = A @ B, A.abs() @ B.abs() + 8
+        return d, (a, b), out, want if bias is None else want + bias.double(), terms
+
+    for extra in ("plain", "heads" if kind != "w" else "plain", "scaled", "rowadd" if kind != "fwd" else "plain"):
+        print("case: gemm pair", kind, s0, s1, extra, flush=True)
+        M, N, K = s0
+        bias = torch.randn(N, device=dev, generator=g) if kind == "fwd" else None
+        d0, keep0, o0, w0, t0 = product(s0, False, kind == "w", torch.bfloat16, bias)
+        b1 = torch.randn(s1[1], device=dev, generator=g) if kind == "fwd" else None
+        d1, keep1, o1, w1, t1 = product(s1, kind != "fwd", kind != "fwd", torch.bfloat16 if kind == "fwd" else torch.float32, b1)
+        rs = torch.full((s1[0],), float("nan"), device=dev)
+        if kind != "fwd":
+            d1.a_rowsum = rs.data_ptr()
+        roundings = 1
+        if extra == "scaled":
+            aux = rnd(M, N, 0)
+            d0.act, d0.aux, d0.ld_aux = L.ACT_MUL_AUX, aux.data_ptr(), N
+            w0, t0, roundings = w0 * aux.double(), t0 * (aux.double().abs() + 1), 2
+        elif extra == "heads":
+            d0.c_heads = L.LlattnHeadsLayout(M, 8, N // 8, 0)
+        elif extra == "rowadd":
+            seg = 5
+            n = -(-M // seg)
+            rows = rnd(n, N, 0)
+            d0.rowadd[0] = L.LlattnGemmRowadd(rows.data_ptr(), N, M, seg, n, L.DIV_SEG)
+            w0 = w0 + rows.double().repeat_interleave(seg, 0)[:M] / seg
+        lib = L.load()
+        nws = lib.llattn_gemm_pair_workspace_size(ref(d0), ref(d1))
+        ws = torch.empty(max(nws, 16), dtype=torch.uint8, device=dev)
+        L.check(lib.llattn_gemm_pair(ref(d0), ref(d1), ws.data_ptr(), nws, L.stream_ptr(dev)), "llattn_gemm_pair")
+        if extra == "heads":
+            o0 = o0.view(-1).view(N // 8, M, 8).transpose(0, 1).reshape(M, N)
+        assert near(o0, w0, t0, roundings), extra
+        assert near(o1, w1, t1, 1 if kind == "fwd" else 0), extra
+        if kind != "fwd":
+            a1 = keep1[0].t().double()
+            assert near(rs, a1.sum(1), a1.abs().sum(1) + 8, 0), extra

@@ -70,6 +70,8 @@ BLOCKS = [  # B, T, d_model, heads, latent width, latent heads, window, latents,
     (2, 650, 256, 4, 32, 2, 300, 10, 48),  # others
     (2, 2100, 256, 4, 128, 2, 64, 16, 0),  # transposed weights (4200 rows), split-head storage
     (16, 1024, 1408, 16, 512, 8, 64, 16, 0),  # gradients stored split-head as well
+    (1, 3287, 1536, 16, 384, 8, 64, 16, 0),  # two projections in one launch of 128 x 128 tiles
+    (13, 362, 1024, 16, 64, 2, 64, 50, 0),  # an input gradient through its transposed weight beside a weight gradient
 ]
 
 
