@@ -9,12 +9,15 @@ data that is already resident in HBM, under bf16 autocast with fp32 master
 weights (how the reference trainer runs it).  The default workload is
 the 0.55b-preset layer at B=16, T=2048.
 
-Prints ONE JSON line.  Besides the driver's fields it carries
+Prints ONE JSON line.  Besides the measurement it carries
 ``roofline`` (the C-ABI entry point with the most time per step, priced
 against bf16 MFMA peak for the projection GEMM and against HBM peak for the
 attention kernels; durations measured with HIP events on the launch stream
 in a second timed region of K steps, because an event record costs the GPU
-about 5 us between kernels and would inflate the step time of the first),
+about 5 us between kernels and would inflate the step time of the first; with
+a log the entry points are called one by one from Python, where the first
+region's steps are one native call per direction of the same products, in which
+weight casts and poolings, or two small products, may share a launch),
 ``mfma_frac_module`` (algorithmic module FLOPs / step time / bf16 dense
 peak), per-kernel event timings, and ``cpu_baseline`` (the reference
 PyTorch path restated in fp32, timed on the host cores on a bounded
@@ -692,9 +695,10 @@ def main():
         step()
     torch.cuda.synchronize()
     t1 = time.perf_counter()
-    # Timed region 2: the same K steps with a HIP event pair on the launch stream around every C-ABI call
-    # -> per-entry-point durations for `roofline` / `kernels`.  Each event record costs the GPU about 5 us
-    # between kernels, so these steps are not the ones `value` is measured on.
+    # Timed region 2: K steps whose entry points are called one by one, a HIP event pair on the launch stream
+    # around each -> per-entry-point durations for `roofline` / `kernels`.  Each event record costs the GPU about
+    # 5 us between kernels, and while calls are logged the native steps (one call per direction, weight casts and
+    # poolings in one launch) are not used, so these steps are not the ones `value` is measured on.
     torch.cuda.synchronize()
     llops.EVENT_LOG = []
     t2 = time.perf_counter()

@@ -293,7 +293,7 @@ int32_t llattn_cast(int32_t nseg, const float* const* src, void* const* dst, con
  * segment i is then a row-major fp32 [rows[i], n[i] / rows[i]] matrix (rows and columns multiples of 8,
  * src, dst and dst_t 16-byte aligned, bf16 output) and dst_t[i][c * ld_t[i] + r] = bf16(src[i][r * cols + c])
  * (ld_t[i] >= rows[i], a multiple of 8).  dst_t, ld_t and rows are nseg-entry arrays, or dst_t is NULL for
- * none.  The bf16 W^T copies that input gradients run on (dy W as dy (W^T)^T on the persistent GEMM, the
+ * none.  The bf16 W^T copies that input gradients run on (dy W as dy (W^T)^T, both operands k-contiguous, the
  * nn.Linear backward of reference models.py:80-84 under autocast), written while the cast reads W anyway:
  * one extra 2-byte write per element instead of an llattn_transpose pass in the backward. */
 int32_t llattn_cast_transposed(int32_t nseg, const float* const* src, void* const* dst, const int64_t* n,
@@ -302,7 +302,7 @@ int32_t llattn_cast_transposed(int32_t nseg, const float* const* src, void* cons
 
 /* dst[c][r] = src[r][c] for a bf16 matrix of rows x cols (both multiples of 8; 16-byte aligned, leading
  * dimensions in elements, multiples of 8).  The input gradient dy W of a projection runs as
- * dy (W^T)^T on the persistent GEMM (both operands k-contiguous) with this transposed copy of the bf16
+ * dy (W^T)^T (both operands k-contiguous) with this transposed copy of the bf16
  * weight (reference models.py:80-84, the nn.Linear backward under autocast). */
 int32_t llattn_transpose(const void* src, int64_t ld_src, int32_t rows, int32_t cols, void* dst, int64_t ld_dst,
                          void* stream);

@@ -22,7 +22,7 @@ struct GemmArgs {
   void* C; int64_t ldc;
   const float* bias;
   float* part;     // split-K partials [S][M][N], then (rowsum) [S][M]
-  float* rowsum;   // fp32 [M] or null: sum_k A(m, k), from a column of ones in place of B's column N
+  float* rowsum;   // fp32 [M] or null: sum_k A(m, k), from a column of ones in place of B's column N or summed beside the products
   // bf16 C only: C[m][n] += ra[(m / T) * n_seg + (m % T) / seg][n] / divisor for each of up to two addends
   const uint16_t* ra_ptr[2];
   int64_t ra_ld[2];
@@ -31,7 +31,7 @@ struct GemmArgs {
   int act;
   uint16_t* aux;
   int64_t ld_aux;
-  HeadsMap ch;  // bf16 C stored split-head (ch.T > 0; persistent kernel)
+  HeadsMap ch;  // bf16 C stored split-head (ch.T > 0): the persistent kernel, the smaller tiles and their reduction
 };
 
 // Exact GELU u * Phi(u) of the reference FeedForward (reference models.py:57, F.gelu) and its derivative

@@ -32,7 +32,7 @@
 // ordered reduction adds them (deterministic, no atomics).
 //
 // Split-head C (llattn_heads_layout, the q|k|v projection output stored as per-sequence head slabs): the
-// persistent kernel's stores take each 8-column piece to its slab; the arithmetic is the same.
+// persistent kernel's stores (and those of the smaller tiles) take each 8-column piece to its slab; the arithmetic is the same.
 //
 // K need not be a multiple of the step: the last steps read zero past K.  Rows of an m/n-contiguous
 // operand past K lie beyond its buffer extent and read zero by themselves; a k-contiguous operand
@@ -775,7 +775,7 @@ void launch(const GemmArgs& a, int S, int c_dtype, hipStream_t st) {
 }
 
 
-// Number of K splits: 1 when the output tiles alone fill most of the chip; otherwise the split count S
+// Number of K splits of the 256 x 256 kernels (the smaller tiles, tried first, have a plan of their own): 1 when the output tiles alone fill most of the chip; otherwise the split count S
 // that minimises a time model of the product: the busiest CU runs ceil(tiles S / 256) workgroups of
 // 1/S of a tile's k range each (one 128 KB workgroup per CU), plus the fp32 partials that the ordered
 // reduction reads and writes (S M N 4 bytes at ~5 TB/s, against a tile rate of ~4.4 TFLOP/s per CU).
@@ -783,8 +783,8 @@ void launch(const GemmArgs& a, int S, int c_dtype, hipStream_t st) {
 // splits fill three rounds exactly, where 2 would leave a quarter of the CUs idle.
 int resolve_split(const llattn_gemm_desc* d) {
   if (d->split_k > 0) return d->split_k;
-  if (d->c_heads.T != 0) return 1;  // a split-head C comes from the persistent kernel
-  // so do row addends with a k-contiguous B (an input gradient through the transposed weight)
+  if (d->c_heads.T != 0) return 1;  // of these kernels the persistent one alone stores a split-head C
+  // and adds row addends with a k-contiguous B (an input gradient through the transposed weight)
   if (!d->a_trans && !d->b_trans && (d->rowadd[0].ptr || d->rowadd[1].ptr)) return 1;
   const int64_t tiles = (int64_t)((d->M + BM - 1) / BM) * ((d->N + BN - 1) / BN);
   if (tiles >= 224) return 1;

@@ -327,8 +327,9 @@ static double big_us(int64_t M, int64_t N, int steps, int S) {
 //   (128 x 128 x 4096: 8.2 us in 16 splits against 16 in two k groups and 20 on 256 x 256 tiles in 16 splits;
 //   512 x 512 x 4096 15.3 in 8 splits against 19; 333 x 1408 x 4096, 132 tiles, 20 in 4 splits against 18.)
 // Only where 256 x 256 tiles leave CUs idle (below 224 of them): from there on
-// those tiles' half as large operand traffic wins (4011 x 4992 x 1536: 69 us against 81).  Neither the epilogue nor
-// the layouts enter, so a product has the same bits whichever way it is stored.
+// those tiles' half as large operand traffic wins (4011 x 4992 x 1536: 69 us against 81).  Epilogue and layouts enter
+// through the 256 x 256 kernels' split count alone: near the line a product stored split-head or with row addends takes
+// these tiles where the plain one is split there, and its sums run in another k order (2950 x 1408 x 4096, x Wᵀ).
 // Measured on operands just written, in us: 333 x 4736 x 1408 13.5, 1024 x 1408 x 1408 13.3,
 // 1024 x 1408 x 4096 26.8, 1024 x 4096 x 1408 18.7, 4011 x 384 x 1536 (dy W) 14.3, 1536 x 384 x 4011 (dyT x) 18.5;
 // with L2-resident operands against the 256 x 256 kernels and the register-staged 64 x 64 tiles that this replaced:

@@ -86,7 +86,7 @@ struct Exec {
     d.act = act; d.aux = aux; d.ld_aux = aux ? N : 0;
     return d;
   }
-  // dx [M][K] = dy [M][N] w [N][K] (+ row addends; * aux): through w_t where the persistent kernel takes it
+  // dx [M][K] = dy [M][N] w [N][K] (+ row addends; * aux): through w_t where there is one
   static llattn_gemm_desc input_grad(int dt, int M, int N, int K, const void* dy, const void* w, const void* w_t, void* dx,
                   const llattn_heads_layout* heads = nullptr, const llattn_gemm_rowadd* ra = nullptr, int n_ra = 0,
                   void* aux = nullptr) {
@@ -164,8 +164,8 @@ struct Casts {
   }
 };
 
-// bf16 input gradients of this many rows run on the persistent kernel with a transposed weight (gemm.py:
-// input_grad_persistent); fewer read the weight by transposing LDS loads
+// bf16 input gradients of this many rows run through a transposed weight (gemm.py: input_grad_persistent), on the
+// persistent kernel or, with too few tiles for it, the smaller ones; fewer rows read the weight by transposing LDS loads
 bool persistent_grad(int64_t M, int64_t N, int64_t K) { return M >= 4096 && K % 8 == 0 && N % 8 == 0 && N > 64; }
 
 llattn_tensor view(const void* p, int64_t off, int64_t es, int64_t sb, int64_t sn, int64_t sh) {

@@ -74,7 +74,7 @@ def _run(M: int, N: int, K: int, A: torch.Tensor, a_trans: bool, B: torch.Tensor
 def linear(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None = None, out: torch.Tensor | None = None,
            accumulate: bool = False, heads=None, rowadd=()) -> torch.Tensor:
     """``x [M, K] @ w [N, K]^T (+ bias fp32 [N])`` -> bf16 ``[M, N]`` (``heads``: stored split-head; ``rowadd``:
-    the broadcast row addends of :func:`matmul_nn`, on the persistent kernel only)."""
+    the broadcast row addends of :func:`matmul_nn`)."""
     _check2d("x", x)
     _check2d("w", w)
     M, K = x.shape
@@ -106,7 +106,7 @@ def matmul_nn_scaled(a: torch.Tensor, b: torch.Tensor, s: torch.Tensor, b_t: tor
     """``bf16(a [M, K] @ b [K, N]) * s`` elementwise in bf16 (``s`` bf16 ``[M, N]``): with ``s = gelu'(h)`` from
     :func:`linear_gelu`, the input gradient of a projection whose input was ``gelu(h)``, through the GELU.
     ``b_t``: ``b``'s transposed copy, if the caller has it; for large M (:func:`input_grad_persistent`) the product
-    then runs on the persistent kernel, as :func:`input_grad` does (the same bits)."""
+    then runs through it, as :func:`input_grad` does."""
     _check2d("a", a)
     _check2d("b", b)
     M, K = a.shape
@@ -153,23 +153,25 @@ def transpose(w: torch.Tensor) -> torch.Tensor:
     return out
 
 
-# input gradients with row addends through the transposed weight and the persistent kernel (else matmul_nn)
+# input gradients with row addends through the transposed weight (else matmul_nn)
 ROWADD_PERSISTENT = True
 
 
 def input_grad_persistent(M: int, N: int, K: int, rowadd=()) -> bool:
-    """Whether :func:`input_grad` of ``dy [M, N]`` and ``w [N, K]`` runs on the persistent kernel."""
+    """Whether :func:`input_grad` of ``dy [M, N]`` and ``w [N, K]`` runs through the transposed weight: on the
+    persistent kernel, or on the smaller tiles where its tiles are too few."""
     return (not rowadd or ROWADD_PERSISTENT) and M >= 4096 and K % 8 == 0 and N % 8 == 0 and N > 64
 
 
 def input_grad(dy: torch.Tensor, w: torch.Tensor, rowadd=(), w_t: torch.Tensor | None = None,
                heads=None) -> torch.Tensor:
     """``dy [M, N] @ w [N, K]`` (+ the ``rowadd`` addends of :func:`matmul_nn`) -> bf16 ``[M, K]``, the input
-    gradient of ``y = x w^T``.  For large M (:func:`input_grad_persistent`) as ``dy (w^T)^T`` on the persistent
-    kernel with a transposed copy of ``w`` (both operands k-contiguous: plain LDS fragment reads, the epilogue
-    overlapped with the next tile): ``w_t`` when the caller has it (``llattn_cast_transposed`` writes it with the
-    weight cast), else made here; otherwise :func:`matmul_nn` (transposing fragment reads of ``w``).  All routes
-    give the same bits.  ``heads``: the output stored split-head as :func:`linear` does (persistent route only)."""
+    gradient of ``y = x w^T``.  For large M (:func:`input_grad_persistent`) as ``dy (w^T)^T`` with a
+    transposed copy of ``w`` (both operands k-contiguous: plain LDS fragment reads and, on the persistent kernel, the
+    epilogue overlapped with the next tile): ``w_t`` when the caller has it (``llattn_cast_transposed`` writes it with
+    the weight cast), else made here; otherwise :func:`matmul_nn` (transposing fragment reads of ``w``).  From 224
+    output tiles of 256 x 256 on, where nothing is split over k, both routes give the same bits.  ``heads``: the output
+    stored split-head as :func:`linear` does (with the transposed copy only)."""
     M, N = dy.shape
     K = w.shape[1]
     if input_grad_persistent(M, N, K, rowadd):
@@ -179,7 +181,7 @@ def input_grad(dy: torch.Tensor, w: torch.Tensor, rowadd=(), w_t: torch.Tensor |
             raise ValueError(f"w_t is {tuple(w_t.shape)}, expected the transpose of w {tuple(w.shape)}")
         return linear(dy, w_t, rowadd=rowadd, heads=heads)
     if heads is not None:
-        raise ValueError(f"a split-head input gradient needs the persistent kernel (M={M}, N={N}, K={K})")
+        raise ValueError(f"a split-head input gradient needs the transposed weight's route (M={M}, N={N}, K={K})")
     return matmul_nn(dy, w, rowadd=rowadd)
 
 

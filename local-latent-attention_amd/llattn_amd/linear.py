@@ -211,8 +211,8 @@ def project(x: torch.Tensor, *linears: torch.nn.Linear, pools=(), packed=None, h
     ``heads``: ``(T, dh, n[, tail_dh])`` -- the output ``[B, T, N]`` is stored split-head (its first ``n * dh``
     columns as ``[B][n][T][dh]`` slabs, the rest after them, packed or as slabs of ``tail_dh`` columns;
     :mod:`llattn_amd.gemm`), for a consumer that reads it by strides (:class:`llattn_amd.ops.LLAttnCore`); its
-    gradient comes back as a plain row-major tensor.  ``grad_heads``: the input gradient (bf16, on the
-    persistent kernel's route of :func:`llattn_amd.gemm.input_grad`, no poolings) is stored split-head that way
+    gradient comes back as a plain row-major tensor.  ``grad_heads``: the input gradient (bf16, through the
+    transposed weight of :func:`llattn_amd.gemm.input_grad`, no poolings) is stored split-head that way
     instead, for a producer of ``x`` whose backward reads its output gradient by strides (``dy_heads`` of
     :class:`llattn_amd.ops.LLAttnCore`)."""
     params = []

@@ -150,7 +150,7 @@ class LocalLatentAttentionTriton(nn.Module):
             prof.lap("qkv_ms")
         if pooled is None:
             pooled = pool(x, *latents)
-        # the pooled latents' projection (256 rows at config 2) on the MFMA GEMM as well: split-K forward,
+        # the pooled latents' projection (256 rows at config 2) on the MFMA GEMM as well: the smaller tiles,
         # bias gradient from the weight-gradient pass
         gkgv = project(pooled, self.rkv_proj, packed=packed["rkv"]) if bf16 else project_f32(pooled, self.rkv_proj)
         if prof is not None:

@@ -165,7 +165,7 @@ class _Prof:
 
 def _remote_heads(lay: L.Layout, dt) -> bool:
     """Whether ``r_out``'s output R [B, n_q, D] is stored split-head ([B][H][n_q][Dh] slabs): in bf16, where its
-    persistent GEMM writes it so (latent width above 64, below 2 GiB).  Only the local-attention kernels read R,
+    GEMM writes it so (latent width above 64, below 2 GiB).  Only the local-attention kernels read R,
     by strides, so each head of a sequence streams as one contiguous run."""
     return dt == torch.bfloat16 and lay.Lh * lay.Ldh > 64 and lay.Dh % 8 == 0 and \
         lay.B * lay.n_q * lay.H * lay.Dh * 2 < (1 << 31)
@@ -174,7 +174,7 @@ def _remote_heads(lay: L.Layout, dt) -> bool:
 def grad_heads_ok(M: int, N: int, K: int, dh: int) -> bool:
     """Whether a bf16 input gradient ``dy [M, N] @ w [N, K]`` can be stored split-head with heads of ``dh``
     columns: on the persistent kernel with at least 224 output tiles of 256 x 256 (row-major it then runs there
-    unsplit too, so both layouts hold the same bits; with fewer tiles a row-major product is split over k),
+    unsplit too, so both layouts hold the same bits; with fewer tiles a row-major product may be split over k),
     below 2 GiB."""
     return input_grad_persistent(M, N, K) and dh % 8 == 0 and N > 64 and M * K * 2 < (1 << 31) and \
         ((M + 255) // 256) * ((K + 255) // 256) >= 224
@@ -305,7 +305,7 @@ def _qkv_views(lay: L.Layout, qkv: torch.Tensor, token_rq: bool, heads: bool):
 
 def heads_layout_ok(lay: L.Layout, d_model: int, token_rq: bool) -> bool:
     """Whether the block's q|k|v projection can be stored split-head (``heads`` of :class:`LLAttnCore`): the
-    GEMM writes it from its persistent kernel (d_model > 64), all of it below 2 GiB."""
+    GEMM's persistent kernel and smaller tiles write it so (d_model > 64), all of it below 2 GiB."""
     D = lay.H * lay.Dh
     width = 3 * D + (lay.Lh * lay.Ldh if token_rq else 0)
     return d_model > 64 and lay.Dh % 8 == 0 and lay.Ldh % 8 == 0 and width % 8 == 0 and \
