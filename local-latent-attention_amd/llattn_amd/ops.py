@@ -471,12 +471,14 @@ class LLAttnFunction(torch.autograd.Function):
             (r_out_b is None or r_out_b.numel() == H * Dh) and (dt == torch.float32 or (Dh % 8 == 0 and Ldh % 8 == 0))
         if ctx.native:
             per_head = gl.dim() == 2 and gl.shape[0] > 1
-            ctx.cfg = L.LlattnBlockCfg(lay.shape(dt, per_head), H * Dh, 0, 0, 1, 0, int(_remote_heads(lay, dt)), 0,
+            saved = any(ctx.needs_input_grad)  # else no backward follows: what only it reads is not written
+            ctx.cfg = L.LlattnBlockCfg(lay.shape(dt, per_head), H * Dh, 0, 0, int(saved), 0, int(_remote_heads(lay, dt)), 0,
                                        int(dt == torch.bfloat16 and _latent_grad_heads(lay)))
             y = _empty((B, S, H, Dh), dt, device)
             kept = steps.core_forward(ctx.cfg, L.LlattnCoreViews(*views), gl, gr, r_out_w, r_out_b, L.view_bnhd(y),
                                       device)
-            ctx.save_for_backward(Q, K, V, GQ, GK, GV, gl, gr, r_out_w, kept)
+            if saved:
+                ctx.save_for_backward(Q, K, V, GQ, GK, GV, gl, gr, r_out_w, kept)
             return y.permute(0, 2, 1, 3)
         y, ol, lse, w, lat, lse_lat, R = _core_forward(lay, *views, gl, gr, r_out_w, r_out_b, dt, device)
         ctx.save_for_backward(Q, K, V, GQ, GK, GV, gl, gr, r_out_w, lat, lse_lat, R, ol, lse, w)
