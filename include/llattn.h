@@ -253,7 +253,7 @@ typedef struct llattn_gemm_desc {
   int32_t act;                  /* LLATTN_ACT_* */
   void* aux;                    /* bf16 [M][ld_aux]: gelu' written (LLATTN_ACT_GELU) or read (_MUL_AUX) */
   int64_t ld_aux;
-  /* bf16 C [M][ldc] stored split-head (the forward of a projection: a_trans = b_trans = 0, split_k = 0 or 1,
+  /* bf16 C [M][ldc] stored split-head (the forward of a projection: a_trans = b_trans = 0, no split_k above 1,
      accumulation or activation). */
   llattn_heads_layout c_heads;
 } llattn_gemm_desc;
