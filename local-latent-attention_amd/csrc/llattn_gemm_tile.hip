@@ -305,13 +305,13 @@ void launch_dt(const GemmArgs& a, const TilePlan& p, int c_dtype, hipStream_t st
 
 // Time in us of the 256 x 256 kernels with S k splits: 6 us to fill and drain, rounds of (tile, split) workgroups over 256 CUs, 1.2 us per
 // 64-k step of a workgroup alone up to 1.75 with every CU at work, and for S > 1 the ordered reduction with its fp32
-// partials written and read at 9 TB/s.  (1024 x 4736 x 1408, 76 tiles: 32 us; 8192 x 4096 x 1408, 512: 83;
+// partials written and read at 7 TB/s.  (1024 x 4736 x 1408, 76 tiles: 32 us; 8192 x 4096 x 1408, 512: 83;
 // 1536 x 1536 x 4011, 36 tiles in 7 splits: 41.)
 static double big_us(int64_t M, int64_t N, int steps, int S) {
   const int64_t n = ((M + BM - 1) / BM) * ((N + BN - 1) / BN) * S;
   const double last = (double)(n % 256) / 256.0;
   const double per = (double)(n / 256) * 1.75 + (n % 256 ? 1.2 + 0.55 * last * last : 0.0);
-  return 6.0 + (double)((steps + S - 1) / S) * per + (S > 1 ? 7.0 + 8.0 * S * (double)M * (double)N / 9e6 : 0.0);
+  return 6.0 + (double)((steps + S - 1) / S) * per + (S > 1 ? 7.0 + 8.0 * S * (double)M * (double)N / 7e6 : 0.0);
 }
 
 // The tiles that a product takes, fitted to the times of 38 products (16 x 1024 x 1408 to 3000 x 4736 x 1408; all
@@ -324,8 +324,8 @@ static double big_us(int64_t M, int64_t N, int steps, int S) {
 //   (Four k groups: no faster.)
 //   64 x 64 split over workgroups: 5.2 us and 0.07 per split with the reduction's launch, the same steps (from memory 2.8 TB/s at most, in
 //   pieces of 128 bytes a k row), partials written and read at 4.2 TB/s.
-//   (128 x 128 x 4096: 8.2 us in 16 splits against 16 in two k groups and 20 on 256 x 256 tiles in 16 splits;
-//   512 x 512 x 4096 15.3 in 8 splits against 19; 333 x 1408 x 4096, 132 tiles, 20 in 4 splits against 18.)
+//   (dyᵀ x, 128 x 128 x 16384: 15.6 us in 16 splits against 62 in two k groups and 36 on 256 x 256 tiles in 64 splits;
+//   512 x 512 x 16384 27 in 16 splits against 42 there; 1408 x 512 x 8192, 176 tiles, 31 in 4 splits against 36.)
 // Only where 256 x 256 tiles leave CUs idle (below 224 of them): from there on
 // those tiles' half as large operand traffic wins (4011 x 4992 x 1536: 69 us against 81).  Epilogue and layouts enter
 // through the 256 x 256 kernels' split count alone: near the line a product stored split-head or with row addends takes
@@ -358,10 +358,12 @@ TilePlan tile_plan(const llattn_gemm_desc* d, double* us) {
   take(4.5 + steps * ((double)(t64 / 1024) * 0.85 + last[r64]), 2, 1);
   if (steps >= 4 && t64 <= 256) take(3.8 + split(2) * 0.44, 2, 2);
   if (steps >= 4 && t64 > 256 && t64 <= 512) take(5.6 + split(2) * 0.68, 2, 2);
-  // a few tiles of a long contraction (from K = 2048 on; below, it gains a microsecond at most): 64 x 64 tiles over S
-  // ranges of at least two steps, their partials reduced in order
+  // a few tiles of a long contraction: 64 x 64 tiles over S ranges of at least two steps, their partials reduced in order.
+  // From K = 6144 on: below, the GPU gains at most 10 us (128 x 128 x 4096 16 -> 8), and a step of products this small
+  // waits for the host, to which the second launch costs 4 (with it from K = 2048: the 0.55b model over 64 tokens
+  // 3310 -> 3460 us, a 256-wide block's training pass over 4096 tokens 308 -> 320).
   const double stream = 2.0 * (double)(M + N) * (double)d->K / 2.8e6;
-  for (int S = 2; S <= 32 && steps >= 32; S *= 2) {
+  for (int S = 2; S <= 32 && steps >= 96; S *= 2) {
     const int64_t per = (steps + S - 1) / S, parts = (steps + per - 1) / per, n = t64 * parts;  // no range is empty
     if (per < 2 || n > 2048) break;
     take(5.2 + 0.07 * (double)parts + std::max(stream, (double)per * ((double)(n / 1024) * 0.85 + last[(n % 1024 + 255) / 256])) +

@@ -181,7 +181,7 @@ def input_grad(dy: torch.Tensor, w: torch.Tensor, rowadd=(), w_t: torch.Tensor |
             raise ValueError(f"w_t is {tuple(w_t.shape)}, expected the transpose of w {tuple(w.shape)}")
         return linear(dy, w_t, rowadd=rowadd, heads=heads)
     if heads is not None:
-        raise ValueError(f"a split-head input gradient needs the transposed weight's route (M={M}, N={N}, K={K})")
+        raise ValueError(f"a split-head input gradient needs the persistent kernel's route (M={M}, N={N}, K={K})")
     return matmul_nn(dy, w, rowadd=rowadd)
 
 

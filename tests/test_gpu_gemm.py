@@ -701,7 +701,7 @@ def test_scaled_input_grad_through_the_transpose(M, K, N):
                                    (1000, 1416, 328), (1000, 4104, 264), (1000, 4104, 1032), (1024, 4096, 1408),
                                    (1288, 72, 4008),
                                    # split over workgroups: few tiles, a k tail in the last of 2, 16 and 32 ranges
-                                   (72, 136, 2056), (24, 64, 4104), (264, 520, 2120), (136, 128, 16392)])
+                                   (72, 136, 6152), (24, 64, 8200), (264, 520, 8264), (136, 128, 16392)])
 def test_gemm_tiles_layouts_and_epilogues(M, N, K):
     """The smaller tiles (64 x 64 and 128 x 128, one and two k groups, split over workgroups): every operand layout at strides of its own,
     into bf16 and fp32, with bias, accumulation, row addends, the activations, split-head storage and row sums,
