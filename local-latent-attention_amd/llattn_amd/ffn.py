@@ -20,7 +20,7 @@ import torch
 from . import _lib as L
 from . import gemm, ops
 from .linear import pack_params, weight_grad
-from .steps import Ffn, plain
+from .steps import Ffn, plain_as
 
 BF16 = torch.bfloat16
 
@@ -69,23 +69,29 @@ class _FeedForward(torch.autograd.Function):
                 None if db1 is None else db1.to(b1dt), dw2.to(w2dt), None if db2 is None else db2.to(b2dt))
 
 
+def _param(m, name: str):
+    """``getattr(m, name)``, without nn.Module's search where the parameter is registered as itself."""
+    held = getattr(m, "_parameters", ())
+    return held[name] if name in held else getattr(m, name)
+
+
 def _step_cfg(x: torch.Tensor, ps) -> L.LlattnFfnCfg | None:
     """The native step's configuration for ``x`` and ``(w1, b1, w2, b2)``, or None where it does not take them: it
     sees pointers alone, so every shape is compared here."""
-    dev, d = x.device, x.shape[-1]
+    d = x.shape[-1]
     rows = x.numel() // max(1, d)
     d_ff, d_out = ps[0].shape[0], ps[2].shape[0]
-    if not 0 < rows < 1 << 31 or d % 8 or d_ff % 8 or d_out % 8 or not plain(x, dev, BF16):
+    if not 0 < rows < 1 << 31 or d % 8 or d_ff % 8 or d_out % 8 or x.dtype is not BF16 or not x.is_contiguous() \
+            or x.data_ptr() & 15:
         return None
-    for p, s in zip(ps, ((d_ff, d), (d_ff,), (d_out, d_ff), (d_out,))):
-        if p is not None and (p.shape != s or not plain(p, dev)):
-            return None
+    if not plain_as(ps, ((d_ff, d), (d_ff,), (d_out, d_ff), (d_out,)), x.device):
+        return None
     saved = torch.is_grad_enabled() and (x.requires_grad or any(p is not None and p.requires_grad for p in ps))
     return L.LlattnFfnCfg(rows, d, d_ff, d_out, int(saved))
 
 
 def feed_forward(x: torch.Tensor, w1: torch.nn.Linear, w2: torch.nn.Linear) -> torch.Tensor:
     """bf16 ``w2(gelu(w1(x)))`` on the GEMM kernels (GPU only; widths multiples of 8)."""
-    ps = (w1.weight, w1.bias, w2.weight, w2.bias)
+    ps = (_param(w1, "weight"), _param(w1, "bias"), _param(w2, "weight"), _param(w2, "bias"))
     cfg = _step_cfg(x, ps) if x.is_cuda and not ops.observed() else None
     return _FeedForward.apply(x, *ps) if cfg is None else Ffn.apply(x, cfg, *ps)

@@ -32,13 +32,6 @@ from .linear import pack_params, project, project_f32
 from .ops import LLAttnCore, _Prof, grad_heads_ok, heads_layout_ok, pool
 
 
-def _held(m: nn.Module, name: str):
-    """``getattr(m, name)``, without nn.Module's search where the parameter is registered as itself.  (A forward over
-    333 tokens is bound by the host: with one buffer for a forward-only call 58.7 -> 56.0 us.)"""
-    p = m._parameters.get(name)
-    return getattr(m, name) if p is None else p
-
-
 class LocalLatentAttentionTriton(nn.Module):
     """``LocalLatentAttentionTriton(d_model, n_heads, latent_heads, latent_dim, n_latents, window,
     bias=True, local_block_size=256, latent_query_block_size=0)``.
@@ -178,34 +171,38 @@ class LocalLatentAttentionTriton(nn.Module):
         dev = x.device
         bf16 = torch.is_autocast_enabled("cuda") and torch.get_autocast_dtype("cuda") == torch.bfloat16
         dt = torch.bfloat16 if bf16 else torch.float32
+        # the parameters without nn.Module's search where they are registered as themselves.  (A forward over 333 tokens
+        # takes the host about as long as its six launches take the GPU: with this and one buffer for a forward-only
+        # call 58.7 -> 56.0 us.)
         mods = self._modules
         params = []
-        for name in ("qkv_proj", "rq_proj", "rkv_proj", "r_out", "out"):
+        for name in ("qkv_proj", "rq_proj", "rkv_proj", "r_out", "out", "gate_local", "gate_remote"):
             m = mods[name]
-            params += (_held(m, "weight"), _held(m, "bias"))
-        params += (_held(mods["gate_local"], "weight"), _held(mods["gate_remote"], "weight"))
-        biases = [p is not None for p in params[1:10:2]]
-        if not steps.plain(x, dev, dt) or any(b != biases[0] for b in biases):
-            return None
-        for p in params:
-            if p is not None and not steps.plain(p, dev):
+            held = m._parameters
+            w, b = held.get("weight"), held.get("bias")
+            params.append(m.weight if w is None else w)
+            if len(params) < 11:
+                params.append(m.bias if b is None else b)
+        has_bias = params[1] is not None
+        for p in params[3:10:2]:
+            if (p is not None) is not has_bias:
                 return None
+        if x.dtype is not dt or not x.is_contiguous() or x.data_ptr() & 15:
+            return None
+        # another width of a replaced projection, or gates per head, run (or are refused) product by product
+        Ld = lay.Lh * lay.Ldh
+        d, gate = (D,), (1, lay.Dh)
+        if not steps.plain_as(params, ((3 * D, D), (3 * D,), (Ld, D), (Ld,), (2 * Ld, D), (2 * Ld,), (D, Ld), d, (D, D), d,
+                                       gate, gate), dev):
+            return None
         if bf16 and (D % 8 or lay.Dh % 8 or lay.Ldh % 8):
             return None
-        # the native call takes pointers: another width of a replaced projection, or gates per head, run (or are
-        # refused) product by product
-        Ld = lay.Lh * lay.Ldh
-        shapes = ((3 * D, D), (3 * D,), (Ld, D), (Ld,), (2 * Ld, D), (2 * Ld,), (D, Ld), (D,), (D, D), (D,),
-                  (1, lay.Dh), (1, lay.Dh))
-        for p, s in zip(params, shapes):
-            if p is not None and p.shape != s:
-                return None
         macro = self.latent_query_block_size > 1
         saved = torch.is_grad_enabled() and (x.requires_grad or any(p is not None and p.requires_grad for p in params))
         # one call forms every gradient; with parts frozen ahead of what trains the single products stop early
         if saved and not x.requires_grad and not all(p is None or p.requires_grad for p in params):
             return None
-        cfg = L.LlattnBlockCfg(lay.shape(dt), D, int(macro), int(biases[0]), int(saved),
+        cfg = L.LlattnBlockCfg(lay.shape(dt), D, int(macro), int(has_bias), int(saved),
                                int(bf16 and heads_layout_ok(lay, D, not macro)), int(ops._remote_heads(lay, dt)),
                                int(bf16 and grad_heads_ok(B * T, D, D, lay.Dh)),
                                int(bf16 and ops._latent_grad_heads(lay)))

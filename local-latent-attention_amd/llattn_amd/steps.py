@@ -24,6 +24,16 @@ def plain(t: torch.Tensor, device, dtype=_F32) -> bool:
     return t.dtype is dtype and t.device == device and t.is_contiguous() and not t.data_ptr() & 15
 
 
+def plain_as(params, shapes, device) -> bool:
+    """Whether every parameter that is there is :func:`plain` fp32 of its shape (a native step sees its pointer alone)."""
+    index = device.index if device.type == "cuda" else -1
+    for p, s in zip(params, shapes):
+        if p is not None and (p.dtype is not _F32 or p.shape != s or p.get_device() != index or not p.is_contiguous()
+                              or p.data_ptr() & 15):
+            return False
+    return True
+
+
 def _bytes(n: int, device):
     return torch.empty((n,), dtype=torch.uint8, device=device) if n else None
 
@@ -37,10 +47,16 @@ def _call(name, *args):
 
 
 def _size(name, cfg, which: int) -> int:
-    n = getattr(L.load(), name)(_ref(cfg), which)
-    if n == 0 and which == 0:
+    return getattr(L.load(), name)(_ref(cfg), which)
+
+
+def _forward_sizes(name, ref):
+    """Bytes that a forward keeps and its scratch."""
+    fn = getattr(L.load(), name)
+    kept = fn(ref, 0)
+    if kept == 0:
         L.check(L.ERR_SHAPE, name)
-    return n
+    return kept, fn(ref, 1)
 
 
 def _dense(t: torch.Tensor, dtype) -> torch.Tensor:
@@ -55,8 +71,8 @@ def _dense(t: torch.Tensor, dtype) -> torch.Tensor:
 def block_forward(x, cfg, params):
     """``(out, kept)`` of the block on ``x [B, T, D]``; ``params``: the twelve parameters of ``L.BLOCK_PARAMS``
     (biases None without)."""
-    dev = x.device
-    k, n = _size("llattn_block_bytes", cfg, 0), _size("llattn_block_bytes", cfg, 1)
+    dev, ref = x.device, _ref(cfg)
+    k, n = _forward_sizes("llattn_block_bytes", ref)
     if cfg.saved:
         kept, ws = _bytes(k, dev), _bytes(n, dev)
         at = _ptr(ws)
@@ -65,7 +81,7 @@ def block_forward(x, cfg, params):
         kept = _bytes(k + n, dev)
         at = kept.data_ptr() + k if n else None
     out = torch.empty_like(x)
-    _call("llattn_block_fwd", _ref(cfg), _ref(L.LlattnBlockParams(*[_ptr(p) for p in params])), x.data_ptr(),
+    _call("llattn_block_fwd", ref, _ref(L.LlattnBlockParams(*[_ptr(p) for p in params])), x.data_ptr(),
           kept.data_ptr(), at, n, out.data_ptr(), L.stream_ptr(dev))
     return out, kept
 
@@ -123,10 +139,10 @@ class Block(torch.autograd.Function):
 
 def core_forward(cfg, views, gl, gr, r_w, r_b, y_view, device):
     """Runs the core into ``y_view``; returns what its backward reads."""
-    kept = _bytes(_size("llattn_core_bytes", cfg, 0), device)
-    n = _size("llattn_core_bytes", cfg, 1)
-    ws = _bytes(n, device)
-    _call("llattn_core_fwd", _ref(cfg), _ref(views), gl.data_ptr(), gr.data_ptr(), r_w.data_ptr(), _ptr(r_b),
+    ref = _ref(cfg)
+    k, n = _forward_sizes("llattn_core_bytes", ref)
+    kept, ws = _bytes(k, device), _bytes(n, device)
+    _call("llattn_core_fwd", ref, _ref(views), gl.data_ptr(), gr.data_ptr(), r_w.data_ptr(), _ptr(r_b),
           kept.data_ptr(), _ptr(ws), n, _ref(y_view), L.stream_ptr(device))
     return kept
 
@@ -151,12 +167,11 @@ def core_backward(cfg, views, gl, gr, r_w, has_rb, kept, dy_view, grad_views, de
 # ---------------------------------------------------------------------------
 
 def ffn_forward(x, cfg, w1, b1, w2, b2):
-    dev = x.device
-    kept = _bytes(_size("llattn_ffn_bytes", cfg, 0), dev)
-    n = _size("llattn_ffn_bytes", cfg, 1)
-    ws = _bytes(n, dev)
+    dev, ref = x.device, _ref(cfg)
+    k, n = _forward_sizes("llattn_ffn_bytes", ref)
+    kept, ws = _bytes(k, dev), _bytes(n, dev)
     y = torch.empty((*x.shape[:-1], cfg.d_out), dtype=_BF16, device=dev)
-    _call("llattn_ffn_fwd", _ref(cfg), x.data_ptr(), w1.data_ptr(), _ptr(b1), w2.data_ptr(), _ptr(b2), kept.data_ptr(),
+    _call("llattn_ffn_fwd", ref, x.data_ptr(), w1.data_ptr(), _ptr(b1), w2.data_ptr(), _ptr(b2), kept.data_ptr(),
           _ptr(ws), n, y.data_ptr(), L.stream_ptr(dev))
     return y, kept
 
