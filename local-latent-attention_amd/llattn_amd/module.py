@@ -204,8 +204,9 @@ class LocalLatentAttentionTriton(nn.Module):
             return None
         cfg = L.LlattnBlockCfg(lay.shape(dt), D, int(macro), int(has_bias), int(saved),
                                int(bf16 and heads_layout_ok(lay, D, not macro)), int(ops._remote_heads(lay, dt)),
-                               int(bf16 and grad_heads_ok(B * T, D, D, lay.Dh)),
-                               int(bf16 and ops._latent_grad_heads(lay)))
+                               # storage of gradients
+                               int(bf16 and saved and grad_heads_ok(B * T, D, D, lay.Dh)),
+                               int(bf16 and saved and ops._latent_grad_heads(lay)))
         return steps.Block.apply(x, cfg, *params)
 
     def _packed_weights(self, macro: bool) -> dict:

@@ -81,7 +81,7 @@ def block_forward(x, cfg, params):
         kept = _bytes(k + n, dev)
         at = kept.data_ptr() + k if n else None
     out = torch.empty_like(x)
-    _call("llattn_block_fwd", ref, _ref(L.LlattnBlockParams(*[_ptr(p) for p in params])), x.data_ptr(),
+    _call("llattn_block_fwd", ref, _ref(L.LlattnBlockParams(*[None if p is None else p.data_ptr() for p in params])), x.data_ptr(),
           kept.data_ptr(), at, n, out.data_ptr(), L.stream_ptr(dev))
     return out, kept
 
