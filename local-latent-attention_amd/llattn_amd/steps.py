@@ -2,9 +2,9 @@
 
 Each autograd function here is the whole of a step that :mod:`llattn_amd.module`, :mod:`llattn_amd.ops` and
 :mod:`llattn_amd.ffn` otherwise issue product by product from Python: the same products with what the backward
-reads in one buffer (two independent ones may share a launch).  The calls that take this path have parameters in fp32, whole, 16-byte aligned and
-on the activations' device, activations in the compute dtype, and nobody looking at the single calls
-(:func:`llattn_amd.ops.observed`).  The others, and profiling, stay on the Python path.  Forward-only calls are
+reads in one buffer (two independent ones may share a launch).  The calls that take this path have parameters of the
+layout's shapes in fp32, whole, 16-byte aligned and on the activations' device, activations in the compute dtype,
+and nobody looking at the single calls (:func:`llattn_amd.ops.observed`).  The others, and profiling, stay on the Python path.  Forward-only calls are
 applied as functions too: a tangent, a batched tensor or a tracer is then met as by any other autograd function.
 """
 from __future__ import annotations
