@@ -4,8 +4,8 @@
 // output tensors) the GPU waited for the host.  One call issues them in about 4 us each.  Measured (MI355X, a pass
 // before -> with these calls; in brackets with the kernels for small products since): a 0.55b layer's forward over 333
 // tokens 267 -> 100 us (57), its fwd + bwd over 3 x 1337 tokens (0.60b) 905 -> 640 us (574), the op at head dim 128 over
-// 2 x 3001 tokens 488 -> 293 us (264 to 305, the host's; 53 us of it gradients laid out as their inputs, which autograd then need not
-// copy), the 0.55b model over 1024 tokens 9.4 -> 4.9 ms (3.9).
+// 2 x 3001 tokens 488 -> 293 us (264 to 305, the host's; 53 us of it gradients laid out as their inputs, which autograd
+// then need not copy), the 0.55b model over 1024 tokens 9.4 -> 4.9 ms (3.9).
 //
 // The sequences are those of the Python path (module.py, ops.py, linear.py, ffn.py: kept for profiling and for
 // parameters this path does not take), product by product with the same operands and roundings.  Two products that do

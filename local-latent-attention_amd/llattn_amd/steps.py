@@ -4,8 +4,8 @@ Each autograd function here is the whole of a step that :mod:`llattn_amd.module`
 :mod:`llattn_amd.ffn` otherwise issue product by product from Python: the same products with what the backward
 reads in one buffer (two independent ones may share a launch).  The calls that take this path have parameters of the
 layout's shapes in fp32, whole, 16-byte aligned and on the activations' device, activations in the compute dtype,
-and nobody looking at the single calls (:func:`llattn_amd.ops.observed`).  The others, and profiling, stay on the Python path.  Forward-only calls are
-applied as functions too: a tangent, a batched tensor or a tracer is then met as by any other autograd function.
+and nobody looking at the single calls (:func:`llattn_amd.ops.observed`).  The others, and profiling, stay on the
+Python path.  Forward-only calls are applied as functions too: a tangent, a batched tensor or a tracer is then met as by any other autograd function.
 """
 from __future__ import annotations
 
@@ -81,8 +81,8 @@ def block_forward(x, cfg, params):
         kept = _bytes(k + n, dev)
         at = kept.data_ptr() + k if n else None
     out = torch.empty_like(x)
-    _call("llattn_block_fwd", ref, _ref(L.LlattnBlockParams(*[None if p is None else p.data_ptr() for p in params])), x.data_ptr(),
-          kept.data_ptr(), at, n, out.data_ptr(), L.stream_ptr(dev))
+    ptrs = L.LlattnBlockParams(*[None if p is None else p.data_ptr() for p in params])
+    _call("llattn_block_fwd", ref, _ref(ptrs), x.data_ptr(), kept.data_ptr(), at, n, out.data_ptr(), L.stream_ptr(dev))
     return out, kept
 
 
